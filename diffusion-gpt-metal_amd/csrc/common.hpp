@@ -45,6 +45,17 @@ struct dgm_gpu {
     int n_streams = 0;
     bool many_streams = false;   // more than kMaxStreams: destroy waits for the device
     bool spin_waits = false;
+    // Operand planes of the large GEMMs (gemm_planes.hip): apart from `ws`,
+    // which captured graphs may read while eager work runs on another stream.
+    // Grow-only like it; used by eager calls only, and a call on another
+    // stream than the last one's waits for that one's work.
+    void* planes = nullptr;
+    size_t planes_bytes = 0;
+    void* planes_retired[kMaxRetired] = {};
+    int n_planes_retired = 0;
+    bool planes_fixed = false;             // dgm_gpu_reserve was called: it grows no more by itself
+    hipStream_t planes_stream = nullptr;   // of the last use
+    hipEvent_t planes_event = nullptr;
 };
 
 namespace dgm {
@@ -66,6 +77,11 @@ int check_launch(dgm_gpu* g, const char* name);
 void* workspace(dgm_gpu* g, size_t bytes);
 // The status a caller returns when workspace() gave nullptr.
 int ws_error(dgm_gpu* g);
+// The buffer of the large GEMMs' operand planes, at least `bytes`, ordered
+// after its last use. nullptr (recording nothing) under graph capture, in
+// dgm_gemmNT_noalloc, when dgm_gpu_reserve fixed a smaller one, or when the
+// memory is not there: the caller then takes the kernels that need no planes.
+uint8_t* planes_buffer(dgm_gpu* g, size_t bytes);
 // After a synchronize: records an error on g if a decode kernel gave up a
 // bounded in-workgroup wait since the last check (gemm_decode.hip), and
 // clears the device's flag.
@@ -194,6 +210,16 @@ int wt_prep(dgm_gpu* g, int bits, int nlin, const void* const* W, const float* c
 bool bwd_fold_ok(int M, int N, int K, int G);
 int gemm_bwd_fold(dgm_gpu* g, const int8_t* codesT, const float* scalesT, const float* dY, const float* X, float* dX,
                   float* dW, int M, int N, int K, int G, bool accumulate, const float* sg_gate, const float* sg_up);
+
+// Large GEMMs on 16-bit MFMA over split operands (gemm_planes.hip): the
+// forward, dX and dW in the fp32 mode, where planes_pay says that they are
+// the faster way. Each product returns kNotFused, launching nothing, when planes_buffer has none.
+bool planes_pay(int64_t M, int64_t N, int64_t K);
+int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias,
+               float* Y, const dgm_GemmP* p);
+int planes_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, float* dX,
+              const dgm_GemmP* p);
+int planes_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p, bool accumulate);
 
 inline bool aligned(const void* p, size_t a) {
     return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;

@@ -1,5 +1,6 @@
 // Context lifecycle and dispatch-region semantics of the C ABI
 // (mirrors src/GPU.swift:118-198: init, begin, end, go's bookkeeping).
+#include <algorithm>
 #include <cstdarg>
 #include <mutex>
 #include <new>
@@ -113,6 +114,39 @@ void* workspace(dgm_gpu* g, size_t bytes) {
     return g->ws;
 }
 
+uint8_t* planes_buffer(dgm_gpu* g, size_t bytes) {
+    if (g->use_scratch) return nullptr;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(g->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (bytes > g->planes_bytes) {
+        if (g->planes_fixed || g->n_planes_retired == dgm_gpu::kMaxRetired) return nullptr;
+        void* p = nullptr;
+        const size_t want = std::max(bytes, std::min(2 * g->planes_bytes, bytes + (size_t(256) << 20)));
+        if (hipMalloc(&p, want) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (g->planes) g->planes_retired[g->n_planes_retired++] = g->planes;
+        g->planes = p;
+        g->planes_bytes = want;
+        g->planes_stream = nullptr;   // nothing has used this one
+    }
+    if (g->planes_stream && g->planes_stream != g->stream) {
+        if (hipStreamIsCapturing(g->planes_stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
+            (!g->planes_event && hipEventCreateWithFlags(&g->planes_event, hipEventDisableTiming) != hipSuccess) ||
+            hipEventRecord(g->planes_event, g->planes_stream) != hipSuccess ||
+            hipStreamWaitEvent(g->stream, g->planes_event, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
+    g->planes_stream = g->stream;
+    return static_cast<uint8_t*>(g->planes);
+}
+
 int ws_error(dgm_gpu* g) { return g->first_err != DGM_OK ? g->first_err : DGM_ERR_HIP; }
 
 }  // namespace dgm
@@ -156,6 +190,9 @@ void dgm_gpu_destroy(dgm_gpu* g) {
     if (g->many_streams) (void)hipDeviceSynchronize();
     if (g->ws) (void)hipFree(g->ws);
     for (int i = 0; i < g->n_retired; ++i) (void)hipFree(g->retired[i]);
+    if (g->planes) (void)hipFree(g->planes);
+    for (int i = 0; i < g->n_planes_retired; ++i) (void)hipFree(g->planes_retired[i]);
+    if (g->planes_event) (void)hipEventDestroy(g->planes_event);
     if (g->own_stream) (void)hipStreamDestroy(g->own_stream);
     delete g;
 }

@@ -156,11 +156,16 @@ int64_t dgm_gemmNT_workspace_bound(int64_t M, int64_t N, int64_t K) {
 
 int dgm_gpu_reserve(dgm_gpu* g, int64_t bytes) {
     if (!g || bytes < 0) return DGM_ERR_ARG;
-    if (size_t(bytes) <= g->ws_bytes) return DGM_OK;
-    return dgm::workspace(g, size_t(bytes)) ? DGM_OK : dgm::ws_error(g);
+    if (size_t(bytes) > g->ws_bytes && !dgm::workspace(g, size_t(bytes))) return dgm::ws_error(g);
+    // The plane buffer too, which from now on grows here only: a call that
+    // finds it too small runs without it.
+    g->planes_fixed = false;
+    if (size_t(bytes) > g->planes_bytes) (void)dgm::planes_buffer(g, size_t(bytes));
+    g->planes_fixed = true;
+    return DGM_OK;
 }
 
-int64_t dgm_gpu_workspace_bytes(const dgm_gpu* g) { return g ? int64_t(g->ws_bytes) : -1; }
+int64_t dgm_gpu_workspace_bytes(const dgm_gpu* g) { return g ? int64_t(g->ws_bytes + g->planes_bytes) : -1; }
 
 int dgm_gemmDX(dgm_gpu* g, int64_t bits, const float* w, const void* q, const float* scale,
                const float* dy, float* dx, int64_t M, int64_t N, int64_t K, int64_t qGroup) {

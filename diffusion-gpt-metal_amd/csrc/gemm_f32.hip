@@ -1602,6 +1602,10 @@ int gemm_f32_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const 
     // Larger M in the reduced-precision mode: bf16 MFMA with W dequantized in LDS.
     if (g->math == DGM_MATH_BF16 && bf16_ok(bits, W, X, scale, p))
         return bf16_fwd(g, bits, W, scale, X, bias, Y, p);
+    if (planes_pay(p->M, p->N, p->K)) {
+        const int rc = planes_fwd(g, bits, W, scale, X, bias, Y, p);
+        if (rc != kNotFused) return rc;
+    }
     GemmArgs a{};
     a.A = X; a.B = W; a.scale = scale; a.bias = bias; a.out = Y;
     a.M = p->M; a.N = p->N; a.K = p->K;
@@ -1638,6 +1642,10 @@ int gemm_f32_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const 
 
 int gemm_f32_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY,
                 float* dX, const dgm_GemmP* p) {
+    if (planes_pay(p->M, p->N, p->K)) {
+        const int rc = planes_dx(g, bits, W, scale, dY, dX, p);
+        if (rc != kNotFused) return rc;
+    }
     GemmArgs a{};
     a.A = dY; a.B = W; a.scale = scale; a.out = dX;
     a.M = p->M; a.N = p->N; a.K = p->K;
@@ -1664,6 +1672,10 @@ int gemm_f32_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const f
 
 int gemm_f32_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p,
                 bool accumulate) {
+    if (planes_pay(p->M, p->N, p->K)) {
+        const int rc = planes_dw(g, dY, X, dW, p, accumulate);
+        if (rc != kNotFused) return rc;
+    }
     GemmArgs a{};
     a.A = dY; a.B = X; a.out = dW;
     a.M = p->M; a.N = p->N; a.K = p->K;
@@ -1687,6 +1699,7 @@ int gemm_f32_bwd_pair(dgm_gpu* g, int bits, const void* W, const float* scale, c
                       float* dX, float* dW, const dgm_GemmP* p, bool accumulate, bool* fused, const float* sg_gate,
                       const float* sg_up) {
     *fused = false;
+    if (!sg_gate && planes_pay(p->M, p->N, p->K)) return DGM_OK;
     GemmArgs ax{};
     ax.A = dY; ax.B = W; ax.scale = scale; ax.out = dX;
     ax.sg_gate = sg_gate; ax.sg_up = sg_up;

@@ -1,0 +1,760 @@
+// Large GEMMs on 16-bit MFMA over operands split into planes (gfx950):
+//
+//   out[i,j] = sum_c A[i,c] * B[j,c]  (+ bias[j], or += out)
+//
+// The forward (A = X, B = deq(W)), dX (A = dY, B = deq(W)^T) and
+// dW (A = dY^T, B = X^T) of the linears are all this product; only where
+// element (row, c) of an operand lies differs (struct Src).
+//
+// Every operand row is scaled by a power of two that brings its largest
+// element into [2^14, 2^15), and split into two f16 pieces x = h + l with
+// h = f16(x), l = f16(x - h): 22 bits and a sign, an error of at most
+// 2^-24 |x| for elements down to 2^-15 of the row's largest (below that 2^-40
+// of the largest). The product is hh + hl + lh on v_mfma_f32_32x32x16_f16 with
+// fp32 accumulation; the omitted ll is below 2^-24 of the product. Products of
+// f16 pieces are exact, and the matrix unit rounds its sum once per 8 of them
+// (measured: 4.0e-7 in the 2-norm over 4096 random products, the figure of a
+// CPU chain rounded every 8), so hh, summed by itself, has half the roundings
+// of v_mfma_f32_16x16x4_f32; hl and lh go to a second accumulator whose
+// roundings are 2^-11 of those. Against 64 bits, the fp32 MFMA kernels first:
+// 2048 x 14336 x 4096 5.3e-7, 4.0e-7; dX and dW of 2048 x 4096 x 4096 5.7e-7
+// and 4.2e-7, 4.1e-7 and 3.1e-7; dW over 12288 rows 1.0e-6, 2.8e-7.
+// Rows with an infinity or NaN are computed from the original operands in
+// fp32 (an infinity times a low piece of the other sign would be NaN).
+//
+// What it gains: v_mfma_f32_16x16x4_f32 peaks at 157 TFLOP/s and its kernels
+// here ran at 50-57; three f16 products per fp32 product at 2.5 PFLOP/s peak at
+// 833. Measured, both sides in turn: 2048 x 14336 x 4096 int4 4816 -> 656 us
+// (366 TFLOP/s), 517 x 4100 x 4128 int8 320 -> 93, dX + dW of 2048 x 4096 x
+// 4096 2416 -> 442, forward + dX + dW of fp32 12288 x 1536 x 384 779 -> 301.
+// What bounds it: the power the matrix unit draws. With zeros for data the
+// GEMM of 4096 x 4096 x 4096 takes 225 us instead of 320 (the clock stays up);
+// interleaving the LDS reads with the MFMAs, raising their priority, one wave
+// per SIMD with twice the tile (64 instead of 85 LDS bytes per clock), all
+// within 3% of this form.
+//
+// Three launches: the rows' largest elements, the split into planes, the
+// GEMM; a fourth adds the parts of tiles that are cut along c (struct Plan).
+//
+// Plane layout: 32 rows x 16 c of a plane are one fragment of the MFMA, 1 KB
+// in lane order (lane l: row l % 32, c = 8 (l / 32) .. + 7), and a 32-row
+// block's h and l fragments of the same 16 c are neighbours. So every
+// direct-to-LDS load and every LDS read is 1 KB contiguous (whole cache lines,
+// no bank conflicts, no swizzle), the rows are padded to whole tiles and c to
+// whole stages with zeros, and the GEMM has no bounds checks before its stores.
+//
+// GEMM: WM x WN waves, each MT x NT tiles of 32 x 32. A ring of four stages
+// of 16 c; a step waits for the next stage by count, meets the other waves,
+// issues the loads of the stage three ahead and reads the next stage's
+// fragments into registers while the MFMAs of the current one run, so the
+// load latency, the LDS latency and the barrier are off the MFMAs' path.
+#include "common.hpp"
+
+#include <algorithm>
+
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kFlag = 1 << 30;      // exps[]: the row holds an infinity or NaN
+constexpr int kMaxParts = 16;       // row chunks of a column-maximum pass
+
+// One operand: element (r, c) of R x C.
+struct Src {
+    const void* p;
+    const float* scale;   // codes: per (weight row, group)
+    int64_t ld;           // elements from one stored row to the next
+    int R, C;
+    int bits;             // 32, 8, 4
+    int col;              // 0: p[r * ld + c], 1: p[c * ld + r] (codes: the weight row is c)
+    int G, groups;        // codes
+    int vec;              // 8 consecutive stored elements can be loaded at once
+};
+
+struct Operand {
+    Src s;
+    uint8_t* planes;
+    uint32_t* part;       // largest |element| (its bits) of each row: parts x width
+    int parts, width;
+    int* exps;            // row scale 2^e, or kFlag
+    int rb, kb;           // 32-row blocks and 16-c blocks written (padded)
+};
+
+__device__ __forceinline__ float code_at(const void* p, int bits, int64_t i) {
+    if (bits == 8) return float(static_cast<const int8_t*>(p)[i]);
+    const uint8_t b = static_cast<const uint8_t*>(p)[i >> 1];
+    return float(int8_t((i & 1) ? b : uint8_t(b << 4)) >> 4);
+}
+
+__device__ __forceinline__ float elem(const Src& s, int r, int c) {
+    const int64_t i = s.col ? int64_t(c) * s.ld + r : int64_t(r) * s.ld + c;
+    if (s.bits == 32) return static_cast<const float*>(s.p)[i];
+    const int64_t si = s.col ? int64_t(c) * s.groups + r / s.G : int64_t(r) * s.groups + c / s.G;
+    return code_at(s.p, s.bits, i) * s.scale[si];
+}
+
+// ---- launch 1: largest |element| of each row ---------------------------------------
+// One pass over fp32 data (X, dY, W, or the scales that bound the codes'
+// weights). Rows stored contiguously: lpr lanes per row. Rows stored across:
+// a block takes 64 of them and one of `parts` chunks of c.
+struct MaxArg {
+    const float* p;
+    int64_t ld;
+    int R, C, col, lpr, parts, blocks;
+    uint32_t* out;
+};
+
+__device__ __forceinline__ void max_part(const MaxArg& a, int block) {
+    const int t = threadIdx.x;
+    if (!a.col) {
+        const int per = 256 / a.lpr;
+        const int r = block * per + t / a.lpr, l = t % a.lpr;
+        uint32_t m = 0;
+        if (r < a.R) {
+            const float* row = a.p + int64_t(r) * a.ld;
+            const bool vec = (a.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(a.p) & 15) == 0;
+            int c = 0;
+            if (vec) {
+                const int n4 = a.C >> 2;
+#pragma unroll 4
+                for (int i = l; i < n4; i += a.lpr) {
+                    const u32x4 v = reinterpret_cast<const u32x4*>(row)[i] & 0x7fffffffu;
+                    m = max(max(m, max(v[0], v[1])), max(v[2], v[3]));
+                }
+                c = n4 << 2;
+            }
+            for (int i = c + l; i < a.C; i += a.lpr) m = max(m, __float_as_uint(row[i]) & 0x7fffffffu);
+        }
+        for (int off = a.lpr >> 1; off >= 1; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off)));
+        if (r < a.R && l == 0) a.out[r] = m;
+        return;
+    }
+    __shared__ uint32_t sh[4][64];
+    const int nb = (a.R + 63) / 64;
+    const int r = (block % nb) * 64 + (t & 63), part = block / nb;
+    const int64_t chunk = (int64_t(a.C) + a.parts - 1) / a.parts;
+    const int64_t c1 = min(int64_t(a.C), (part + 1) * chunk);
+    uint32_t m = 0;
+    if (r < a.R) {
+#pragma unroll 8
+        for (int64_t c = part * chunk + (t >> 6); c < c1; c += 4)
+            m = max(m, __float_as_uint(a.p[c * a.ld + r]) & 0x7fffffffu);
+    }
+    sh[t >> 6][t & 63] = m;
+    __syncthreads();
+    if (t < 64 && r < a.R) a.out[int64_t(part) * a.R + r] = max(max(sh[0][t], sh[1][t]), max(sh[2][t], sh[3][t]));
+}
+
+__global__ __launch_bounds__(256) void row_max_kernel(MaxArg a, MaxArg b) {
+    if (int(blockIdx.x) < a.blocks) max_part(a, blockIdx.x);
+    else max_part(b, blockIdx.x - a.blocks);
+}
+
+// ---- launch 2: the split ---------------------------------------------------------------
+// Elements (r, c .. c + 7), zero outside R x C.
+template <int BITS, int COL>
+__device__ __forceinline__ void load8(const Src& s, int r, int c, float (&v)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = 0.0f;
+    if (r >= s.R || c >= s.C) return;
+    if constexpr (COL) {
+        const int n = min(8, s.C - c);
+        if constexpr (BITS == 32) {
+            const float* p = static_cast<const float*>(s.p) + int64_t(c) * s.ld + r;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (j < n) v[j] = p[j * s.ld];
+        } else {
+            const float* sp = s.scale + int64_t(c) * s.groups + r / s.G;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (j < n) v[j] = code_at(s.p, BITS, int64_t(c + j) * s.ld + r) * sp[j * s.groups];
+        }
+    } else if (s.vec && c + 8 <= s.C) {
+        const int64_t i = int64_t(r) * s.ld + c;
+        if constexpr (BITS == 32) {
+            const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(s.p) + i);
+            const float4 x = p[0], y = p[1];
+            v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+            v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+        } else {
+            const float sc = s.scale[int64_t(r) * s.groups + c / s.G];   // G % 8 == 0
+            if constexpr (BITS == 8) {
+                const int2 q = *reinterpret_cast<const int2*>(static_cast<const int8_t*>(s.p) + i);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[j] = float((q.x << (24 - 8 * j)) >> 24) * sc;
+                    v[4 + j] = float((q.y << (24 - 8 * j)) >> 24) * sc;
+                }
+            } else {
+                const int q = *reinterpret_cast<const int*>(static_cast<const uint8_t*>(s.p) + (i >> 1));
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = float((q << (28 - 4 * j)) >> 28) * sc;
+            }
+        }
+    } else {
+        const int n = min(8, s.C - c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (j < n) v[j] = elem(s, r, c + j);
+    }
+}
+
+// 2^e brings a row of largest magnitude `bits` below 2^15 (extra: the codes'
+// bits above the scale); e <= 126 keeps the factor a normal number.
+__device__ __forceinline__ int row_exp(uint32_t bits, int extra) {
+    if (bits >= 0x7f800000u) return kFlag;
+    return bits == 0 ? 0 : min(126, 14 + 127 - int(bits >> 23) - extra);
+}
+
+template <int BITS, int COL>
+__device__ __forceinline__ void split_part(const Operand& o, int block) {
+    const int chunks = (o.kb + 15) / 16;
+    const int rb = block / chunks, chunk = block % chunks;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = rb * 32 + (lane & 31), h = lane >> 5;
+    const int at = BITS != 32 && COL ? r / o.s.G : r;
+    uint32_t m = 0;
+    if (r < o.s.R)
+        for (int i = 0; i < o.parts; ++i) m = max(m, o.part[int64_t(i) * o.width + at]);
+    const int e = row_exp(m, BITS == 32 ? 0 : (BITS == 8 ? 7 : 3));
+    if (chunk == 0 && wave == 0 && h == 0) o.exps[r] = e;
+    const float f = __uint_as_float(uint32_t((e == kFlag ? 0 : e) + 127) << 23);
+    float v[4][8];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load8<BITS, COL>(o.s, r, (chunk * 16 + u * 4 + wave) * 16 + 8 * h, v[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int kb = chunk * 16 + u * 4 + wave;
+        if (kb >= o.kb) continue;
+        f16x8 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float x = v[u][j] * f;
+            hi[j] = _Float16(x);
+            lo[j] = _Float16(x - float(hi[j]));
+        }
+        uint8_t* out = o.planes + (int64_t(rb) * o.kb + kb) * 2048 + lane * 16;
+        *reinterpret_cast<f16x8*>(out) = hi;
+        *reinterpret_cast<f16x8*>(out + 1024) = lo;
+    }
+}
+
+__device__ __forceinline__ void split_any(const Operand& o, int block) {
+    if (o.s.col) {
+        if (o.s.bits == 32) split_part<32, 1>(o, block);
+        else if (o.s.bits == 8) split_part<8, 1>(o, block);
+        else split_part<4, 1>(o, block);
+    } else {
+        if (o.s.bits == 32) split_part<32, 0>(o, block);
+        else if (o.s.bits == 8) split_part<8, 0>(o, block);
+        else split_part<4, 0>(o, block);
+    }
+}
+
+__global__ __launch_bounds__(256) void split_kernel(Operand a, Operand b, int blocks_a) {
+    if (int(blockIdx.x) < blocks_a) split_any(a, blockIdx.x);
+    else split_any(b, blockIdx.x - blocks_a);
+}
+
+// ---- launch 3: the GEMM ----------------------------------------------------------------
+struct PlaneArgs {
+    const uint8_t *A, *B;
+    const int *ea, *eb;
+    Src sa, sb;           // the original operands, for rows with an infinity or NaN
+    const float* bias;
+    float* out;
+    int M, N;             // rows of A, rows of B; out is [M, N]
+    int stages;           // a multiple of 2
+    int tiles_m, tiles_n;
+    int full, per_full;   // tiles computed whole, and how many of them an XCD takes
+    int splits, per_part; // the other tiles: c in `splits` parts, and an XCD's share of the parts
+    float* part;          // their sums: [tile - full][part][wave][float4 of the accumulators][lane]
+    int accumulate;
+};
+
+constexpr int RING = 4;
+constexpr int GROUP_M = 8;   // tile rows of the order inside an XCD
+
+template <int WM_, int WN_, int MT_, int NT_>
+struct Geo {
+    static constexpr int WM = WM_, WN = WN_, MT = MT_, NT = NT_;
+    static constexpr int WAVES = WM * WN;
+    static constexpr int TM = WM * MT * 32, TN = WN * NT * 32;
+    static constexpr int UNITS = (TM + TN) / 32 * 2;   // 1 KB loads of a stage
+    static constexpr int UPW = UNITS / WAVES;
+    static constexpr int STAGE = UNITS * 1024;
+    static constexpr int LDS = RING * STAGE + (TM + TN) * 4;
+    static_assert(UNITS % WAVES == 0, "");
+};
+
+__device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+}
+
+// Tile L of the order: groups of GROUP_M tile rows, column after column, so
+// that the tiles an XCD runs at once share their strips in its L2.
+__device__ __forceinline__ void tile_at(const PlaneArgs& a, int L, int& ti, int& tj) {
+    const int group = L / (GROUP_M * a.tiles_n);
+    const int gm = min(GROUP_M, a.tiles_m - group * GROUP_M);
+    const int within = L - group * GROUP_M * a.tiles_n;
+    ti = group * GROUP_M + within % gm;
+    tj = within / gm;
+}
+
+// Stores one 32 x 32 tile of sums at (r0, c0). Lane l holds column l % 32,
+// rows 8 (e / 4) + 4 (l / 32) + e % 4. ea: the rows' exponents from r0.
+__device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r0, int c0, const int* ea, int eb) {
+    const int lane = threadIdx.x & 63, q = lane >> 5;
+    const int M = a.M, N = a.N, c = c0 + (lane & 31);
+    const float bv = a.bias ? a.bias[min(c, N - 1)] : 0.0f;
+    int er[16];
+    bool odd = eb == kFlag;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        er[e] = ea[8 * (e >> 2) + 4 * q + (e & 3)];
+        odd = odd || er[e] == kFlag;
+        acc[e] = ldexpf(acc[e], -(er[e] + eb));
+    }
+    if (a.bias) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] += bv;
+    }
+    float* o = a.out + int64_t(r0 + 4 * q) * N + c;
+    if (r0 + 32 <= M && c0 + 32 <= N && !__any(odd)) {
+        if (a.accumulate) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[e] += o[int64_t(8 * (e >> 2) + (e & 3)) * N];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[int64_t(8 * (e >> 2) + (e & 3)) * N] = acc[e];
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int r = r0 + 8 * (e >> 2) + 4 * q + (e & 3);
+        if (r < M && c < N && er[e] != kFlag && eb != kFlag) {
+            float* at = o + int64_t(8 * (e >> 2) + (e & 3)) * N;
+            *at = a.accumulate ? *at + acc[e] : acc[e];
+        }
+    }
+    if (!__any(odd) || c >= N) return;
+    for (int e = 0; e < 16; ++e) {   // from the operands, in fp32
+        const int lr = 8 * (e >> 2) + 4 * q + (e & 3), r = r0 + lr;
+        if (r >= M || (ea[lr] != kFlag && eb != kFlag)) continue;
+        float v = 0.0f;
+        for (int k = 0; k < a.sa.C; ++k) v = __builtin_fmaf(elem(a.sa, r, k), elem(a.sb, c, k), v);
+        v += bv;
+        float* at = a.out + int64_t(r) * N + c;
+        *at = a.accumulate ? *at + v : v;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) {
+    constexpr int MT = T::MT, NT = T::NT;
+    extern __shared__ __align__(16) uint8_t smem[];
+    int* exps = reinterpret_cast<int*>(smem + RING * T::STAGE);
+    const int t = threadIdx.x;
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave / T::WN, wn = wave % T::WN;
+
+    // XCD x (workgroups x, x + 8, ...) takes a run of the whole tiles, then a
+    // run of the parts.
+    const int b = int(blockIdx.x), nfull = a.per_full * 8;
+    const bool whole = b < nfull;
+    int L, part = 0;
+    if (whole) {
+        L = (b & 7) * a.per_full + (b >> 3);
+        if (L >= a.full) return;
+    } else {
+        const int u = ((b - nfull) & 7) * a.per_part + ((b - nfull) >> 3);
+        L = a.full + u / a.splits;
+        part = u % a.splits;
+        if (L >= a.tiles_m * a.tiles_n) return;
+    }
+    const int pairs = a.stages >> 1;
+    const int first = whole ? 0 : 2 * (part * pairs / a.splits);
+    const int end = whole ? a.stages : 2 * ((part + 1) * pairs / a.splits);
+    int ti, tj;
+    tile_at(a, L, ti, tj);
+    const int m0 = ti * T::TM, n0 = tj * T::TN;
+
+    for (int i = t; i < T::TM + T::TN; i += 64 * T::WAVES)
+        exps[i] = i < T::TM ? a.ea[m0 + i] : a.eb[n0 + i - T::TM];
+
+    // This wave's loads of a stage: units wave * UPW ..; unit u is part u % 2
+    // of the tile's 32-row block u / 2 (A's blocks, then B's).
+    const uint8_t* src[T::UPW];
+    const int64_t strip = int64_t(a.stages) * 2048;
+#pragma unroll
+    for (int i = 0; i < T::UPW; ++i) {
+        const int u = wave * T::UPW + i, blk = u >> 1;
+        src[i] = (blk < T::TM / 32 ? a.A + (m0 / 32 + blk) * strip : a.B + (n0 / 32 + blk - T::TM / 32) * strip) +
+                 (u & 1) * 1024;
+    }
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(smem));
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    auto issue = [&](int s) {   // past the last stage: the last one again, never read
+        const uint32_t off = uint32_t(min(s, end - 1)) * 2048u + uint32_t(lane) * 16u;
+        const uint32_t lds = lds0 + uint32_t(s & (RING - 1)) * T::STAGE + uint32_t(wave * T::UPW) * 1024u;
+#pragma unroll
+        for (int i = 0; i < T::UPW; ++i)
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + i * 1024), "v"(off),
+                         "s"(src[i])
+                         : "memory", "m0");
+    };
+#pragma clang diagnostic pop
+
+    struct Frags {
+        u32x4 a[MT][2], b[NT][2];
+    };
+    auto fetch = [&](int s, Frags& f) {
+        const uint8_t* st = smem + (s & (RING - 1)) * T::STAGE + lane * 16;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                f.a[i][p] = *reinterpret_cast<const u32x4*>(st + (wm * MT + i) * 2048 + p * 1024);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                f.b[j][p] = *reinterpret_cast<const u32x4*>(st + (T::TM / 32 + wn * NT + j) * 2048 + p * 1024);
+    };
+    // The matrix unit rounds once per 8 products. hh is summed apart from
+    // hl + lh, whose roundings are then 2^-11 of those of the sum.
+    f32x16 acc[MT][NT], low[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.0f;
+    auto multiply = [&](const Frags& f) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] = mfma(f.a[i][0], f.b[j][0], acc[i][j]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) low[i][j] = mfma(f.a[i][0], f.b[j][1], low[i][j]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) low[i][j] = mfma(f.a[i][1], f.b[j][0], low[i][j]);
+    };
+
+    __syncthreads();   // exps; and no plain load is in flight when the counted ones start
+    issue(first);
+    issue(first + 1);
+    issue(first + 2);
+    Frags f0, f1;
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * T::UPW) : "memory");
+    fetch(first, f0);
+    // Step s: the fragments of stage s are in `cur`. Stage s + 1 has landed
+    // once at most stage s + 2's loads are in flight; past the barrier that
+    // holds for every wave, and the ring slot of stage s - 1 is free (its
+    // fragments were used before the barrier).
+    auto step = [&](int s, const Frags& cur, Frags& nxt) {
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(T::UPW) : "memory");
+        issue(s + 3);
+        fetch(s + 1, nxt);
+        multiply(cur);
+    };
+    for (int s = first; s < end; s += 2) {
+        step(s, f0, f1);
+        step(s + 1, f1, f0);
+    }
+    // No direct-to-LDS load may outlive the workgroup's LDS.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            acc[i][j] += low[i][j];
+            if (whole) {
+                const int lr = (wm * MT + i) * 32, lc = (wn * NT + j) * 32;
+                store_tile(a, acc[i][j], m0 + lr, n0 + lc, exps + lr, exps[T::TM + lc + (lane & 31)]);
+            } else {
+                f32x4* o = reinterpret_cast<f32x4*>(a.part) +
+                           ((int64_t(L - a.full) * a.splits + part) * T::WAVES + wave) * (MT * NT * 4 * 64) +
+                           (i * NT + j) * 4 * 64 + lane;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o[e * 64] = f32x4{acc[i][j][4 * e], acc[i][j][4 * e + 1], acc[i][j][4 * e + 2],
+                                      acc[i][j][4 * e + 3]};
+            }
+        }
+}
+
+// The parts of the split tiles, added in order: one wave per 32 x 32 tile.
+template <typename T>
+__global__ __launch_bounds__(256) void part_sum_kernel(PlaneArgs a) {
+    constexpr int SUB = T::MT * T::NT;
+    const int lane = threadIdx.x & 63;
+    const int u = int(blockIdx.x) * 4 + (threadIdx.x >> 6);   // (tile, wave, subtile)
+    const int sub = u % SUB, wave = u / SUB % T::WAVES, tile = u / (SUB * T::WAVES);
+    int ti, tj;
+    tile_at(a, a.full + tile, ti, tj);
+    const int r0 = ti * T::TM + (wave / T::WN * T::MT + sub / T::NT) * 32;
+    const int c0 = tj * T::TN + (wave % T::WN * T::NT + sub % T::NT) * 32;
+    if (r0 >= a.M || c0 >= a.N) return;
+    f32x16 acc;
+    for (int p = 0; p < a.splits; ++p) {
+        const f32x4* o = reinterpret_cast<const f32x4*>(a.part) +
+                         ((int64_t(tile) * a.splits + p) * T::WAVES + wave) * (SUB * 4 * 64) + sub * 4 * 64 + lane;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const f32x4 v = o[e * 64];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[4 * e + k] = p == 0 ? v[k] : acc[4 * e + k] + v[k];
+        }
+    }
+    store_tile(a, acc, r0, c0, a.ea + r0, a.eb[c0 + (lane & 31)]);
+}
+
+template <typename T>
+int launch_gemm(dgm_gpu* g, const PlaneArgs& a) {
+    auto kern = plane_gemm_kernel<T>;
+    if (T::LDS > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
+        if (e != hipSuccess)
+            return dgm::fail(g, DGM_ERR_HIP, "plane gemm: cannot reserve %d bytes of LDS: %s", T::LDS,
+                             hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(kern, dim3(unsigned(a.per_full + a.per_part) * 8u), dim3(64 * T::WAVES), T::LDS, g->stream, a);
+    const int cut = a.tiles_m * a.tiles_n - a.full;
+    if (cut > 0)
+        hipLaunchKernelGGL(part_sum_kernel<T>, dim3(unsigned(cut) * (T::MT * T::NT * T::WAVES / 4)), dim3(256), 0,
+                           g->stream, a);
+    return DGM_OK;
+}
+
+// Tiles of 8 waves (128 x 256, 256 x 128: one workgroup per CU) and of 4
+// (128 x 128: two).
+using Wide = Geo<2, 4, 2, 2>;
+using Tall = Geo<4, 2, 2, 2>;
+using Small = Geo<2, 2, 2, 2>;
+
+struct Tile {
+    int tm, tn, slots;   // slots: workgroups a CU holds
+};
+constexpr Tile kTiles[] = {{128, 256, 1}, {256, 128, 1}, {128, 128, 2}};
+
+int64_t round_up(int64_t v, int64_t to) { return (v + to - 1) / to * to; }
+
+// How a product is cut into tiles and parts, and its time in microseconds.
+// Measured on 256 CUs (one 16-c stage of every busy slot): 128 x 256 tiles
+// 0.36 us with few CUs busy and 0.62 us with all (the clock falls under the
+// matrix load), 128 x 128 tiles 0.26 us alone on a CU and 0.70 us for the two
+// of a CU. A round also fills and drains (4 us). Where the tiles leave the
+// last round partly empty, that round's tiles are cut along c; the sums of
+// the parts cost a launch and their traffic. Whole against cut, same run:
+// 517 x 4100 x 4128 134 -> 93 us, 1024 x 512 x 2048 69 -> 31 us, the dW of
+// 12288 rows at 1536 x 384 with its dX and forward 531 -> 286 us.
+struct Plan {
+    int tile;
+    int64_t tiles, full;   // all; computed whole (the others in `splits` parts)
+    int splits;
+    double us;
+};
+
+double round_us(int tile, int64_t units, int cus, double stages) {
+    const double busy = std::min(1.0, double(units) / cus);
+    if (tile < 2) return 4.0 + (0.36 + 0.26 * busy) * stages;
+    return 4.0 + (units <= cus ? 0.26 + 0.10 * busy : 0.70) * stages;
+}
+
+double rounds_us(int tile, int64_t units, int cus, double stages) {
+    const int64_t slots = int64_t(cus) * kTiles[tile].slots;
+    const int64_t rest = units % slots;
+    return double(units / slots) * round_us(tile, slots, cus, stages) +
+           (rest ? round_us(tile, rest, cus, stages) : 0.0);
+}
+
+Plan plan_for(int64_t M, int64_t N, int64_t stages, int cus) {
+    Plan best{0, 0, 0, 1, 1e30};
+    for (int tile = 0; tile < 3; ++tile) {
+        const Tile& t = kTiles[tile];
+        const int64_t tiles = int64_t(dgm::ceil_div(M, t.tm)) * dgm::ceil_div(N, t.tn);
+        const double us = rounds_us(tile, tiles, cus, double(stages));
+        if (us < best.us) best = Plan{tile, tiles, tiles, 1, us};
+        const int64_t slots = int64_t(cus) * t.slots, full = tiles / slots * slots, cut = tiles - full;
+        for (int s = 2; s <= 8 && cut > 0 && stages / s >= 16; ++s) {
+            const double cut_us = rounds_us(tile, full, cus, double(stages)) +
+                                  rounds_us(tile, cut * s, cus, double(stages) / s) + 4.0 +
+                                  double(cut) * s * t.tm * t.tn * 8.0 / 4e6;
+            if (cut_us < best.us) best = Plan{tile, tiles, full, s, cut_us};
+        }
+    }
+    return best;
+}
+
+Operand operand(const Src& s, int tile, int64_t stages) {
+    Operand o{};
+    o.s = s;
+    o.rb = int(round_up(s.R, tile) / 32);
+    o.kb = int(stages);
+    o.parts = s.col ? int(std::min<int64_t>(kMaxParts, std::max<int64_t>(1, s.C / 64))) : 1;
+    o.width = s.col && s.bits != 32 ? s.groups : s.R;
+    return o;
+}
+
+MaxArg max_arg(const Operand& o) {
+    MaxArg m{};
+    const Src& s = o.s;
+    const bool codes = s.bits != 32;
+    m.p = codes ? s.scale : static_cast<const float*>(s.p);
+    m.ld = codes ? s.groups : s.ld;
+    m.col = s.col;
+    m.parts = o.parts;
+    m.out = o.part;
+    m.R = o.width;
+    m.C = codes && !s.col ? s.groups : s.C;
+    m.lpr = m.C >= 512 ? 64 : m.C >= 128 ? 16 : 8;
+    m.blocks = s.col ? int(dgm::ceil_div(m.R, 64)) * o.parts : int(dgm::ceil_div(m.R, 256 / m.lpr));
+    return m;
+}
+
+// Where the pieces of a product lie in the plane buffer.
+struct Layout {
+    size_t planes_a, planes_b, exps_a, exps_b, max_a, max_b, parts, bytes;
+};
+
+Layout layout(const Operand& a, const Operand& b, int cut, int splits, const Tile& t) {
+    Layout l{};
+    auto take = [&](int64_t bytes) {
+        const size_t at = l.bytes;
+        l.bytes += size_t(round_up(bytes, 256));
+        return at;
+    };
+    l.planes_a = take(int64_t(a.rb) * a.kb * 2048);
+    l.planes_b = take(int64_t(b.rb) * b.kb * 2048);
+    l.exps_a = take(int64_t(a.rb) * 128);
+    l.exps_b = take(int64_t(b.rb) * 128);
+    l.max_a = take(int64_t(a.parts) * a.width * 4);
+    l.max_b = take(int64_t(b.parts) * b.width * 4);
+    l.parts = take(int64_t(cut) * splits * t.tm * t.tn * 4);
+    return l;
+}
+
+int64_t stages_of(int64_t C) { return round_up(dgm::ceil_div(C, 16), 2); }
+
+// out[M, N] (+)= A B^T (+ bias); kNotFused, launching nothing,
+// without a plane buffer.
+int run(dgm_gpu* g, const Src& sa, const Src& sb, const float* bias, float* out, bool accumulate) {
+    const int64_t stages = stages_of(sa.C);
+    const Plan plan = plan_for(sa.R, sb.R, stages, g->num_cus);
+    if (plan.tiles > (1 << 24)) return dgm::kNotFused;   // 32-bit tile numbers
+    const Tile& tile = kTiles[plan.tile];
+    Operand a = operand(sa, tile.tm, stages), b = operand(sb, tile.tn, stages);
+    const int cut = int(plan.tiles - plan.full);
+    const Layout at = layout(a, b, cut, plan.splits, tile);
+    uint8_t* ws = dgm::planes_buffer(g, at.bytes);
+    if (!ws) return dgm::kNotFused;
+    a.planes = ws + at.planes_a;
+    b.planes = ws + at.planes_b;
+    a.exps = reinterpret_cast<int*>(ws + at.exps_a);
+    b.exps = reinterpret_cast<int*>(ws + at.exps_b);
+    a.part = reinterpret_cast<uint32_t*>(ws + at.max_a);
+    b.part = reinterpret_cast<uint32_t*>(ws + at.max_b);
+    const MaxArg x = max_arg(a), y = max_arg(b);
+    hipLaunchKernelGGL(row_max_kernel, dim3(unsigned(x.blocks + y.blocks)), dim3(256), 0, g->stream, x, y);
+    const int ba = a.rb * int(dgm::ceil_div(a.kb, 16)), bb = b.rb * int(dgm::ceil_div(b.kb, 16));
+    hipLaunchKernelGGL(split_kernel, dim3(unsigned(ba + bb)), dim3(256), 0, g->stream, a, b, ba);
+    PlaneArgs p{};
+    p.A = a.planes;
+    p.B = b.planes;
+    p.ea = a.exps;
+    p.eb = b.exps;
+    p.sa = sa;
+    p.sb = sb;
+    p.bias = bias;
+    p.out = out;
+    p.M = sa.R;
+    p.N = sb.R;
+    p.stages = int(stages);
+    p.tiles_m = a.rb * 32 / tile.tm;
+    p.tiles_n = b.rb * 32 / tile.tn;
+    p.full = int(plan.full);
+    p.per_full = (p.full + 7) / 8;
+    p.splits = plan.splits;
+    p.per_part = (cut * plan.splits + 7) / 8;
+    p.part = reinterpret_cast<float*>(ws + at.parts);
+    p.accumulate = accumulate;
+    if (plan.tile == 0) return launch_gemm<Wide>(g, p);
+    if (plan.tile == 1) return launch_gemm<Tall>(g, p);
+    return launch_gemm<Small>(g, p);
+}
+
+Src dense(const float* p, int R, int C, int64_t ld, int col) {
+    Src s{};
+    s.p = p;
+    s.ld = ld;
+    s.R = R;
+    s.C = C;
+    s.bits = 32;
+    s.col = col;
+    s.G = 1;
+    s.vec = (ld & 3) == 0 && dgm::aligned(p, 16);
+    return s;
+}
+
+// The weights [N, K]: rows n over k (col 0), or rows k over n (col 1).
+Src weights(int bits, const void* W, const float* scale, const dgm_GemmP* p, int col) {
+    const int N = int(p->N), K = int(p->K);
+    if (bits == 32) return dense(static_cast<const float*>(W), col ? K : N, col ? N : K, K, col);
+    Src s{};
+    s.p = W;
+    s.scale = scale;
+    s.ld = K;
+    s.R = col ? K : N;
+    s.C = col ? N : K;
+    s.bits = bits;
+    s.col = col;
+    s.G = int(p->qGroup);
+    s.groups = K / s.G;
+    s.vec = K % 8 == 0 && s.G % 8 == 0 && dgm::aligned(W, 8);
+    return s;
+}
+
+}  // namespace
+
+namespace dgm {
+
+// Where three launches and the planes' traffic cost less than they save. The
+// fp32 MFMA kernels run at 43-57 TFLOP/s from about 2^28 products on; the
+// planes take 18 us and more before the first MFMA. Measured: 256 x 1024 x 1024
+// (2^28) 10.8 us against 23, 512 x 1024 x 768 dX + dW 37 against 62,
+// 1024 x 2048 x 512 (2^30) 35 against 26, 1024 x 512 x 2048 51 against 30,
+// 128 x 14336 x 4096 307 against 130.
+bool planes_pay(int64_t M, int64_t N, int64_t K) {
+    return M >= 128 && N >= 128 && K >= 128 && double(M) * double(N) * double(K) >= double(int64_t(7) << 27);
+}
+
+int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias,
+               float* Y, const dgm_GemmP* p) {
+    return run(g, dense(X, int(p->M), int(p->K), p->K, 0), weights(bits, W, scale, p, 0),
+               p->hasBias ? bias : nullptr, Y, false);
+}
+
+int planes_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, float* dX,
+              const dgm_GemmP* p) {
+    return run(g, dense(dY, int(p->M), int(p->N), p->N, 0), weights(bits, W, scale, p, 1), nullptr, dX, false);
+}
+
+int planes_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p, bool accumulate) {
+    return run(g, dense(dY, int(p->N), int(p->M), p->N, 1), dense(X, int(p->K), int(p->M), p->K, 1), nullptr, dW,
+               accumulate);
+}
+
+}  // namespace dgm

@@ -158,7 +158,9 @@ int dgm_gemmNT(dgm_gpu* g, int64_t bits, const float* w, const void* q,
 /* No counterpart in the reference: dgm_gemmNT for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). Same arguments, kernels and results
- * (bitwise) as dgm_gemmNT, but every staging buffer (the decode kernels'
+ * (bitwise; where dgm_gemmNT takes the f16 pieces of large products, this
+ * entry takes the kernels that stage nothing, with the same error bound) as
+ * dgm_gemmNT, but every staging buffer (the decode kernels'
  * activation pieces, the bf16 copy of X of the reduced-precision prefill
  * path) comes from a static device scratch of DGM_NOALLOC_SCRATCH_BYTES per
  * GPU, held from library load until the process ends; nothing is allocated.
@@ -179,12 +181,20 @@ int dgm_gemmNT_noalloc(dgm_gpu* g, int64_t bits, const float* w, const void* q,
  * buffers (activation pieces of the decode-shaped kernels, partial sums of the
  * K-sliced kernel, the bf16 copy of X of the prefill path) come from a
  * workspace of the context that is otherwise allocated by the first call that
- * needs it. dgm_gemmNT_workspace_bound returns bytes that cover every path a
+ * needs it; the f16 pieces of large products (dX and dW among them) from a
+ * second buffer of the context, which calls under graph capture do not use
+ * (they, and calls for which no memory is left, take the kernels that stage
+ * nothing). A call on another stream than the last one to use that buffer
+ * waits for that one. dgm_gemmNT_workspace_bound returns bytes that cover every path a
  * dgm_gemmNT call of that shape can take, in either math mode (-1 for
- * negative sizes); dgm_gpu_reserve grows the workspace to at least `bytes`
+ * negative sizes); dgm_gpu_reserve grows both buffers to at least `bytes`
  * now (DGM_ERR_UNSUPPORTED during a graph capture), so that later calls whose
- * bound it covers allocate nothing; dgm_gpu_workspace_bytes returns its size
- * (0 before anything was allocated). */
+ * bound it covers allocate nothing (the bound leaves the f16 pieces out: after
+ * a reserve, large products whose pieces do not fit the reserved bytes take
+ * the kernels that stage nothing; they need 4 bytes for each element of both
+ * operands, rows padded to 256, and some tens of MB of partial sums);
+ * dgm_gpu_workspace_bytes returns the size of both (0 before anything was
+ * allocated). */
 int64_t dgm_gemmNT_workspace_bound(int64_t M, int64_t N, int64_t K);
 int dgm_gpu_reserve(dgm_gpu* g, int64_t bytes);
 int64_t dgm_gpu_workspace_bytes(const dgm_gpu* g);

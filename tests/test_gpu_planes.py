@@ -1,0 +1,193 @@
+"""The large products on split operands (csrc/gemm_planes.hip): forward, dX and dW.
+
+Sizes sit at the edges of its tiles (128 and 256 rows), stages (16 and 32 of
+the contraction) and parts (tiles cut along the contraction), on both sides of
+where it is taken (7 * 2^27 products). The reference is the float64 product of
+the same operands. Bound per element, against the row's and column's 2-norms
+|a| |b| (every element of a split operand is within 2^-24 of its value, and a
+sum of n products, rounded once per 8, is within n/8 * 2^-24 of |a| |b| at
+worst): (2 + n / 8) * 2^-24 |a| |b|.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(gpu, bits, M, N, K, G, seed):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    dy = torch.randn(M, N, generator=g, device="cuda") * 1e-3
+    w = torch.randn(N, K, generator=g, device="cuda") * 0.02
+    bias = torch.randn(N, generator=g, device="cuda")
+    if bits == 32:
+        return x, dy, w, None, None, w.double(), bias
+    q = torch.empty(N * K // (2 if bits == 4 else 1), dtype=torch.uint8, device="cuda")
+    s = torch.empty(N * (K // G), device="cuda")
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.quantize(w, q, s, N, K, bits, G)
+    gpu.end()
+    if bits == 8:
+        codes = q.view(torch.int8).double()
+    else:
+        lo, hi = (q << 4).view(torch.int8) >> 4, q.view(torch.int8) >> 4
+        codes = torch.stack([lo, hi], dim=1).reshape(-1).double()
+    wd = (codes.reshape(N, K // G, G) * s.double().reshape(N, K // G, 1)).reshape(N, K)
+    return x, dy, w, q, s, wd, bias
+
+
+def _within(got, ref, a, b, n):
+    """got against ref = a b^T (a [R, n], b [C, n]), where ref is finite."""
+    import torch
+    bound = (2 + n / 8) * 2.0 ** -24 * a.norm(dim=1)[:, None] * b.norm(dim=1)[None, :] + 2.0 ** -149
+    return bool(((got.double() - ref).abs() <= bound + ref.abs() * 2.0 ** -24).all()) and torch.isfinite(got).all()
+
+
+SHAPES = [   # bits, M, N, K, G
+    (8, 1024, 1024, 1024, 8),       # groups smaller than a stage
+    (4, 1025, 1023, 1024, 32),      # one row above a tile, one column below
+    (4, 129, 8191, 1024, 64),       # a last tile of one row; odd N
+    (32, 1537, 385, 2040, 8),       # a contraction that is no multiple of a stage
+    (8, 130, 2050, 4100, 10),       # groups of 10: no vector loads
+    (4, 128, 14336, 1026, 18),      # odd row bytes for int4
+    (8, 517, 640, 4128, 32),        # few tiles: cut along the contraction
+    (4, 2048, 4352, 256, 128),      # whole tiles and a cut last round
+]
+
+
+@pytest.mark.parametrize("bits,M,N,K,G", SHAPES)
+def test_products(gpu, bits, M, N, K, G):
+    import torch
+    x, dy, w, q, s, wd, bias = _inputs(gpu, bits, M, N, K, G, M + N)
+    y, dx = (torch.full(sh, float("nan"), device="cuda") for sh in ((M, N), (M, K)))
+    dw0 = torch.randn(N, K, device="cuda")
+    dw, acc = torch.full((N, K), float("nan"), device="cuda"), dw0.clone()
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.gemmNT(bits, w, q, s, x, bias, y, M, N, K, G)
+    gpu.gemmDX(bits, w, q, s, dy, dx, M, N, K, G)
+    gpu.gemmDW(dy, x, dw, M, N, K)
+    gpu.gemmDWAcc(dy, x, acc, M, N, K)
+    gpu.end()
+    xd, dyd = x.double(), dy.double()
+    assert _within(y, xd @ wd.T + bias.double(), xd, wd, K)
+    assert _within(dx, dyd @ wd, dyd, wd.T.contiguous(), N)
+    ref = dyd.T.contiguous() @ xd
+    assert _within(dw, ref, dyd.T.contiguous(), xd.T.contiguous(), M)
+    assert _within(acc, ref + dw0.double(), dyd.T.contiguous(), xd.T.contiguous(), M)
+    # gemmBwd is the two calls, bitwise.
+    dx2, dw2 = torch.empty_like(dx), torch.empty_like(dw)
+    gpu.begin()
+    gpu.gemmBwd(bits, w, q, s, dy, x, dx2, dw2, M, N, K, G)
+    gpu.end()
+    assert torch.equal(dx, dx2) and torch.equal(dw, dw2)
+
+
+@pytest.mark.parametrize("kind", ["nonfinite", "rows", "tiny", "zeros"])
+def test_values(gpu, kind):
+    """Infinities and NaN land where the products of the operands put them;
+    rows of very different size each keep their own precision."""
+    import torch
+    bits, M, N, K, G = 4, 1030, 1000, 1024, 32
+    x, dy, w, q, s, wd, _ = _inputs(gpu, bits, M, N, K, G, 5)
+    if kind == "nonfinite":
+        x[3, 5], x[7, 9], x[11, 2], dy[4, 6], dy[1029, 999] = float("inf"), -float("inf"), float("nan"), float("inf"), \
+            float("nan")
+    elif kind == "rows":
+        x *= torch.exp2(torch.randint(-60, 60, (M, 1), device="cuda").float())
+        dy *= torch.exp2(torch.randint(-30, 30, (1, N), device="cuda").float())
+    elif kind == "tiny":
+        x *= 1e-38
+        dy *= 1e-6
+    else:
+        x[5], x[:, 3], dy[8], dy[:, 2] = 0, 0, 0, 0
+    y, dx, dw = (torch.full(sh, 7.0, device="cuda") for sh in ((M, N), (M, K), (N, K)))
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.gemmNT(bits, w, q, s, x, None, y, M, N, K, G)
+    gpu.gemmBwd(bits, w, q, s, dy, x, dx, dw, M, N, K, G)
+    gpu.end()
+    xd, dyd = x.double(), dy.double()
+    for got, a, b, n in ((y, xd, wd, K), (dx, dyd, wd.T.contiguous(), N),
+                         (dw, dyd.T.contiguous(), xd.T.contiguous(), M)):
+        ref = a @ b.T
+        if kind == "nonfinite":
+            assert torch.equal(torch.isnan(got), torch.isnan(ref))
+            inf = torch.isinf(ref)
+            assert torch.equal(torch.isinf(got), inf) and torch.equal(got[inf].double(), ref[inf])
+            assert not torch.isfinite(ref).all()
+            ra, cb = torch.isfinite(a).all(1), torch.isfinite(b).all(1)
+            got, ref, a, b = got[ra][:, cb], ref[ra][:, cb], a[ra], b[cb]
+        if kind == "tiny":      # results below 2^-126 keep an absolute 2^-149
+            assert bool(((got.double() - ref).abs() <= (2 + n / 8) * 2.0 ** -24 * a.norm(dim=1)[:, None] *
+                         b.norm(dim=1)[None, :] + 2.0 ** -148).all())
+        else:
+            assert _within(got, ref, a, b, n)
+
+
+def test_buffer_capture_and_streams(dgm, gpu, torch_cuda):
+    """Calls that alternate between two streams give the same product; a
+    captured call, dgm_gemmNT_noalloc and a context that reserved less than
+    the planes take the kernels that stage nothing, and nothing is allocated."""
+    torch = torch_cuda
+    bits, M, N, K, G = 8, 1024, 2048, 1024, 32
+    x, _, w, q, s, wd, _ = _inputs(gpu, bits, M, N, K, G, 9)
+    ref = x.double() @ wd.T
+    st = [torch.cuda.Stream(), torch.cuda.Stream()]
+    ys = [torch.zeros(M, N, device="cuda") for _ in range(8)]
+    torch.cuda.synchronize()
+    g = dgm.GPU(stream=st[0])
+    try:
+        assert g.workspaceBytes() == 0
+        g.reserve(64 << 20)
+        held = g.workspaceBytes()
+        g.begin()
+        for i, y in enumerate(ys):      # each stream's call uses the one plane buffer
+            g.set_stream(st[i % 2])
+            g.gemmNT(bits, w, q, s, x, None, y, M, N, K, G)
+        g.end()
+        torch.cuda.synchronize()
+        assert g.workspaceBytes() == held
+        for y in ys:
+            assert _within(y, ref, x.double(), wd, K) and torch.equal(y, ys[0])
+        g.set_stream(st[0])
+        yc = torch.zeros(M, N, device="cuda")
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st[0]):
+            g.begin()
+            g.gemmNT(bits, w, q, s, x, None, yc, M, N, K, G)
+        for _ in range(3):
+            yc.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(st[0]):
+                graph.replay()
+            g.begin()
+            g.gemmNT(bits, w, q, s, x, None, ys[0], M, N, K, G)
+            g.end()
+            st[0].synchronize()
+            assert _within(yc, ref, x.double(), wd, K)
+        yn = torch.zeros(M, N, device="cuda")
+        torch.cuda.synchronize()
+        g.begin()
+        g.gemmNT_noalloc(bits, w, q, s, x, None, yn, M, N, K, G)
+        g.end()
+        assert torch.equal(yn, yc)
+        assert g.workspaceBytes() == held
+        small = dgm.GPU(stream=st[0])
+        small.reserve(small.gemmNT_workspace_bound(M, N, K))
+        held = small.workspaceBytes()
+        ys[1].zero_()
+        torch.cuda.synchronize()
+        small.begin()
+        small.gemmNT(bits, w, q, s, x, None, ys[1], M, N, K, G)
+        small.end()
+        assert torch.equal(ys[1], yc) and not torch.equal(ys[0], yc) and small.workspaceBytes() == held
+        small.close()
+        del graph
+    finally:
+        torch.cuda.synchronize()
+        g.close()
