@@ -287,6 +287,7 @@ struct AttnBwdArgs {
     float *dq, *dk, *dv, *dprobs, *dscores;
     int B, T, H, D;
     float scale;
+    bool keep_dp;   // dprobs is read by the caller
 };
 
 __global__ __launch_bounds__(kThreads) void attn_bwd_dv_kernel(AttnBwdArgs a) {
@@ -675,6 +676,172 @@ bool attn_bwd_fused_ok(const AttnBwdArgs& a) {
            dgm::aligned(a.dprobs, 16);
 }
 
+// ---- attention backward of long heads on fp32 MFMA --------------------------------
+// For T and D multiples of 16 whose head does not fit the kernels above
+// (T = 256, D = 64: 2 T D floats are 128 KB), two launches on
+// v_mfma_f32_16x16x4_f32:
+//  * rows kernel, workgroup (b, h, 16 query rows): dP = dO V^T into LDS with
+//    the row dots, dS = P (dP - dot), then dQ = scale dS K from LDS;
+//  * keys kernel, workgroup (b, h, 16 key rows, 64 columns): dV = P^T dO and
+//    dK = scale dS^T Q, a quarter of the rows t to each wave (which shares its
+//    P and dS operands over all the column tiles), the quarters added in LDS.
+// A contraction's index order is free as long as both operands agree, so where
+// a row is contiguous along it a lane takes four consecutive k in one 16-byte
+// load. What bounds them is moving K, V, Q and dO of the head from L2 into
+// each of its T / 16 workgroups (128 KB at T = 256, D = 64). 4 x 256 tokens,
+// 8 heads of 64 (1.07 GFLOP a call): 31 + 17 us; the five passes of one thread
+// per output, which still take the sizes left over, 89 + 443 + 194 + 88 + 88.
+constexpr int kAmThreads = 256;
+constexpr int kAmMaxT = 960;    // 16 (T + 4) floats of LDS within 64 KB
+constexpr int kAmMaxD = 128;    // dO operands of a lane: D / 16 float4
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+bool attn_mfma_bwd_ok(const AttnBwdArgs& a) {
+    return a.T % 16 == 0 && a.D % 16 == 0 && a.T <= kAmMaxT && a.D <= kAmMaxD && dgm::aligned(a.v, 16) &&
+           dgm::aligned(a.dout, 16);
+}
+
+__global__ __launch_bounds__(kAmThreads) void attn_mfma_rows_kernel(AttnBwdArgs a) {
+    extern __shared__ __align__(16) float lds[];
+    const int T = a.T, D = a.D, H = a.H, ld = T + 4;
+    float* S = lds;               // dP, then dS: [16][ld]
+    float* dots = S + 16 * ld;    // [4 waves][16], then the row dots in [0][..]
+    const int nblk = T / 16;
+    const int bh = blockIdx.x / nblk, t0 = blockIdx.x % nblk * 16;
+    const int b = bh / H, h = bh % H;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
+    const int64_t row = int64_t(H) * D;
+    const int64_t head0 = (int64_t(b) * T * H + h) * D;
+    const int64_t pm0 = (int64_t(bh) * T + t0) * T;
+
+    // dP tiles of 16 keys: wave w takes w, w + 4, ...
+    f32x4 g[kAmMaxD / 16];
+    const float* gp = a.dout + head0 + (t0 + r16) * row + 4 * q4;
+#pragma unroll
+    for (int j = 0; j < kAmMaxD / 16; ++j)
+        if (j * 16 < D) g[j] = *reinterpret_cast<const f32x4*>(gp + j * 16);
+    float dot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = wave * 16; s0 < T; s0 += 64) {
+        const float* vp = a.v + head0 + (s0 + r16) * row + 4 * q4;
+        const float* pp = a.probs + pm0 + int64_t(4 * q4) * T + s0 + r16;
+        f32x4 v[kAmMaxD / 16];
+        float pr[4];
+#pragma unroll
+        for (int j = 0; j < kAmMaxD / 16; ++j)
+            if (j * 16 < D) v[j] = *reinterpret_cast<const f32x4*>(vp + j * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pr[e] = pp[e * T];
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < kAmMaxD / 16; ++j)
+            if (j * 16 < D) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(g[j][u], v[j][u], acc, 0, 0, 0);
+            }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            S[(4 * q4 + e) * ld + s0 + r16] = acc[e];
+            if (a.keep_dp) a.dprobs[pm0 + int64_t(4 * q4 + e) * T + s0 + r16] = acc[e];
+            dot[e] += acc[e] * pr[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1) dot[e] += __shfl_xor(dot[e], off, 16);
+        if (r16 == 0) dots[wave * 16 + 4 * q4 + e] = dot[e];
+    }
+    __syncthreads();
+    for (int i = tid; i < 16 * T; i += kAmThreads) {
+        const int r = i / T, s = i % T;
+        const float d = (dots[r] + dots[16 + r]) + (dots[32 + r] + dots[48 + r]);
+        const float ds = a.probs[pm0 + i] * (S[r * ld + s] - d);
+        S[r * ld + s] = ds;
+        a.dscores[pm0 + i] = ds;
+    }
+    __syncthreads();
+    for (int d0 = wave * 16; d0 < D; d0 += 64) {
+        const float* sp = S + r16 * ld + 4 * q4;
+        const float* kp = a.k + head0 + int64_t(4 * q4) * row + d0 + r16;
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+        for (int s0 = 0; s0 < T; s0 += 16) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(sp + s0);
+            float y[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) y[u] = kp[(s0 + u) * row];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a.dq[head0 + (t0 + 4 * q4 + e) * row + d0 + r16] = acc[e] * a.scale;
+    }
+}
+
+__global__ __launch_bounds__(kAmThreads) void attn_mfma_keys_kernel(AttnBwdArgs a) {
+    __shared__ f32x4 part[3][8][64];   // waves 1 .. 3
+    const int T = a.T, D = a.D, H = a.H;
+    const int nblk = T / 16;
+    const int bh = blockIdx.x / nblk, s0 = blockIdx.x % nblk * 16;
+    const int b = bh / H, h = bh % H;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, q4 = lane >> 4;
+    const int64_t row = int64_t(H) * D;
+    const int64_t head0 = (int64_t(b) * T * H + h) * D;
+    const int dbase = blockIdx.y * 64, nd = min(4, (D - dbase) / 16);
+    const int64_t pm0 = int64_t(bh) * T * T + s0 + r16;
+    const int tq = T / 4;
+    f32x4 accv[4], acck[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) accv[j] = acck[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int t = wave * tq + q4; t < (wave + 1) * tq; t += 4) {
+        const float p = a.probs[pm0 + int64_t(t) * T], ds = a.dscores[pm0 + int64_t(t) * T];
+        const int64_t at = head0 + t * row + dbase + r16;
+        float x[4], y[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x[j] = j < nd ? a.dout[at + j * 16] : 0.0f;
+            y[j] = j < nd ? a.q[at + j * 16] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            accv[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, x[j], accv[j], 0, 0, 0);
+            acck[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ds, y[j], acck[j], 0, 0, 0);
+        }
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            part[wave - 1][j][lane] = accv[j];
+            part[wave - 1][4 + j][lane] = acck[j];
+        }
+    }
+    __syncthreads();
+    // Wave w adds and stores column tile w.
+    const int j = wave;
+    if (wave == 0) {   // wave 0 keeps its sums in registers: hand the other tiles over
+#pragma unroll
+        for (int u = 1; u < 4; ++u) {
+            part[0][u][lane] += accv[u];
+            part[0][4 + u][lane] += acck[u];
+        }
+    }
+    __syncthreads();
+    if (j >= nd) return;
+    f32x4 v = part[0][j][lane] + part[1][j][lane] + part[2][j][lane];
+    f32x4 k = part[0][4 + j][lane] + part[1][4 + j][lane] + part[2][4 + j][lane];
+    if (wave == 0) {
+        v += accv[0];
+        k += acck[0];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int64_t at = head0 + (s0 + 4 * q4 + e) * row + dbase + j * 16 + r16;
+        a.dv[at] = v[e];
+        a.dk[at] = k[e] * a.scale;
+    }
+}
+
 // ---- rope_bwd (metal/kernels.metal:891-909) --------------------------------------
 __global__ __launch_bounds__(kThreads) void rope_bwd_kernel(const float* __restrict__ dy, float* __restrict__ dx,
                                                             const float* __restrict__ cosv,
@@ -837,6 +1004,14 @@ int launch_attn_bwd(dgm_gpu* g, const AttnBwdArgs& a) {
             return dgm::fail(g, DGM_ERR_HIP, "attn_bwd: cannot reserve %zu bytes of LDS: %s", lds,
                              hipGetErrorString(e));
         hipLaunchKernelGGL(attn_bwd_fused_kernel, dim3(unsigned(a.B * a.H)), dim3(kAbThreads), lds, g->stream, a);
+        return dgm::check_launch(g, "attn_bwd");
+    }
+    if (attn_mfma_bwd_ok(a)) {
+        const unsigned grid = unsigned(a.B) * unsigned(a.H) * unsigned(a.T / 16);
+        hipLaunchKernelGGL(attn_mfma_rows_kernel, dim3(grid), dim3(kAmThreads),
+                           (size_t(16) * (a.T + 4) + 64) * sizeof(float), g->stream, a);
+        hipLaunchKernelGGL(attn_mfma_keys_kernel, dim3(grid, unsigned((a.D + 63) / 64)), dim3(kAmThreads), 0, g->stream,
+                           a);
         return dgm::check_launch(g, "attn_bwd");
     }
     hipLaunchKernelGGL(attn_bwd_dv_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, g->stream, a);
@@ -1037,7 +1212,7 @@ int dgm_attnBwd(dgm_gpu* g, const float* q, const float* k, const float* v, cons
     if (B * T * H * D && (!q || !k || !v || !probs || !dout || !dq || !dk || !dv || !dprobs || !dscores))
         return dgm::fail(g, DGM_ERR_ARG, "attnBwd: null buffer");
     AttnBwdArgs a{q, k, v, probs, dout, dq, dk, dv, dprobs, dscores, int(B), int(T), int(H), int(D),
-                  D > 0 ? 1.0f / sqrtf(float(D)) : 0.0f};
+                  D > 0 ? 1.0f / sqrtf(float(D)) : 0.0f, true};
     return launch_attn_bwd(g, a);
 }
 
@@ -1406,8 +1581,9 @@ int dgm_dit_backward(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w,
                 return dgm::fail(g, DGM_ERR_UNSUPPORTED, "dit_backward: attention backward shape changed");
             DGM_TRY(ra);
         } else {
-            DGM_TRY(dgm_attnBwd(g, A(l, A_Q), A(l, A_K), A(l, A_V), A(l, A_PROBS), S[B_DAV], S[B_DQ], S[B_DK],
-                                S[B_DV], S[B_DPROBS], S[B_DSCORES], B, T, H, D));
+            const AttnBwdArgs ab{A(l, A_Q), A(l, A_K), A(l, A_V), A(l, A_PROBS), S[B_DAV], S[B_DQ], S[B_DK], S[B_DV],
+                                 S[B_DPROBS], S[B_DSCORES], B, T, H, D, 1.0f / sqrtf(float(D)), false};
+            DGM_TRY(launch_attn_bwd(g, ab));
             DGM_TRY(launch_qkv_grad(g, S[B_DQ], S[B_DK], S[B_DV], cosv, sinv, oq, ldq, ok, ldkv, ov, ldkv,
                                     S[B_DFIRST], B, T, H, D, l == 0, mix));
         }

@@ -250,3 +250,38 @@ def test_block_backward_rejects(gpu, dgm):
         finally:
             gpu.lib.dgm_end(gpu.h)
     assert e.value.code == dgm.DGM_ERR_SHAPE
+
+
+# Heads beyond the kernels above, T and D multiples of 16 (MFMA), at the edges
+# of their tiles: one column group of 64 and more, a part of one, odd counts of
+# 16-key tiles over the four waves. Bound: sums of n <= 288 products of which
+# each is rounded once or twice, and (for dq and dk) of dscores that are
+# themselves such sums: 2 n 2^-24 of the largest sum of absolute products.
+@pytest.mark.parametrize("B,T,H,D", [(1, 256, 2, 64), (2, 144, 1, 80), (1, 288, 3, 48), (1, 128, 2, 128), (1, 960, 1, 16)])
+def test_attn_bwd_long_heads(gpu, orc, B, T, H, D):
+    import torch
+    rng = np.random.default_rng(B * T + H * D)
+    n, tt = B * T * H * D, B * H * T * T
+    q, k, v, dout = (rng.standard_normal(n).astype(np.float32) for _ in range(4))
+    _, probs, _ = orc.attn_fwd(q, k, v, B, T, H, D, 0)
+    outs = [torch.full((m,), float("nan"), device="cuda") for m in (n, n, n, tt, tt)]
+    gpu.begin()
+    gpu.attnBwd(to_dev(q), to_dev(k), to_dev(v), to_dev(probs), to_dev(dout), *outs, B, T, H, D)
+    gpu.end()
+
+    def heads(a):
+        return a.astype(np.float64).reshape(B, T, H, D).transpose(0, 2, 1, 3)
+    Q, K, V, G, P = heads(q), heads(k), heads(v), heads(dout), probs.astype(np.float64).reshape(B, H, T, T)
+    t = lambda m: m.transpose(0, 1, 3, 2)  # noqa: E731
+    dP = G @ t(V)
+    dS = P * (dP - (dP * P).sum(-1, keepdims=True))
+    sc, eps = 1 / np.sqrt(D), 2.0 ** -24
+    bP = 2 * D * eps * (np.abs(G) @ t(np.abs(V)))
+    bS = P * (bP + (bP * P).sum(-1, keepdims=True)) + 2 * T * eps * P * (np.abs(dP) + (np.abs(dP) * P).sum(-1, keepdims=True))
+    refs = {"dq": (sc * dS @ K, sc * (bS @ np.abs(K) + 2 * T * eps * np.abs(dS) @ np.abs(K))),
+            "dk": (sc * t(dS) @ Q, sc * (t(bS) @ np.abs(Q) + 2 * T * eps * t(np.abs(dS)) @ np.abs(Q))),
+            "dv": (t(P) @ G, 2 * T * eps * t(P) @ np.abs(G)), "dprobs": (dP, bP), "dscores": (dS, bS)}
+    for (name, (ref, bound)), got in zip(refs.items(), outs):
+        got = from_dev(got)
+        got = got.reshape(B, H, T, T) if got.size == tt and name in ("dprobs", "dscores") else heads(got)
+        assert np.all(np.abs(got - ref) <= bound + 1e-30), (name, float(np.max(np.abs(got - ref) / (bound + 1e-30))))
