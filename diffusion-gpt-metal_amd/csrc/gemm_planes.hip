@@ -19,13 +19,18 @@
 // roundings are 2^-11 of those. Against 64 bits, the fp32 MFMA kernels first:
 // 2048 x 14336 x 4096 5.3e-7, 4.0e-7; dX and dW of 2048 x 4096 x 4096 5.7e-7
 // and 4.2e-7, 4.1e-7 and 3.1e-7; dW over 12288 rows 1.0e-6, 2.8e-7.
+// A forward whose codes come in groups of whole 32-c stages keeps them as one
+// plane (integers of 8 bits, exact in f16): h and l of x against the codes,
+// summed per group, and the sum goes to the accumulator times the group's
+// scale. Two products instead of three, and no rounding of code * scale: 1.4e-7
+// for the first case above.
 // Rows with an infinity or NaN are computed from the original operands in
 // fp32 (an infinity times a low piece of the other sign would be NaN).
 //
 // What it gains: v_mfma_f32_16x16x4_f32 peaks at 157 TFLOP/s and its kernels
 // here ran at 50-57; three f16 products per fp32 product at 2.5 PFLOP/s peak at
-// 833. Measured, both sides in turn: 2048 x 14336 x 4096 int4 4816 -> 656 us
-// (366 TFLOP/s), 517 x 4100 x 4128 int8 320 -> 93, dX + dW of 2048 x 4096 x
+// 833, two at 1250. Measured, both sides in turn: 2048 x 14336 x 4096 int4
+// 4816 -> 457 us (527 TFLOP/s), 517 x 4100 x 4128 int8 320 -> 77, dX + dW of 2048 x 4096 x
 // 4096 2416 -> 442, forward + dX + dW of fp32 12288 x 1536 x 384 779 -> 301.
 // What bounds it: the power the matrix unit draws. With zeros for data the
 // GEMM of 4096 x 4096 x 4096 takes 225 us instead of 320 (the clock stays up);
@@ -43,9 +48,9 @@
 // no bank conflicts, no swizzle), the rows are padded to whole tiles and c to
 // whole stages with zeros, and the GEMM has no bounds checks before its stores.
 //
-// GEMM: WM x WN waves, each MT x NT tiles of 32 x 32. A ring of four stages
-// of 16 c; a step waits for the next stage by count, meets the other waves,
-// issues the loads of the stage three ahead and reads the next stage's
+// GEMM: WM x WN waves, each MT x NT tiles of 32 x 32. A ring of three or four
+// stages of 16 or 32 c; a step waits for the next stage by count, meets the other waves,
+// issues the loads of the stage two or three ahead and reads the next stage's
 // fragments into registers while the MFMAs of the current one run, so the
 // load latency, the LDS latency and the barrier are off the MFMAs' path.
 #include "common.hpp"
@@ -81,6 +86,8 @@ struct Operand {
     int parts, width;
     int* exps;            // row scale 2^e, or kFlag
     int rb, kb;           // 32-row blocks and 16-c blocks written (padded)
+    float* scales;        // codes kept as one plane: their scales 2^e, [group][32 rb]
+    int gpad;             // groups written there (padded)
 };
 
 __device__ __forceinline__ float code_at(const void* p, int bits, int64_t i) {
@@ -203,11 +210,62 @@ __device__ __forceinline__ void load8(const Src& s, int r, int c, float (&v)[8])
     }
 }
 
+// 8 codes as f16 (exact), zero outside R x C.
+template <int BITS>
+__device__ __forceinline__ f16x8 codes8(const Src& s, int r, int c) {
+    f16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (r >= s.R || c >= s.C) return v;   // C is a multiple of 32
+    const int64_t i = int64_t(r) * s.ld + c;
+    if (!s.vec) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = _Float16(code_at(s.p, BITS, i + j));
+    } else if constexpr (BITS == 8) {
+        const int2 q = *reinterpret_cast<const int2*>(static_cast<const int8_t*>(s.p) + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[j] = _Float16((q.x << (24 - 8 * j)) >> 24);
+            v[4 + j] = _Float16((q.y << (24 - 8 * j)) >> 24);
+        }
+    } else {
+        const int q = *reinterpret_cast<const int*>(static_cast<const uint8_t*>(s.p) + (i >> 1));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = _Float16((q << (28 - 4 * j)) >> 28);
+    }
+    return v;
+}
+
 // 2^e brings a row of largest magnitude `bits` below 2^15 (extra: the codes'
 // bits above the scale); e <= 126 keeps the factor a normal number.
 __device__ __forceinline__ int row_exp(uint32_t bits, int extra) {
     if (bits >= 0x7f800000u) return kFlag;
     return bits == 0 ? 0 : min(126, 14 + 127 - int(bits >> 23) - extra);
+}
+
+__device__ __forceinline__ float exp_factor(int e) {
+    return __uint_as_float(uint32_t((e == kFlag ? 0 : e) + 127) << 23);
+}
+
+template <int BITS>
+__device__ __forceinline__ void codes_part(const Operand& o, int block) {
+    const int chunks = (o.kb + 15) / 16;
+    const int rb = block / chunks, chunk = block % chunks;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = rb * 32 + (lane & 31), h = lane >> 5;
+    f16x8 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = codes8<BITS>(o.s, r, (chunk * 16 + u * 4 + wave) * 16 + 8 * h);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int kb = chunk * 16 + u * 4 + wave;
+        if (kb < o.kb) *reinterpret_cast<f16x8*>(o.planes + (int64_t(rb) * o.kb + kb) * 1024 + lane * 16) = v[u];
+    }
+    if (chunk != 0) return;
+    const int e = row_exp(r < o.s.R ? o.part[r] : 0u, BITS == 8 ? 7 : 3);
+    if (wave == 0 && h == 0) o.exps[r] = e;
+    const float f = exp_factor(e);
+    for (int g = threadIdx.x >> 5; g < o.gpad; g += 8)
+        o.scales[int64_t(g) * (o.rb * 32) + r] =
+            r < o.s.R && g < o.s.groups ? o.s.scale[int64_t(r) * o.s.groups + g] * f : 0.0f;
 }
 
 template <int BITS, int COL>
@@ -222,7 +280,7 @@ __device__ __forceinline__ void split_part(const Operand& o, int block) {
         for (int i = 0; i < o.parts; ++i) m = max(m, o.part[int64_t(i) * o.width + at]);
     const int e = row_exp(m, BITS == 32 ? 0 : (BITS == 8 ? 7 : 3));
     if (chunk == 0 && wave == 0 && h == 0) o.exps[r] = e;
-    const float f = __uint_as_float(uint32_t((e == kFlag ? 0 : e) + 127) << 23);
+    const float f = exp_factor(e);
     float v[4][8];
 #pragma unroll
     for (int u = 0; u < 4; ++u) load8<BITS, COL>(o.s, r, (chunk * 16 + u * 4 + wave) * 16 + 8 * h, v[u]);
@@ -244,7 +302,10 @@ __device__ __forceinline__ void split_part(const Operand& o, int block) {
 }
 
 __device__ __forceinline__ void split_any(const Operand& o, int block) {
-    if (o.s.col) {
+    if (o.scales) {
+        if (o.s.bits == 8) codes_part<8>(o, block);
+        else codes_part<4>(o, block);
+    } else if (o.s.col) {
         if (o.s.bits == 32) split_part<32, 1>(o, block);
         else if (o.s.bits == 8) split_part<8, 1>(o, block);
         else split_part<4, 1>(o, block);
@@ -268,7 +329,9 @@ struct PlaneArgs {
     const float* bias;
     float* out;
     int M, N;             // rows of A, rows of B; out is [M, N]
-    int stages;           // a multiple of 2
+    int stages, chunk;    // parts are whole chunks of stages
+    const float* scales;  // CODE: [group][scale_ld]
+    int scale_ld, gps;    // stages of a group
     int tiles_m, tiles_n;
     int full, per_full;   // tiles computed whole, and how many of them an XCD takes
     int splits, per_part; // the other tiles: c in `splits` parts, and an XCD's share of the parts
@@ -276,19 +339,25 @@ struct PlaneArgs {
     int accumulate;
 };
 
-constexpr int RING = 4;
 constexpr int GROUP_M = 8;   // tile rows of the order inside an XCD
 
-template <int WM_, int WN_, int MT_, int NT_>
+// CODE: B is one plane of codes. A stage is KB blocks of 16 c, in LDS per
+// 32-row block of A its KB h and l fragments, of B its KB fragments (one or
+// two planes), then (CODE) the tile's scales of the stage's group.
+template <int WM_, int WN_, int MT_, int NT_, bool CODE_, int RING_>
 struct Geo {
-    static constexpr int WM = WM_, WN = WN_, MT = MT_, NT = NT_;
+    static constexpr int WM = WM_, WN = WN_, MT = MT_, NT = NT_, RING = RING_;
+    static constexpr bool CODE = CODE_;
     static constexpr int WAVES = WM * WN;
     static constexpr int TM = WM * MT * 32, TN = WN * NT * 32;
-    static constexpr int UNITS = (TM + TN) / 32 * 2;   // 1 KB loads of a stage
+    static constexpr int KB = CODE ? 2 : 1;
+    static constexpr int AU = 2 * KB, BU = 2;   // 1 KB units of a 32-row block (BU: 2 planes, or 2 blocks of c)
+    static constexpr int UNITS = TM / 32 * AU + TN / 32 * BU;
     static constexpr int UPW = UNITS / WAVES;
-    static constexpr int STAGE = UNITS * 1024;
+    static constexpr int LOADS = UPW + (CODE ? 1 : 0);   // loads a wave issues for a stage
+    static constexpr int STAGE = UNITS * 1024 + (CODE ? TN * 4 : 0);
     static constexpr int LDS = RING * STAGE + (TM + TN) * 4;
-    static_assert(UNITS % WAVES == 0, "");
+    static_assert(UNITS % WAVES == 0 && LDS <= 160 * 1024, "");
 };
 
 __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
@@ -356,7 +425,8 @@ __device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r
 
 template <typename T>
 __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) {
-    constexpr int MT = T::MT, NT = T::NT;
+    constexpr int MT = T::MT, NT = T::NT, RING = T::RING;
+    constexpr bool CODE = T::CODE;
     extern __shared__ __align__(16) uint8_t smem[];
     int* exps = reinterpret_cast<int*>(smem + RING * T::STAGE);
     const int t = threadIdx.x;
@@ -377,9 +447,9 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) 
         part = u % a.splits;
         if (L >= a.tiles_m * a.tiles_n) return;
     }
-    const int pairs = a.stages >> 1;
-    const int first = whole ? 0 : 2 * (part * pairs / a.splits);
-    const int end = whole ? a.stages : 2 * ((part + 1) * pairs / a.splits);
+    const int chunks = a.stages / a.chunk;
+    const int first = whole ? 0 : a.chunk * (part * chunks / a.splits);
+    const int end = whole ? a.stages : a.chunk * ((part + 1) * chunks / a.splits);
     int ti, tj;
     tile_at(a, L, ti, tj);
     const int m0 = ti * T::TM, n0 = tj * T::TN;
@@ -387,90 +457,155 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) 
     for (int i = t; i < T::TM + T::TN; i += 64 * T::WAVES)
         exps[i] = i < T::TM ? a.ea[m0 + i] : a.eb[n0 + i - T::TM];
 
-    // This wave's loads of a stage: units wave * UPW ..; unit u is part u % 2
-    // of the tile's 32-row block u / 2 (A's blocks, then B's).
+    // This wave's loads of a stage: units wave * UPW ..; first A's (AU to a
+    // 32-row block), then B's. A stage further is AU or BU KB further.
     const uint8_t* src[T::UPW];
-    const int64_t strip = int64_t(a.stages) * 2048;
+    uint32_t step_bytes[T::UPW];
+    const int64_t strip_a = int64_t(a.stages) * T::AU * 1024, strip_b = int64_t(a.stages) * T::BU * 1024;
 #pragma unroll
     for (int i = 0; i < T::UPW; ++i) {
-        const int u = wave * T::UPW + i, blk = u >> 1;
-        src[i] = (blk < T::TM / 32 ? a.A + (m0 / 32 + blk) * strip : a.B + (n0 / 32 + blk - T::TM / 32) * strip) +
-                 (u & 1) * 1024;
+        const int u = wave * T::UPW + i, v = u - T::TM / 32 * T::AU;
+        const bool isa = v < 0;
+        src[i] = isa ? a.A + (m0 / 32 + u / T::AU) * strip_a + (u % T::AU) * 1024
+                     : a.B + (n0 / 32 + v / T::BU) * strip_b + (v % T::BU) * 1024;
+        step_bytes[i] = (isa ? T::AU : T::BU) * 1024u;
     }
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(smem));
+    const uint32_t scol = uint32_t((n0 + (t & (T::TN - 1))) * 4);   // CODE: this lane's column of the scales
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-    auto issue = [&](int s) {   // past the last stage: the last one again, never read
-        const uint32_t off = uint32_t(min(s, end - 1)) * 2048u + uint32_t(lane) * 16u;
-        const uint32_t lds = lds0 + uint32_t(s & (RING - 1)) * T::STAGE + uint32_t(wave * T::UPW) * 1024u;
+    auto issue = [&](int s, int slot) {   // past the last stage: the last one again, never read
+        const uint32_t at = uint32_t(min(s, end - 1));
+        const uint32_t lds = lds0 + uint32_t(slot) * T::STAGE + uint32_t(wave * T::UPW) * 1024u;
 #pragma unroll
         for (int i = 0; i < T::UPW; ++i)
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + i * 1024), "v"(off),
-                         "s"(src[i])
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + i * 1024),
+                         "v"(at * (T::AU == T::BU ? T::AU * 1024u : step_bytes[i]) + uint32_t(lane) * 16u), "s"(src[i])
+                         : "memory", "m0");
+        if constexpr (CODE)   // waves past the tile's columns load them again
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(
+                             lds0 + uint32_t(slot) * T::STAGE + T::UNITS * 1024u +
+                             uint32_t(wave % (T::TN / 64)) * 256u),
+                         "v"(at / uint32_t(a.gps) * uint32_t(a.scale_ld) * 4u + scol), "s"(a.scales)
                          : "memory", "m0");
     };
 #pragma clang diagnostic pop
 
+    // Fragments of 16 c: A's h and l; B's h and l, or (CODE) its codes.
     struct Frags {
-        u32x4 a[MT][2], b[NT][2];
+        u32x4 a[MT][2], b[NT][CODE ? 1 : 2];
     };
-    auto fetch = [&](int s, Frags& f) {
-        const uint8_t* st = smem + (s & (RING - 1)) * T::STAGE + lane * 16;
+    auto fetch = [&](int slot, int kb, Frags& f) {
+        const uint8_t* st = smem + slot * T::STAGE + lane * 16;
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int p = 0; p < 2; ++p)
-                f.a[i][p] = *reinterpret_cast<const u32x4*>(st + (wm * MT + i) * 2048 + p * 1024);
+                f.a[i][p] = *reinterpret_cast<const u32x4*>(st + ((wm * MT + i) * T::AU + 2 * kb + p) * 1024);
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int p = 0; p < 2; ++p)
-                f.b[j][p] = *reinterpret_cast<const u32x4*>(st + (T::TM / 32 + wn * NT + j) * 2048 + p * 1024);
+            for (int p = 0; p < (CODE ? 1 : 2); ++p)
+                f.b[j][p] = *reinterpret_cast<const u32x4*>(
+                    st + (T::TM / 32 * T::AU + (wn * NT + j) * T::BU + kb + p) * 1024);
     };
-    // The matrix unit rounds once per 8 products. hh is summed apart from
-    // hl + lh, whose roundings are then 2^-11 of those of the sum.
+    // The matrix unit rounds once per 8 products. Two planes: hh is summed
+    // apart from hl + lh, whose roundings are then 2^-11 of those of the sum.
+    // CODE: `low` is the sum of the group, x as h and l against the codes, and
+    // goes to acc times the group's scale.
     f32x16 acc[MT][NT], low[MT][NT];
+    const f32x16 zero = {};
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < NT; ++j) acc[i][j] = low[i][j] = zero;
+    auto multiply = [&](const Frags& f, bool fresh) {
+        if constexpr (CODE) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.0f;
-    auto multiply = [&](const Frags& f) {
+            for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+                for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[i][j] = mfma(f.a[i][0], f.b[j][0], acc[i][j]);
+                    for (int j = 0; j < NT; ++j)
+                        low[i][j] = mfma(f.a[i][p], f.b[j][0], fresh && p == 0 ? zero : low[i][j]);
+        } else {
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+            for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) low[i][j] = mfma(f.a[i][0], f.b[j][1], low[i][j]);
+                for (int j = 0; j < NT; ++j) acc[i][j] = mfma(f.a[i][0], f.b[j][0], acc[i][j]);
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+            for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) low[i][j] = mfma(f.a[i][1], f.b[j][0], low[i][j]);
+                for (int j = 0; j < NT; ++j) low[i][j] = mfma(f.a[i][0], f.b[j][CODE ? 0 : 1], low[i][j]);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) low[i][j] = mfma(f.a[i][1], f.b[j][0], low[i][j]);
+        }
     };
 
     __syncthreads();   // exps; and no plain load is in flight when the counted ones start
-    issue(first);
-    issue(first + 1);
-    issue(first + 2);
+#pragma unroll
+    for (int i = 0; i < RING - 1; ++i) issue(first + i, i);
     Frags f0, f1;
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * T::UPW) : "memory");
-    fetch(first, f0);
-    // Step s: the fragments of stage s are in `cur`. Stage s + 1 has landed
-    // once at most stage s + 2's loads are in flight; past the barrier that
-    // holds for every wave, and the ring slot of stage s - 1 is free (its
-    // fragments were used before the barrier).
-    auto step = [&](int s, const Frags& cur, Frags& nxt) {
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(T::UPW) : "memory");
-        issue(s + 3);
-        fetch(s + 1, nxt);
-        multiply(cur);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((RING - 2) * T::LOADS) : "memory");
+    fetch(0, 0, f0);
+    // Start of step s: its first fragments are in registers. Stage s + 1 has
+    // landed once at most the loads of the stages after it are in flight; past
+    // the barrier that holds for every wave, and the ring slot of stage s - 1
+    // is free (its fragments were used before the barrier).
+    int slot = 0;   // of stage s
+    auto start = [&](int s) {
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((RING - 3) * T::LOADS) : "memory");
+        issue(s + RING - 1, slot == 0 ? RING - 1 : slot - 1);
     };
-    for (int s = first; s < end; s += 2) {
-        step(s, f0, f1);
-        step(s + 1, f1, f0);
+    auto next = [&](int v) { return v == RING - 1 ? 0 : v + 1; };
+    if constexpr (CODE) {
+        float sc[NT];   // of the stage's group
+        auto step = [&](int s, bool fresh) {
+            start(s);
+            fetch(slot, 1, f1);
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                sc[j] = *reinterpret_cast<const float*>(smem + slot * T::STAGE + T::UNITS * 1024 +
+                                                        ((wn * NT + j) * 32 + (lane & 31)) * 4);
+            multiply(f0, fresh);
+            slot = next(slot);
+            fetch(slot, 0, f0);
+            multiply(f1, false);
+        };
+        auto fold = [&] {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] = __builtin_fmaf(sc[j], low[i][j][e], acc[i][j][e]);
+        };
+        if (a.gps == 1) {
+            for (int s = first; s < end; ++s) {
+                step(s, true);
+                fold();
+            }
+        } else {
+            for (int s = first; s < end;) {
+                const int stop = s + a.gps;
+                step(s, true);
+                for (++s; s < stop; ++s) step(s, false);
+                fold();
+            }
+        }
+    } else {
+        auto step = [&](int s, const Frags& cur, Frags& nxt) {
+            start(s);
+            slot = next(slot);
+            fetch(slot, 0, nxt);
+            multiply(cur, false);
+        };
+        for (int s = first; s < end; s += 2) {
+            step(s, f0, f1);
+            step(s + 1, f1, f0);
+        }
     }
     // No direct-to-LDS load may outlive the workgroup's LDS.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -479,7 +614,7 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) 
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            acc[i][j] += low[i][j];
+            if constexpr (!CODE) acc[i][j] += low[i][j];
             if (whole) {
                 const int lr = (wm * MT + i) * 32, lc = (wn * NT + j) * 32;
                 store_tile(a, acc[i][j], m0 + lr, n0 + lc, exps + lr, exps[T::TM + lc + (lane & 31)]);
@@ -541,9 +676,12 @@ int launch_gemm(dgm_gpu* g, const PlaneArgs& a) {
 
 // Tiles of 8 waves (128 x 256, 256 x 128: one workgroup per CU) and of 4
 // (128 x 128: two).
-using Wide = Geo<2, 4, 2, 2>;
-using Tall = Geo<4, 2, 2, 2>;
-using Small = Geo<2, 2, 2, 2>;
+using Wide = Geo<2, 4, 2, 2, false, 4>;
+using Tall = Geo<4, 2, 2, 2, false, 4>;
+using Small = Geo<2, 2, 2, 2, false, 4>;
+using CodeWide = Geo<2, 4, 2, 2, true, 4>;
+using CodeTall = Geo<4, 2, 2, 2, true, 3>;
+using CodeSmall = Geo<2, 2, 2, 2, true, 3>;
 
 struct Tile {
     int tm, tn, slots;   // slots: workgroups a CU holds
@@ -553,14 +691,17 @@ constexpr Tile kTiles[] = {{128, 256, 1}, {256, 128, 1}, {128, 128, 2}};
 int64_t round_up(int64_t v, int64_t to) { return (v + to - 1) / to * to; }
 
 // How a product is cut into tiles and parts, and its time in microseconds.
-// Measured on 256 CUs (one 16-c stage of every busy slot): 128 x 256 tiles
-// 0.36 us with few CUs busy and 0.62 us with all (the clock falls under the
-// matrix load), 128 x 128 tiles 0.26 us alone on a CU and 0.70 us for the two
-// of a CU. A round also fills and drains (4 us). Where the tiles leave the
-// last round partly empty, that round's tiles are cut along c; the sums of
-// the parts cost a launch and their traffic. Whole against cut, same run:
-// 517 x 4100 x 4128 134 -> 93 us, 1024 x 512 x 2048 69 -> 31 us, the dW of
-// 12288 rows at 1536 x 384 with its dX and forward 531 -> 286 us.
+// Fitted to runs on 256 CUs, one 16-c block in every busy slot: 128 x 256 tiles
+// of two planes take 0.36 us with few CUs busy and 0.62 us with all (the clock
+// falls under the matrix load), 128 x 128 tiles 0.26 us alone on a CU and 0.70
+// us for the two of a CU; codes two thirds of that, and 0.10 us where the
+// block's stage ends a group. A round also fills and drains (4 us). Where the
+// tiles leave the last round partly empty, that round's tiles are cut along c:
+// the sums of the parts cost a launch and their traffic, mostly in the
+// Infinity Cache. Whole against cut, same run, the better tile of each: int8
+// 517 x 4100 x 4128 104 and 76 us, int4 256 x 4096 x 4096 89 and 48, fp32 512
+// x 4096 x 4096 105 and 94, fp32 1536 x 384 x 12288 226 and 98; whole is better
+// at fp32 2048 x 2048 x 2048 (70 against 81).
 struct Plan {
     int tile;
     int64_t tiles, full;   // all; computed whole (the others in `splits` parts)
@@ -568,42 +709,48 @@ struct Plan {
     double us;
 };
 
-double round_us(int tile, int64_t units, int cus, double stages) {
+// One round of `units` workgroups, each `blocks` of 16 c long. fold: codes, the
+// share of a block that ends a group's stage (0: two planes).
+double round_us(int tile, int64_t units, int cus, double blocks, double fold) {
     const double busy = std::min(1.0, double(units) / cus);
-    if (tile < 2) return 4.0 + (0.36 + 0.26 * busy) * stages;
-    return 4.0 + (units <= cus ? 0.26 + 0.10 * busy : 0.70) * stages;
+    const bool pair = units > cus;   // two 128 x 128 tiles to a CU
+    double block;
+    if (fold > 0.0) block = (tile < 2 ? 0.24 + 0.17 * busy : pair ? 0.47 : 0.24) + 0.10 * fold;
+    else block = tile < 2 ? 0.36 + 0.26 * busy : pair ? 0.70 : 0.26 + 0.10 * busy;
+    return 4.0 + block * blocks;
 }
 
-double rounds_us(int tile, int64_t units, int cus, double stages) {
+double rounds_us(int tile, int64_t units, int cus, double blocks, double fold) {
     const int64_t slots = int64_t(cus) * kTiles[tile].slots;
     const int64_t rest = units % slots;
-    return double(units / slots) * round_us(tile, slots, cus, stages) +
-           (rest ? round_us(tile, rest, cus, stages) : 0.0);
+    return double(units / slots) * round_us(tile, slots, cus, blocks, fold) +
+           (rest ? round_us(tile, rest, cus, blocks, fold) : 0.0);
 }
 
-Plan plan_for(int64_t M, int64_t N, int64_t stages, int cus) {
+Plan plan_for(int64_t M, int64_t N, int64_t blocks, int chunk, double fold, int cus) {
     Plan best{0, 0, 0, 1, 1e30};
     for (int tile = 0; tile < 3; ++tile) {
         const Tile& t = kTiles[tile];
         const int64_t tiles = int64_t(dgm::ceil_div(M, t.tm)) * dgm::ceil_div(N, t.tn);
-        const double us = rounds_us(tile, tiles, cus, double(stages));
+        const double us = rounds_us(tile, tiles, cus, double(blocks), fold);
         if (us < best.us) best = Plan{tile, tiles, tiles, 1, us};
         const int64_t slots = int64_t(cus) * t.slots, full = tiles / slots * slots, cut = tiles - full;
-        for (int s = 2; s <= 8 && cut > 0 && stages / s >= 16; ++s) {
-            const double cut_us = rounds_us(tile, full, cus, double(stages)) +
-                                  rounds_us(tile, cut * s, cus, double(stages) / s) + 4.0 +
-                                  double(cut) * s * t.tm * t.tn * 8.0 / 4e6;
+        for (int s = 2; s <= 8 && cut > 0 && blocks / s >= std::max(16, chunk); ++s) {
+            const double part = double(dgm::ceil_div(blocks / chunk, s)) * chunk;
+            const double cut_us = (full ? rounds_us(tile, full, cus, double(blocks), fold) : 0.0) +
+                                  rounds_us(tile, cut * s, cus, part, fold) + 4.0 +
+                                  double(cut) * s * t.tm * t.tn * 8.0 / 8e6;
             if (cut_us < best.us) best = Plan{tile, tiles, full, s, cut_us};
         }
     }
     return best;
 }
 
-Operand operand(const Src& s, int tile, int64_t stages) {
+Operand operand(const Src& s, int tile, int64_t blocks) {
     Operand o{};
     o.s = s;
     o.rb = int(round_up(s.R, tile) / 32);
-    o.kb = int(stages);
+    o.kb = int(blocks);
     o.parts = s.col ? int(std::min<int64_t>(kMaxParts, std::max<int64_t>(1, s.C / 64))) : 1;
     o.width = s.col && s.bits != 32 ? s.groups : s.R;
     return o;
@@ -627,7 +774,7 @@ MaxArg max_arg(const Operand& o) {
 
 // Where the pieces of a product lie in the plane buffer.
 struct Layout {
-    size_t planes_a, planes_b, exps_a, exps_b, max_a, max_b, parts, bytes;
+    size_t planes_a, planes_b, exps_a, exps_b, max_a, max_b, scales, parts, bytes;
 };
 
 Layout layout(const Operand& a, const Operand& b, int cut, int splits, const Tile& t) {
@@ -643,20 +790,26 @@ Layout layout(const Operand& a, const Operand& b, int cut, int splits, const Til
     l.exps_b = take(int64_t(b.rb) * 128);
     l.max_a = take(int64_t(a.parts) * a.width * 4);
     l.max_b = take(int64_t(b.parts) * b.width * 4);
+    l.scales = take(int64_t(b.gpad) * b.rb * 128);
     l.parts = take(int64_t(cut) * splits * t.tm * t.tn * 4);
     return l;
 }
 
-int64_t stages_of(int64_t C) { return round_up(dgm::ceil_div(C, 16), 2); }
+// The forward keeps the codes as one plane where a stage of 32 c lies in one
+// group: 2 products instead of 3, and half the bytes of B's planes.
+bool one_plane(const Src& b) { return b.bits != 32 && !b.col && b.G % 32 == 0; }
 
 // out[M, N] (+)= A B^T (+ bias); kNotFused, launching nothing,
 // without a plane buffer.
 int run(dgm_gpu* g, const Src& sa, const Src& sb, const float* bias, float* out, bool accumulate) {
-    const int64_t stages = stages_of(sa.C);
-    const Plan plan = plan_for(sa.R, sb.R, stages, g->num_cus);
+    const bool code = one_plane(sb);
+    const int gps = code ? sb.G / 32 : 1, chunk = code ? gps : 2;
+    const int64_t blocks = code ? sa.C / 16 : round_up(dgm::ceil_div(sa.C, 16), 2);
+    const Plan plan = plan_for(sa.R, sb.R, blocks, code ? chunk * 2 : chunk, code ? 1.0 / gps : 0.0, g->num_cus);
     if (plan.tiles > (1 << 24)) return dgm::kNotFused;   // 32-bit tile numbers
     const Tile& tile = kTiles[plan.tile];
-    Operand a = operand(sa, tile.tm, stages), b = operand(sb, tile.tn, stages);
+    Operand a = operand(sa, tile.tm, blocks), b = operand(sb, tile.tn, blocks);
+    if (code) b.gpad = int(blocks / 2 / gps);
     const int cut = int(plan.tiles - plan.full);
     const Layout at = layout(a, b, cut, plan.splits, tile);
     uint8_t* ws = dgm::planes_buffer(g, at.bytes);
@@ -667,6 +820,7 @@ int run(dgm_gpu* g, const Src& sa, const Src& sb, const float* bias, float* out,
     b.exps = reinterpret_cast<int*>(ws + at.exps_b);
     a.part = reinterpret_cast<uint32_t*>(ws + at.max_a);
     b.part = reinterpret_cast<uint32_t*>(ws + at.max_b);
+    if (code) b.scales = reinterpret_cast<float*>(ws + at.scales);
     const MaxArg x = max_arg(a), y = max_arg(b);
     hipLaunchKernelGGL(row_max_kernel, dim3(unsigned(x.blocks + y.blocks)), dim3(256), 0, g->stream, x, y);
     const int ba = a.rb * int(dgm::ceil_div(a.kb, 16)), bb = b.rb * int(dgm::ceil_div(b.kb, 16));
@@ -682,7 +836,11 @@ int run(dgm_gpu* g, const Src& sa, const Src& sb, const float* bias, float* out,
     p.out = out;
     p.M = sa.R;
     p.N = sb.R;
-    p.stages = int(stages);
+    p.stages = int(code ? blocks / 2 : blocks);
+    p.chunk = chunk;
+    p.scales = b.scales;
+    p.scale_ld = b.rb * 32;
+    p.gps = gps;
     p.tiles_m = a.rb * 32 / tile.tm;
     p.tiles_n = b.rb * 32 / tile.tn;
     p.full = int(plan.full);
@@ -691,6 +849,11 @@ int run(dgm_gpu* g, const Src& sa, const Src& sb, const float* bias, float* out,
     p.per_part = (cut * plan.splits + 7) / 8;
     p.part = reinterpret_cast<float*>(ws + at.parts);
     p.accumulate = accumulate;
+    if (code) {
+        if (plan.tile == 0) return launch_gemm<CodeWide>(g, p);
+        if (plan.tile == 1) return launch_gemm<CodeTall>(g, p);
+        return launch_gemm<CodeSmall>(g, p);
+    }
     if (plan.tile == 0) return launch_gemm<Wide>(g, p);
     if (plan.tile == 1) return launch_gemm<Tall>(g, p);
     return launch_gemm<Small>(g, p);

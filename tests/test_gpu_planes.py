@@ -56,6 +56,8 @@ SHAPES = [   # bits, M, N, K, G
     (4, 128, 14336, 1026, 18),      # odd row bytes for int4
     (8, 517, 640, 4128, 32),        # few tiles: cut along the contraction
     (4, 2048, 4352, 256, 128),      # whole tiles and a cut last round
+    (8, 1000, 1029, 960, 96),       # groups of three stages, an odd number of tiles cut
+    (4, 300, 3000, 1056, 32),       # an odd number of stages
 ]
 
 
@@ -85,6 +87,34 @@ def test_products(gpu, bits, M, N, K, G):
     gpu.gemmBwd(bits, w, q, s, dy, x, dx2, dw2, M, N, K, G)
     gpu.end()
     assert torch.equal(dx, dx2) and torch.equal(dw, dw2)
+
+
+@pytest.mark.parametrize("bits,M,N,K,G", [(4, 1024, 1024, 1024, 32), (8, 1000, 1024, 1024, 64), (8, 1024, 1024, 1024, 8),
+                                          (32, 1024, 1024, 1024, 8)])
+def test_unaligned_buffers(gpu, bits, M, N, K, G):
+    """Operands that start 4 bytes past a 16-byte boundary: the split reads
+    them element by element, with the same products."""
+    import torch
+    x, dy, w, q, s, _, _ = _inputs(gpu, bits, M, N, K, G, 3)
+
+    def off(t):
+        if t is None:
+            return None
+        n = 4 // t.element_size()
+        raw = torch.zeros(t.numel() + n, dtype=t.dtype, device="cuda")
+        raw[n:] = t.reshape(-1)
+        return raw[n:]
+    outs = []
+    for a in ((x, dy, w, q, s), tuple(off(t) for t in (x, dy, w, q, s))):
+        y, dx, dw = (torch.full(sh, float("nan"), device="cuda") for sh in ((M, N), (M, K), (N, K)))
+        torch.cuda.synchronize()
+        gpu.begin()
+        gpu.gemmNT(bits, a[2], a[3], a[4], a[0], None, y, M, N, K, G)
+        gpu.gemmBwd(bits, a[2], a[3], a[4], a[1], a[0], dx, dw, M, N, K, G)
+        gpu.end()
+        outs.append((y, dx, dw))
+    for a, b in zip(*outs):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
 @pytest.mark.parametrize("kind", ["nonfinite", "rows", "tiny", "zeros"])
