@@ -53,7 +53,7 @@ struct dgm_gpu {
     size_t planes_bytes = 0;
     void* planes_retired[kMaxRetired] = {};
     int n_planes_retired = 0;
-    bool planes_fixed = false;             // dgm_gpu_reserve was called: it grows no more by itself
+    bool reserved = false;                 // dgm_gpu_reserve was called: staging that a call can do without grows no more
     hipStream_t planes_stream = nullptr;   // of the last use
     hipEvent_t planes_event = nullptr;
 };
@@ -75,6 +75,10 @@ int check_launch(dgm_gpu* g, const char* name);
 // failure (error recorded): allocation failure, or growth needed while the
 // context's stream is capturing a graph.
 void* workspace(dgm_gpu* g, size_t bytes);
+// The same for staging that only makes a call faster: nullptr, with nothing
+// recorded, where the workspace would have to grow under graph capture, after
+// dgm_gpu_reserve, or beyond the static scratch.
+void* workspace_if(dgm_gpu* g, size_t bytes);
 // The status a caller returns when workspace() gave nullptr.
 int ws_error(dgm_gpu* g);
 // The buffer of the large GEMMs' operand planes, at least `bytes`, ordered
@@ -220,6 +224,9 @@ int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const fl
 int planes_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, float* dX,
               const dgm_GemmP* p);
 int planes_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p, bool accumulate);
+
+// Y[m, n] = part[0][m][n] + part[1][m][n] + ... + bias[n] (gemm_slab.hip).
+void slab_sum(dgm_gpu* g, const float* part, const float* bias, float* Y, int slices, int M, int N);
 
 inline bool aligned(const void* p, size_t a) {
     return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;

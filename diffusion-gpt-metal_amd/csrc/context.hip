@@ -114,6 +114,27 @@ void* workspace(dgm_gpu* g, size_t bytes) {
     return g->ws;
 }
 
+void* workspace_if(dgm_gpu* g, size_t bytes) {
+    if (g->use_scratch) return g->scratch && bytes <= kScratchBytes ? g->scratch : nullptr;
+    if (bytes <= g->ws_bytes) return g->ws;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (g->reserved || g->n_retired == dgm_gpu::kMaxRetired || hipStreamIsCapturing(g->stream, &cs) != hipSuccess ||
+        cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const int err = g->first_err;
+    void* p = workspace(g, bytes);
+    if (!p) {   // no memory: leave no error behind
+        (void)hipGetLastError();
+        if (err == DGM_OK) {
+            g->first_err = DGM_OK;
+            g->err_msg[0] = 0;
+        }
+    }
+    return p;
+}
+
 uint8_t* planes_buffer(dgm_gpu* g, size_t bytes) {
     if (g->use_scratch) return nullptr;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -122,7 +143,7 @@ uint8_t* planes_buffer(dgm_gpu* g, size_t bytes) {
         return nullptr;
     }
     if (bytes > g->planes_bytes) {
-        if (g->planes_fixed || g->n_planes_retired == dgm_gpu::kMaxRetired) return nullptr;
+        if (g->reserved || g->n_planes_retired == dgm_gpu::kMaxRetired) return nullptr;
         void* p = nullptr;
         const size_t want = std::max(bytes, std::min(2 * g->planes_bytes, bytes + (size_t(256) << 20)));
         if (hipMalloc(&p, want) != hipSuccess) {

@@ -63,6 +63,7 @@
 #include "common.hpp"
 #include "decode_codes.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -214,6 +215,8 @@ struct DecArgs {
     int M, N, K, groups, gshift, rowb, nchunk, has_bias;
     int mtp;     // row tiles of the prepared pieces and exponents
     int mt0;     // first row tile this launch handles (its MT tiles)
+    int slices;  // K cut over gridDim.y workgroups, their sums to part[slice][M][N] (decode_kernel)
+    float* part;
     int spin;    // rounds of every bounded hand-over wait (decode_small_kernel)
 };
 
@@ -266,12 +269,18 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, c = lane & 15;
     const int n0 = blockIdx.x * DEC_COLS;
-    const int T = (a.nchunk + 3) / 4;
+    // This workgroup's slice of K: chunks ch0 .. ch0 + nch - 1, whole intervals
+    // of four (the last slice ends with K).
+    const int Tk = (a.nchunk + 3) / 4;
+    const int ch0 = 4 * int(blockIdx.y * unsigned(Tk) / unsigned(a.slices));
+    const int nch = min(a.nchunk, 4 * int((blockIdx.y + 1) * unsigned(Tk) / unsigned(a.slices))) - ch0;
+    const int T = (nch + 3) / 4;
+    const int g0 = (2 * ch0) >> a.gshift;   // first group of the slice
     // Interval t of this workgroup holds chunks 4 ((t + rot) % T) + 0..3:
     // workgroups start at different K offsets, so the weight rows they read
     // at the same moment are spread over K rather than all at one offset
     // (whole intervals only).
-    const int rot = a.nchunk % 4 == 0 ? int(blockIdx.x % unsigned(T)) : 0;
+    const int rot = nch % 4 == 0 ? int(blockIdx.x % unsigned(T)) : 0;
     auto iv = [&](int t) { return (t + rot) % T; };
 
     if (w == DEC_KW * MW) {
@@ -291,7 +300,7 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
         auto dma_interval = [&](int t) {
 #pragma unroll
             for (int cw = 0; cw < 4; ++cw) {
-                const int chunk = min(4 * iv(t < T ? t : T - 1) + cw, a.nchunk - 1);
+                const int chunk = ch0 + min(4 * iv(t < T ? t : T - 1) + cw, nch - 1);
                 const uint32_t lds = lds0 + uint32_t((t % DEC_SLOTS) * 4 + cw) * DEC_CHUNK;
                 // M0 carries the LDS destination of a direct-to-LDS load. The
                 // compiler reserves M0 but uses it in this kernel for nothing
@@ -314,9 +323,10 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
             const uint32_t srow = uint32_t(min(n0 + lane, a.N - 1)) * uint32_t(a.groups) * 4u;
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-            for (int g = 0; g < a.groups; ++g)
+            const int ng = ((2 * (ch0 + nch) - 1) >> a.gshift) - g0 + 1;
+            for (int g = 0; g < ng; ++g)
                 asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds0 + DEC_LDS + g * 256),
-                             "v"(srow + 4u * uint32_t(g)), "s"(a.S)
+                             "v"(srow + 4u * uint32_t(g0 + g)), "s"(a.S)
                              : "memory", "m0");
 #pragma clang diagnostic pop
         }
@@ -347,14 +357,14 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
     // tile0 .. tile0 + MT - 1 of the prepared pieces.
     const int kw = w % DEC_KW, mh = w / DEC_KW;
     const int tile0 = a.mt0 + mh * MT;
-    const int cnt = a.nchunk > kw ? (a.nchunk - kw + 3) / 4 : 0;
+    const int cnt = nch > kw ? (nch - kw + 3) / 4 : 0;
     const int nsteps = cnt * SH::SPC;
 
     XF xa[XR][MT][P];
     const uint32_t xlane = uint32_t(lane) * 16u;
     auto load_x = [&](int s, int slot) {   // this wave's step s (clamped)
         const int ss = s < nsteps ? s : nsteps - 1;
-        const int gstep = (kw + 4 * iv(ss / SH::SPC)) * SH::SPC + ss % SH::SPC;
+        const int gstep = (ch0 + kw + 4 * iv(ss / SH::SPC)) * SH::SPC + ss % SH::SPC;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -373,7 +383,7 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
     f32x4 bc[2][BF ? MT : 1];
     auto load_blk = [&](int b, int slot) {   // this wave's block b (clamped)
         const int bb = b < 2 * cnt ? b : 2 * cnt - 1;
-        const int gblk = 2 * (kw + 4 * iv(bb >> 1)) + (bb & 1);
+        const int gblk = 2 * (ch0 + kw + 4 * iv(bb >> 1)) + (bb & 1);
         if constexpr (!SL) {
             const uint32_t g = uint32_t(gblk) >> a.gshift;
 #pragma unroll
@@ -448,7 +458,7 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
                     wc[ct] = *reinterpret_cast<const u32x4*>(cs + r * 128 + sl * 16);
                 }
                 if constexpr (SL) {
-                    const int g = (2 * (kw + 4 * iv(j)) + hb) >> a.gshift;
+                    const int g = ((2 * (ch0 + kw + 4 * iv(j)) + hb) >> a.gshift) - g0;
                     const float* sc = reinterpret_cast<const float*>(smem + DEC_LDS) + g * 64 + c;
 #pragma unroll
                     for (int ct = 0; ct < 4; ++ct) bs[hb][ct] = sc[16 * ct];
@@ -559,17 +569,20 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
     // memory operations, earlier stores included, before each store.
     const int col = threadIdx.x & 63, n = n0 + col;
     if (n >= a.N || w >= DEC_KW * MW) return;   // the stream wave stores nothing
-    float bv = a.has_bias ? a.bias[n] : 0.0f;
+    const bool cut = a.slices > 1;
+    float* out = cut ? a.part + size_t(blockIdx.y) * a.M * a.N : a.Y;
+    const bool bias = a.has_bias && !cut;
+    float bv = bias ? a.bias[n] : 0.0f;
     asm volatile("" : "+v"(bv));
     for (int m4 = w; m4 < (rows + 3) / 4; m4 += DEC_KW * MW) {
         f32x4 y = *reinterpret_cast<const f32x4*>(red + (0 * 64 + col) * RP + 4 * m4);
 #pragma unroll
         for (int v = 1; v < 4; ++v) y += *reinterpret_cast<const f32x4*>(red + (v * 64 + col) * RP + 4 * m4);
-        if (a.has_bias) y += bv;
+        if (bias) y += bv;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = 4 * m4 + r;
-            if (m < rows) a.Y[size_t(16 * a.mt0 + m) * a.N + n] = y[r];
+            if (m < rows) out[size_t(16 * a.mt0 + m) * a.N + n] = y[r];
         }
     }
 }
@@ -960,8 +973,9 @@ int launch_decode_sl(dgm_gpu* g, const DecArgs& a) {
                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess)
         return dgm::fail(g, DGM_ERR_HIP, "decode: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
-    hipLaunchKernelGGL(kern, dim3(unsigned((a.N + DEC_COLS - 1) / DEC_COLS)), dim3(64 * (DEC_KW * MW + 1)), lds,
-                       g->stream, a);
+    hipLaunchKernelGGL(kern, dim3(unsigned((a.N + DEC_COLS - 1) / DEC_COLS), unsigned(a.slices)),
+                       dim3(64 * (DEC_KW * MW + 1)), lds, g->stream, a);
+    if (a.slices > 1) dgm::slab_sum(g, a.part, a.has_bias ? a.bias : nullptr, a.Y, a.slices, a.M, a.N);
     return DGM_OK;
 }
 
@@ -997,7 +1011,23 @@ int decode_dispatch(dgm_gpu* g, DecArgs& a, const float* X) {
     const size_t xp_bytes = size_t(nblk) * SH::SPB * MT * P * 1024;
     // Exponents (int8) or, on the bf16 path, offset terms (fp32) per (block, row).
     const size_t ex_bytes = size_t(nblk) * 16 * MT * ((BITS == 4 && P == 1) ? 4 : 1);
-    uint8_t* ws = static_cast<uint8_t*>(dgm::workspace(g, xp_bytes + ex_bytes + 256));
+    // Few workgroups of 64 columns leave CUs idle: cut K over workgroups,
+    // three intervals or more each, while one per CU has room (the sums of the
+    // slices are a second launch). 64 workgroups, whole and cut in four: 24 x
+    // 4096 x 14336 int8 55.0 -> 26.8 us, int4 43.0 -> 23.3, 64 rows 64.9 -> 31.6;
+    // 16 workgroups, 20 x 1024 x 4096 int8 in two 19.5 -> 15.0. Where no
+    // workspace is to be had for the sums, K stays whole.
+    const int64_t wgs = dgm::ceil_div(a.N, DEC_COLS), intervals = (a.nchunk + 3) / 4;
+    a.slices = int(std::max<int64_t>(1, std::min<int64_t>(g->num_cus / wgs, intervals / 3)));
+    const size_t own = (xp_bytes + ex_bytes + 511) & ~size_t(255);
+    uint8_t* ws = nullptr;
+    if (a.slices > 1)
+        ws = static_cast<uint8_t*>(dgm::workspace_if(g, own + size_t(a.slices) * size_t(a.M) * size_t(a.N) * 4));
+    if (ws) a.part = reinterpret_cast<float*>(ws + own);
+    else {
+        a.slices = 1;
+        ws = static_cast<uint8_t*>(dgm::workspace(g, xp_bytes + ex_bytes + 256));
+    }
     if (!ws) return dgm::ws_error(g);
     _Float16* xp = reinterpret_cast<_Float16*>(ws);
     int8_t* ex = reinterpret_cast<int8_t*>(ws + xp_bytes);

@@ -159,9 +159,9 @@ int dgm_gpu_reserve(dgm_gpu* g, int64_t bytes) {
     if (size_t(bytes) > g->ws_bytes && !dgm::workspace(g, size_t(bytes))) return dgm::ws_error(g);
     // The plane buffer too, which from now on grows here only: a call that
     // finds it too small runs without it.
-    g->planes_fixed = false;
+    g->reserved = false;
     if (size_t(bytes) > g->planes_bytes) (void)dgm::planes_buffer(g, size_t(bytes));
-    g->planes_fixed = true;
+    g->reserved = true;
     return DGM_OK;
 }
 

@@ -344,6 +344,16 @@ int64_t slab_slices(int bits, int64_t K) { return (bits == 4 ? K / 2 : K) / (SB_
 
 namespace dgm {
 
+void slab_sum(dgm_gpu* g, const float* part, const float* bias, float* Y, int slices, int M, int N) {
+    const int64_t total = int64_t(M) * N;
+    if (N % 4 == 0 && aligned(Y, 16))
+        hipLaunchKernelGGL(slab_sum_kernel<4>, dim3(unsigned((total / 4 + 255) / 256)), dim3(256), 0, g->stream, part,
+                           bias, Y, slices, M, N);
+    else
+        hipLaunchKernelGGL(slab_sum_kernel<1>, dim3(unsigned((total + 255) / 256)), dim3(256), 0, g->stream, part, bias,
+                           Y, slices, M, N);
+}
+
 // The K-sliced kernel's domain: quantized weights, M <= 16 in the fp32 mode
 // and M <= 8 in the reduced mode (measured crossovers), whole slices of
 // two 128-byte chunks per row (int4: K % 512 == 0; int8: K % 256 == 0),
@@ -392,14 +402,7 @@ int slab_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const floa
     if (bits == 4) rc = exact ? launch_slab_rt<4, 4>(g, a, slices) : launch_slab_rt<4, 2>(g, a, slices);
     else rc = exact ? launch_slab_rt<8, 4>(g, a, slices) : launch_slab_rt<8, 2>(g, a, slices);
     if (rc) return rc;
-    const int64_t total = int64_t(a.M) * a.N;
-    const float* b = p->hasBias ? bias : nullptr;
-    if (a.N % 4 == 0 && aligned(Y, 16))
-        hipLaunchKernelGGL(slab_sum_kernel<4>, dim3(unsigned((total / 4 + 255) / 256)), dim3(256), 0, g->stream, part,
-                           b, Y, slices, a.M, a.N);
-    else
-        hipLaunchKernelGGL(slab_sum_kernel<1>, dim3(unsigned((total + 255) / 256)), dim3(256), 0, g->stream, part, b,
-                           Y, slices, a.M, a.N);
+    slab_sum(g, part, p->hasBias ? bias : nullptr, Y, slices, a.M, a.N);
     return DGM_OK;
 }
 

@@ -158,9 +158,10 @@ int dgm_gemmNT(dgm_gpu* g, int64_t bits, const float* w, const void* q,
 /* No counterpart in the reference: dgm_gemmNT for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). Same arguments, kernels and results
- * (bitwise; where dgm_gemmNT takes the f16 pieces of large products, this
- * entry takes the kernels that stage nothing, with the same error bound) as
- * dgm_gemmNT, but every staging buffer (the decode kernels'
+ * (bitwise; where dgm_gemmNT takes the f16 pieces of large products, or cuts
+ * a long K at 17 to 64 rows into slices whose sums do not fit the scratch,
+ * this entry takes the kernels without that staging, with the same error
+ * bound) as dgm_gemmNT, but every staging buffer (the decode kernels'
  * activation pieces, the bf16 copy of X of the reduced-precision prefill
  * path) comes from a static device scratch of DGM_NOALLOC_SCRATCH_BYTES per
  * GPU, held from library load until the process ends; nothing is allocated.
@@ -189,10 +190,12 @@ int dgm_gemmNT_noalloc(dgm_gpu* g, int64_t bits, const float* w, const void* q,
  * dgm_gemmNT call of that shape can take, in either math mode (-1 for
  * negative sizes); dgm_gpu_reserve grows both buffers to at least `bytes`
  * now (DGM_ERR_UNSUPPORTED during a graph capture), so that later calls whose
- * bound it covers allocate nothing (the bound leaves the f16 pieces out: after
- * a reserve, large products whose pieces do not fit the reserved bytes take
- * the kernels that stage nothing; they need 4 bytes for each element of both
- * operands, rows padded to 256, and some tens of MB of partial sums);
+ * bound it covers allocate nothing (the bound leaves out what a call can do
+ * without: after a reserve, large products whose f16 pieces do not fit the
+ * reserved bytes take the kernels that stage nothing, and calls of 17 to 64
+ * rows whose slice sums do not fit keep K whole; the pieces need 4 bytes for
+ * each element of both operands, rows padded to 256, and some tens of MB of
+ * partial sums, the slices 4 M N bytes each, 256 / ceil(N / 64) of them at most);
  * dgm_gpu_workspace_bytes returns the size of both (0 before anything was
  * allocated). */
 int64_t dgm_gemmNT_workspace_bound(int64_t M, int64_t N, int64_t K);
