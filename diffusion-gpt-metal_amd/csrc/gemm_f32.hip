@@ -475,8 +475,10 @@ void launch_deep(const GemmArgs& a, int num_cus, hipStream_t st) {
 // scale, instead of four 16-row gathers. X in LDS is stored with the 16-byte
 // slot index XOR-ed by (row & 15): the 16 rows read by one MFMA operand fetch
 // land in 16 distinct slots, free of bank conflicts. Contraction parts are
-// reduced through LDS in a fixed order.
-template <int BITS, int KS>
+// reduced through LDS in a fixed order. SG: scales of a lane's 16 indices
+// (groups of 8 have two; 1024 x 512 x 128 int8 in groups of 8 10.2 us with the
+// deep kernel, 5.0 here).
+template <int BITS, int KS, int SG = 1>
 __global__ __launch_bounds__(kThreads) void gemm_fwd_lds_kernel(GemmArgs a, int tiles_i, int tiles_j, int per_xcd) {
     constexpr int NS = 4 / KS;
     constexpr int TN = 16 * NS;
@@ -498,7 +500,7 @@ __global__ __launch_bounds__(kThreads) void gemm_fwd_lds_kernel(GemmArgs a, int 
     const int n = min(j0 + wn * 16 + r16, a.cols - 1);
     uint32_t wc[MAXST][BITS == 4 ? 2 : 4];
     float4 wf[MAXST][BITS == 32 ? 4 : 1];
-    float sc[MAXST];
+    float sc[MAXST][SG];
 #pragma unroll
     for (int u = 0; u < MAXST; ++u) {
         const int st = wk + u * KS;
@@ -511,11 +513,13 @@ __global__ __launch_bounds__(kThreads) void gemm_fwd_lds_kernel(GemmArgs a, int 
         } else if constexpr (BITS == 8) {
             const uint4 v = *reinterpret_cast<const uint4*>(static_cast<const int8_t*>(a.B) + size_t(n) * K + k);
             wc[u][0] = v.x; wc[u][1] = v.y; wc[u][2] = v.z; wc[u][3] = v.w;
-            sc[u] = a.scale[size_t(n) * a.groups + k / a.G];
+            #pragma unroll
+            for (int e = 0; e < SG; ++e) sc[u][e] = a.scale[size_t(n) * a.groups + (k + 8 * e) / a.G];
         } else {
             const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const uint8_t*>(a.B) + ((size_t(n) * K + k) >> 1));
             wc[u][0] = v.x; wc[u][1] = v.y;
-            sc[u] = a.scale[size_t(n) * a.groups + k / a.G];
+            #pragma unroll
+            for (int e = 0; e < SG; ++e) sc[u][e] = a.scale[size_t(n) * a.groups + (k + 8 * e) / a.G];
         }
     }
 
@@ -550,11 +554,11 @@ __global__ __launch_bounds__(kThreads) void gemm_fwd_lds_kernel(GemmArgs a, int 
             } else if constexpr (BITS == 8) {
                 const uint32_t w = wc[u][c];
 #pragma unroll
-                for (int s2 = 0; s2 < 4; ++s2) bv[s2] = float(int(int8_t((w >> (8 * s2)) & 0xFF))) * sc[u];
+                for (int s2 = 0; s2 < 4; ++s2) bv[s2] = float(int(int8_t((w >> (8 * s2)) & 0xFF))) * sc[u][SG == 2 ? c >> 1 : 0];
             } else {
                 const uint32_t w = wc[u][c >> 1] >> (16 * (c & 1));
 #pragma unroll
-                for (int s2 = 0; s2 < 4; ++s2) bv[s2] = float(int(__builtin_amdgcn_sbfe(int(w), 4 * s2, 4))) * sc[u];
+                for (int s2 = 0; s2 < 4; ++s2) bv[s2] = float(int(__builtin_amdgcn_sbfe(int(w), 4 * s2, 4))) * sc[u][SG == 2 ? c >> 1 : 0];
             }
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv.x, bv[0], acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv.y, bv[1], acc, 0, 0, 0);
@@ -600,14 +604,14 @@ __global__ __launch_bounds__(kThreads) void gemm_fwd_lds_kernel(GemmArgs a, int 
     }
 }
 
-template <int BITS, int KS>
+template <int BITS, int KS, int SG = 1>
 void launch_fwd_lds_ks(const GemmArgs& a, hipStream_t st) {
     constexpr int TN = 16 * (4 / KS);
     const int ti = int(dgm::ceil_div(a.rows, 16)), tj = int(dgm::ceil_div(a.cols, TN));
     const int64_t nt = int64_t(ti) * tj;
     const int per = int((nt + 7) / 8);
     const size_t lds = size_t(16) * a.K * sizeof(float);
-    hipLaunchKernelGGL((gemm_fwd_lds_kernel<BITS, KS>), dim3(unsigned(per) * 8u), dim3(kThreads), lds, st, a, ti, tj,
+    hipLaunchKernelGGL((gemm_fwd_lds_kernel<BITS, KS, SG>), dim3(unsigned(per) * 8u), dim3(kThreads), lds, st, a, ti, tj,
                        per);
 }
 
@@ -979,7 +983,7 @@ bool fwd_lds_ok(const GemmArgs& a, int bits, const void* X, const void* W) {
     if (a.K % 64 != 0 || a.K == 0 || a.K > 1024 || a.rows == 0 || a.cols == 0) return false;
     if (!dgm::aligned(X, 16)) return false;
     if (bits == 32) return a.K <= 512 && dgm::aligned(W, 16);
-    if (a.G % 16 != 0) return false;
+    if (a.G % 8 != 0) return false;
     return dgm::aligned(W, bits == 8 ? 16 : 8);
 }
 
@@ -989,7 +993,15 @@ void launch_fwd_lds(const GemmArgs& a, int num_cus, hipStream_t st) {
     // the grid at least ~1.5 workgroups per CU.
     const int nst = a.K / 64;
     const int64_t ti = dgm::ceil_div(a.rows, 16);
-    const int64_t w4 = ti * dgm::ceil_div(a.cols, 16), w2 = ti * dgm::ceil_div(a.cols, 32);
+    const int64_t w2 = ti * dgm::ceil_div(a.cols, 32);
+    if constexpr (BITS != 32) {
+        if (a.G % 16 != 0) {   // groups of 8, 24, ...: two scales to a lane's 16 indices
+            if (nst >= 4 && (w2 < int64_t(num_cus) * 3 / 2 || nst >= 8)) launch_fwd_lds_ks<BITS, 4, 2>(a, st);
+            else if (nst >= 2) launch_fwd_lds_ks<BITS, 2, 2>(a, st);
+            else launch_fwd_lds_ks<BITS, 1, 2>(a, st);
+            return;
+        }
+    }
     if (nst >= 4 && (w2 < int64_t(num_cus) * 3 / 2 || nst >= 8)) {
         if (nst % 4 == 0) launch_fwd_reg<BITS>(a, st);
         else launch_fwd_lds_ks<BITS, 4>(a, st);
@@ -998,7 +1010,6 @@ void launch_fwd_lds(const GemmArgs& a, int num_cus, hipStream_t st) {
         launch_fwd_lds_ks<BITS, 2>(a, st);
     else
         launch_fwd_lds_ks<BITS, 1>(a, st);
-    (void)w4;
 }
 
 // ---- LDS-staged STE dX for short contractions (N <= 448, N % 64 == 0) ---------

@@ -340,3 +340,23 @@ def test_gemm_bwd_is_the_pair(gpu, orc, bits, M, N, K, G, acc):
     assert rel_err(from_dev(dx1), ref_dx.ravel()) <= TOL
     got_dw = from_dev(dw1).astype(np.float64) - (dw0 if acc else 0.0)
     assert rel_err(got_dw, ref_dw.ravel()) <= (1e-4 if acc else TOL)
+
+
+# Forwards whose groups are a multiple of 8 and not of 16 on the LDS-staged
+# kernel: its three contraction splits, ragged rows and columns.
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("M,N,K,G", [(1024, 512, 128, 8), (70, 33, 64, 8), (1000, 1000, 512, 8), (300, 130, 192, 24),
+                                     (513, 70, 960, 40)])
+def test_forward_groups_of_eight(gpu, orc, bits, M, N, K, G):
+    import torch
+    rng = np.random.default_rng(M + K)
+    x, w, b = rng.standard_normal(M * K), rng.standard_normal(N * K) * 0.02, rng.standard_normal(N)
+    x, w, b = (a.astype(np.float32) for a in (x, w, b))
+    q = torch.zeros(N * K // (2 if bits == 4 else 1), dtype=torch.uint8 if bits == 4 else torch.int8, device="cuda")
+    s, y = torch.zeros(N * (K // G), device="cuda"), torch.full((M * N,), float("nan"), device="cuda")
+    gpu.begin()
+    gpu.quantize(to_dev(w), q, s, N, K, bits, G)
+    gpu.gemmNT(bits, None, q, s, to_dev(x), to_dev(b), y, M, N, K, G)
+    gpu.end()
+    wd = orc.dequant(from_dev(q), from_dev(s), N, K, G, bits).reshape(N, K).astype(np.float64)
+    assert rel_err(from_dev(y).reshape(M, N), x.reshape(M, K).astype(np.float64) @ wd.T + b) <= 1e-5

@@ -380,3 +380,17 @@ def test_optimizer_step_matches_reference_order(gpu, dgm, orc, bits):
 
 def math_sqrt_sum(init):
     return float(np.sqrt(sum(float(np.sum(g.astype(np.float64) ** 2)) for _, g in init)))
+
+
+# Column sums through LDS (128 rows and more): edges of its 256-row tiles, the
+# two tiles' hand-over, a last column block of 4 columns.
+@pytest.mark.parametrize("M,N", [(128, 4), (255, 20), (256, 16), (257, 36), (769, 1000), (1500, 16384)])
+def test_bias_grad_tiles_bitexact(gpu, orc, M, N):
+    import torch
+    rng = np.random.default_rng(M * N)
+    dy = rng.standard_normal(M * N).astype(np.float32)
+    out = torch.full((N + 4,), 3.0, dtype=torch.float32, device="cuda")
+    gpu.begin()
+    gpu.biasGrad(to_dev(dy), out, M, N)
+    gpu.end()
+    assert _same(from_dev(out)[:N], orc.bias_grad(dy, M, N)) and bool((out[N:] == 3.0).all())
