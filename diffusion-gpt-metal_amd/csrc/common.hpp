@@ -219,11 +219,13 @@ int gemm_bwd_fold(dgm_gpu* g, const int8_t* codesT, const float* scalesT, const 
 // forward, dX and dW in the fp32 mode, where planes_pay says that they are
 // the faster way. Each product returns kNotFused, launching nothing, when planes_buffer has none.
 bool planes_pay(int64_t M, int64_t N, int64_t K);
+// Y2 (may be null): the upper half of the columns, Y and Y2 [M, N / 2]
+// (N % 64 == 0). X (dY) null: launches nothing, DGM_OK where the call would not
+// return kNotFused. dX or dW may be null: the other alone.
 int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias,
-               float* Y, const dgm_GemmP* p);
-int planes_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, float* dX,
-              const dgm_GemmP* p);
-int planes_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p, bool accumulate);
+               float* Y, const dgm_GemmP* p, float* Y2 = nullptr);
+int planes_bwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, const float* X, float* dX,
+               float* dW, const dgm_GemmP* p, bool accumulate);
 
 // Y[m, n] = part[0][m][n] + part[1][m][n] + ... + bias[n] (gemm_slab.hip).
 void slab_sum(dgm_gpu* g, const float* part, const float* bias, float* Y, int slices, int M, int N);

@@ -1452,11 +1452,20 @@ int dgm_dit_backward(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w,
         }
         DGM_TRY(dgm::wt_prep(g, bits, 4, Wp, Sp, Nn, Kk, G, ctp, stp));
     }
+    // Linears whose backward is a large product that dgm_gemmBwd runs on split
+    // operands (gemm_planes.hip). 1024 x 4096 x 512 with bf16 dX beside fp32
+    // dW tiles 178 us, 66 so; 1024 x 512 x 2048 81 and 56 with its SwiGLU
+    // backward.
+    auto large = [&](int64_t N, int64_t K) {
+        const dgm_GemmP gp{uint32_t(M), uint32_t(N), uint32_t(K), 0u, uint32_t(bits == 32 ? 0 : G), 0, 0, 0};
+        return dgm::planes_pay(M, N, K) &&
+               dgm::planes_bwd(g, bits, nullptr, nullptr, nullptr, nullptr, t1, t1, &gp, true) == DGM_OK;
+    };
     // gemmBwd of stacked linear li (0 [wq; wk; wv], 1 wo, 2 [wgate; wup],
     // 3 wdown) on the bf16-dX pair when `fold`, else the fp32 pair.
     auto bwdf = [&](int li, const dgm_dit_linear& Lw, const float* dy, const float* in, float* out, float* dW,
                     int64_t N, int64_t K) -> int {
-        if (fold) {
+        if (fold && !large(N, K)) {
             const int r = dgm::gemm_bwd_fold(g, fct[li], fst[li], dy, in, out, dW, int(M), int(N), int(K), G, true,
                                              nullptr, nullptr);
             if (r != dgm::kNotFused) return r;
@@ -1514,13 +1523,14 @@ int dgm_dit_backward(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w,
         const dgm_dw::DwTileArgs dwd{dmlp, A(l, A_SW), gr->wdown, int(M), int(C), int(F), 1};
         if (gu1) {
             // wdown's backward with the SwiGLU backward in its dX epilogue,
-            // else the two launches.
-            const int r = fold ? dgm::gemm_bwd_fold(g, fct[3], fst[3], dmlp, A(l, A_SW), S[B_DG],
-                                                    hwd ? nullptr : gr->wdown, int(M), int(C), int(F), G, true,
-                                                    A(l, A_GATE), A(l, A_UP))
-                               : dgm::gemm_bwd_swiglu(g, bits, w->wdown.w, w->wdown.q, w->wdown.scale, dmlp,
-                                                      A(l, A_SW), A(l, A_GATE), A(l, A_UP), S[B_DG], gr->wdown, M, C,
-                                                      F, bits == 32 ? 8 : G);
+            // else (a large product among them) the two launches.
+            const int r = large(C, F) ? dgm::kNotFused
+                          : fold ? dgm::gemm_bwd_fold(g, fct[3], fst[3], dmlp, A(l, A_SW), S[B_DG],
+                                                      hwd ? nullptr : gr->wdown, int(M), int(C), int(F), G, true,
+                                                      A(l, A_GATE), A(l, A_UP))
+                                 : dgm::gemm_bwd_swiglu(g, bits, w->wdown.w, w->wdown.q, w->wdown.scale, dmlp,
+                                                        A(l, A_SW), A(l, A_GATE), A(l, A_UP), S[B_DG], gr->wdown, M, C,
+                                                        F, bits == 32 ? 8 : G);
             if (r == dgm::kNotFused) {
                 hwd = false;
                 DGM_TRY(bwd(w->wdown, dmlp, A(l, A_SW), S[B_DSW], gr->wdown, C, F));

@@ -1654,7 +1654,7 @@ int gemm_f32_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const 
 int gemm_f32_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY,
                 float* dX, const dgm_GemmP* p) {
     if (planes_pay(p->M, p->N, p->K)) {
-        const int rc = planes_dx(g, bits, W, scale, dY, dX, p);
+        const int rc = planes_bwd(g, bits, W, scale, dY, nullptr, dX, nullptr, p, false);
         if (rc != kNotFused) return rc;
     }
     GemmArgs a{};
@@ -1684,7 +1684,7 @@ int gemm_f32_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const f
 int gemm_f32_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p,
                 bool accumulate) {
     if (planes_pay(p->M, p->N, p->K)) {
-        const int rc = planes_dw(g, dY, X, dW, p, accumulate);
+        const int rc = planes_bwd(g, 32, nullptr, nullptr, dY, X, nullptr, dW, p, accumulate);
         if (rc != kNotFused) return rc;
     }
     GemmArgs a{};
@@ -1710,7 +1710,11 @@ int gemm_f32_bwd_pair(dgm_gpu* g, int bits, const void* W, const float* scale, c
                       float* dX, float* dW, const dgm_GemmP* p, bool accumulate, bool* fused, const float* sg_gate,
                       const float* sg_up) {
     *fused = false;
-    if (!sg_gate && planes_pay(p->M, p->N, p->K)) return DGM_OK;
+    if (!sg_gate && planes_pay(p->M, p->N, p->K)) {
+        const int rc = planes_bwd(g, bits, W, scale, dY, X, dX, dW, p, accumulate);
+        *fused = rc != kNotFused;
+        if (*fused) return rc;
+    }
     GemmArgs ax{};
     ax.A = dY; ax.B = W; ax.scale = scale; ax.out = dX;
     ax.sg_gate = sg_gate; ax.sg_up = sg_up;

@@ -40,6 +40,7 @@
 //
 // Three launches: the rows' largest elements, the split into planes, the
 // GEMM; a fourth adds the parts of tiles that are cut along c (struct Plan).
+// dX and dW of one linear share them (struct Pair).
 //
 // Plane layout: 32 rows x 16 c of a plane are one fragment of the MFMA, 1 KB
 // in lane order (lane l: row l % 32, c = 8 (l / 32) .. + 7), and a 32-row
@@ -88,6 +89,7 @@ struct Operand {
     int rb, kb;           // 32-row blocks and 16-c blocks written (padded)
     float* scales;        // codes kept as one plane: their scales 2^e, [group][32 rb]
     int gpad;             // groups written there (padded)
+    int blocks;           // workgroups of its split
 };
 
 __device__ __forceinline__ float code_at(const void* p, int bits, int64_t i) {
@@ -155,9 +157,21 @@ __device__ __forceinline__ void max_part(const MaxArg& a, int block) {
     if (t < 64 && r < a.R) a.out[int64_t(part) * a.R + r] = max(max(sh[0][t], sh[1][t]), max(sh[2][t], sh[3][t]));
 }
 
-__global__ __launch_bounds__(256) void row_max_kernel(MaxArg a, MaxArg b) {
-    if (int(blockIdx.x) < a.blocks) max_part(a, blockIdx.x);
-    else max_part(b, blockIdx.x - a.blocks);
+// The operands of up to two products.
+struct MaxArgs {
+    MaxArg m[4];
+};
+
+__global__ __launch_bounds__(256) void row_max_kernel(MaxArgs a) {
+    int b = int(blockIdx.x);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (b < a.m[i].blocks) {
+            max_part(a.m[i], b);
+            return;
+        }
+        b -= a.m[i].blocks;
+    }
 }
 
 // ---- launch 2: the split ---------------------------------------------------------------
@@ -316,9 +330,15 @@ __device__ __forceinline__ void split_any(const Operand& o, int block) {
     }
 }
 
-__global__ __launch_bounds__(256) void split_kernel(Operand a, Operand b, int blocks_a) {
-    if (int(blockIdx.x) < blocks_a) split_any(a, blockIdx.x);
-    else split_any(b, blockIdx.x - blocks_a);
+struct Operands {
+    Operand o[4];
+};
+
+__global__ __launch_bounds__(256) void split_kernel(Operands a) {
+    int b = int(blockIdx.x), i = 0;
+    while (i < 3 && b >= a.o[i].blocks) b -= a.o[i++].blocks;
+    const Operand o = i == 0 ? a.o[0] : i == 1 ? a.o[1] : i == 2 ? a.o[2] : a.o[3];
+    split_any(o, b);
 }
 
 // ---- launch 3: the GEMM ----------------------------------------------------------------
@@ -327,8 +347,9 @@ struct PlaneArgs {
     const int *ea, *eb;
     Src sa, sb;           // the original operands, for rows with an infinity or NaN
     const float* bias;
-    float* out;
-    int M, N;             // rows of A, rows of B; out is [M, N]
+    float *out, *out2;    // columns from cols1 on go to out2; rows of ldo floats
+    int ldo, cols1;
+    int M, N;             // rows of A, rows of B
     int stages, chunk;    // parts are whole chunks of stages
     const float* scales;  // CODE: [group][scale_ld]
     int scale_ld, gps;    // stages of a group
@@ -365,6 +386,19 @@ __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
                                                   0);
 }
 
+// Up to two products in one launch: the workgroups of the first, then those
+// of the second, which fill what the first leaves idle.
+struct PlaneGroup {
+    PlaneArgs p[2];
+    int first;   // workgroups of p[0]
+};
+
+// p[second] of the kernel's one argument, read where it is used (a copy of the
+// chosen one would keep 50 more scalar registers than there are).
+__device__ __forceinline__ const PlaneArgs& args_of(bool second) {
+    return ((const PlaneArgs*)__builtin_amdgcn_kernarg_segment_ptr())[second ? 1 : 0];
+}
+
 // Tile L of the order: groups of GROUP_M tile rows, column after column, so
 // that the tiles an XCD runs at once share their strips in its L2.
 __device__ __forceinline__ void tile_at(const PlaneArgs& a, int L, int& ti, int& tj) {
@@ -379,7 +413,8 @@ __device__ __forceinline__ void tile_at(const PlaneArgs& a, int L, int& ti, int&
 // rows 8 (e / 4) + 4 (l / 32) + e % 4. ea: the rows' exponents from r0.
 __device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r0, int c0, const int* ea, int eb) {
     const int lane = threadIdx.x & 63, q = lane >> 5;
-    const int M = a.M, N = a.N, c = c0 + (lane & 31);
+    const int M = a.M, N = a.N, ld = a.ldo, c = c0 + (lane & 31);
+    float* const base = c0 < a.cols1 ? a.out : a.out2 - a.cols1;   // cols1 is a multiple of 32, or N
     const float bv = a.bias ? a.bias[min(c, N - 1)] : 0.0f;
     int er[16];
     bool odd = eb == kFlag;
@@ -393,21 +428,21 @@ __device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[e] += bv;
     }
-    float* o = a.out + int64_t(r0 + 4 * q) * N + c;
+    float* o = base + int64_t(r0 + 4 * q) * ld + c;
     if (r0 + 32 <= M && c0 + 32 <= N && !__any(odd)) {
         if (a.accumulate) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[e] += o[int64_t(8 * (e >> 2) + (e & 3)) * N];
+            for (int e = 0; e < 16; ++e) acc[e] += o[int64_t(8 * (e >> 2) + (e & 3)) * ld];
         }
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[int64_t(8 * (e >> 2) + (e & 3)) * N] = acc[e];
+        for (int e = 0; e < 16; ++e) o[int64_t(8 * (e >> 2) + (e & 3)) * ld] = acc[e];
         return;
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
         const int r = r0 + 8 * (e >> 2) + 4 * q + (e & 3);
         if (r < M && c < N && er[e] != kFlag && eb != kFlag) {
-            float* at = o + int64_t(8 * (e >> 2) + (e & 3)) * N;
+            float* at = o + int64_t(8 * (e >> 2) + (e & 3)) * ld;
             *at = a.accumulate ? *at + acc[e] : acc[e];
         }
     }
@@ -418,13 +453,15 @@ __device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r
         float v = 0.0f;
         for (int k = 0; k < a.sa.C; ++k) v = __builtin_fmaf(elem(a.sa, r, k), elem(a.sb, c, k), v);
         v += bv;
-        float* at = a.out + int64_t(r) * N + c;
+        float* at = base + int64_t(r) * ld + c;
         *at = a.accumulate ? *at + v : v;
     }
 }
 
 template <typename T>
-__global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) {
+__global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g) {
+    const bool second = int(blockIdx.x) >= g.first;
+    const PlaneArgs& a = args_of(second);
     constexpr int MT = T::MT, NT = T::NT, RING = T::RING;
     constexpr bool CODE = T::CODE;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -435,7 +472,7 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) 
 
     // XCD x (workgroups x, x + 8, ...) takes a run of the whole tiles, then a
     // run of the parts.
-    const int b = int(blockIdx.x), nfull = a.per_full * 8;
+    const int b = int(blockIdx.x) - (second ? g.first : 0), nfull = a.per_full * 8;
     const bool whole = b < nfull;
     int L, part = 0;
     if (whole) {
@@ -632,10 +669,12 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneArgs a) 
 
 // The parts of the split tiles, added in order: one wave per 32 x 32 tile.
 template <typename T>
-__global__ __launch_bounds__(256) void part_sum_kernel(PlaneArgs a) {
+__global__ __launch_bounds__(256) void part_sum_kernel(PlaneGroup g) {
     constexpr int SUB = T::MT * T::NT;
+    const bool second = int(blockIdx.x) >= g.first;
+    const PlaneArgs& a = args_of(second);
     const int lane = threadIdx.x & 63;
-    const int u = int(blockIdx.x) * 4 + (threadIdx.x >> 6);   // (tile, wave, subtile)
+    const int u = (int(blockIdx.x) - (second ? g.first : 0)) * 4 + (threadIdx.x >> 6);   // (tile, wave, subtile)
     const int sub = u % SUB, wave = u / SUB % T::WAVES, tile = u / (SUB * T::WAVES);
     int ti, tj;
     tile_at(a, a.full + tile, ti, tj);
@@ -657,7 +696,7 @@ __global__ __launch_bounds__(256) void part_sum_kernel(PlaneArgs a) {
 }
 
 template <typename T>
-int launch_gemm(dgm_gpu* g, const PlaneArgs& a) {
+int launch_gemm(dgm_gpu* g, const PlaneArgs* p, int n) {
     auto kern = plane_gemm_kernel<T>;
     if (T::LDS > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -666,11 +705,19 @@ int launch_gemm(dgm_gpu* g, const PlaneArgs& a) {
             return dgm::fail(g, DGM_ERR_HIP, "plane gemm: cannot reserve %d bytes of LDS: %s", T::LDS,
                              hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(kern, dim3(unsigned(a.per_full + a.per_part) * 8u), dim3(64 * T::WAVES), T::LDS, g->stream, a);
-    const int cut = a.tiles_m * a.tiles_n - a.full;
-    if (cut > 0)
-        hipLaunchKernelGGL(part_sum_kernel<T>, dim3(unsigned(cut) * (T::MT * T::NT * T::WAVES / 4)), dim3(256), 0,
-                           g->stream, a);
+    PlaneGroup grp{};
+    unsigned wgs[2] = {}, sums[2] = {};
+    for (int i = 0; i < n; ++i) {
+        grp.p[i] = p[i];
+        wgs[i] = unsigned(p[i].per_full + p[i].per_part) * 8u;
+        sums[i] = unsigned(p[i].tiles_m * p[i].tiles_n - p[i].full) * unsigned(T::MT * T::NT * T::WAVES / 4);
+    }
+    grp.first = int(wgs[0]);
+    hipLaunchKernelGGL(kern, dim3(wgs[0] + wgs[1]), dim3(64 * T::WAVES), T::LDS, g->stream, grp);
+    if (sums[0] + sums[1] > 0) {
+        grp.first = int(sums[0]);
+        hipLaunchKernelGGL(part_sum_kernel<T>, dim3(sums[0] + sums[1]), dim3(256), 0, g->stream, grp);
+    }
     return DGM_OK;
 }
 
@@ -727,20 +774,62 @@ double rounds_us(int tile, int64_t units, int cus, double blocks, double fold) {
            (rest ? round_us(tile, rest, cus, blocks, fold) : 0.0);
 }
 
-Plan plan_for(int64_t M, int64_t N, int64_t blocks, int chunk, double fold, int cus) {
+// uniform: all tiles whole or all of them cut.
+Plan plan_for(int64_t M, int64_t N, int64_t blocks, int chunk, double fold, bool uniform, int cus) {
     Plan best{0, 0, 0, 1, 1e30};
     for (int tile = 0; tile < 3; ++tile) {
         const Tile& t = kTiles[tile];
         const int64_t tiles = int64_t(dgm::ceil_div(M, t.tm)) * dgm::ceil_div(N, t.tn);
         const double us = rounds_us(tile, tiles, cus, double(blocks), fold);
         if (us < best.us) best = Plan{tile, tiles, tiles, 1, us};
-        const int64_t slots = int64_t(cus) * t.slots, full = tiles / slots * slots, cut = tiles - full;
+        const int64_t slots = int64_t(cus) * t.slots, full = uniform ? 0 : tiles / slots * slots,
+                      cut = tiles - full;
         for (int s = 2; s <= 8 && cut > 0 && blocks / s >= std::max(16, chunk); ++s) {
             const double part = double(dgm::ceil_div(blocks / chunk, s)) * chunk;
             const double cut_us = (full ? rounds_us(tile, full, cus, double(blocks), fold) : 0.0) +
                                   rounds_us(tile, cut * s, cus, part, fold) + 4.0 +
                                   double(cut) * s * t.tm * t.tn * 8.0 / 8e6;
             if (cut_us < best.us) best = Plan{tile, tiles, full, s, cut_us};
+        }
+    }
+    return best;
+}
+
+// The tile for two products of two planes in one launch, each cut (or not) as
+// it would be by itself, so that each element is the same sums either way.
+// Units are dealt in order to `slots` workgroups: the first product's fill
+// whole rounds and part of one, the second's start where a slot is free.
+int pair_tile(const int64_t (&M)[2], const int64_t (&N)[2], const int64_t (&blocks)[2], const int (&splits)[2],
+              int cus) {
+    int best = 0;
+    double best_us = 1e30;
+    for (int tile = 0; tile < 3; ++tile) {
+        const Tile& t = kTiles[tile];
+        const int64_t slots = int64_t(cus) * t.slots;
+        int64_t n[2];
+        for (int i = 0; i < 2; ++i)
+            n[i] = int64_t(dgm::ceil_div(M[i], t.tm)) * dgm::ceil_div(N[i], t.tn) * splits[i];
+        const int64_t all = std::min(n[0] + n[1], slots);
+        const double a = round_us(tile, all, cus, double(blocks[0]) / splits[0], 0.0);
+        const double b = round_us(tile, all, cus, double(blocks[1]) / splits[1], 0.0);
+        const int64_t rest = n[0] % slots;
+        double early = double(n[0] / slots) * a, late = early + a, us = rest ? late : early;
+        if (n[1] > 64 * slots) {   // many rounds: the throughput
+            us = early + (double(rest) * a + double(n[1]) * b) / double(slots);
+        } else {
+            for (int64_t left = n[1]; left > 0;) {
+                const bool e = early <= late || rest == 0;
+                double& clock = e ? early : late;
+                clock += b;
+                us = std::max(us, clock);
+                left -= e ? slots - rest : rest;
+            }
+        }
+        for (int i = 0; i < 2; ++i)
+            if (splits[i] > 1) us += double(n[i]) * t.tm * t.tn * 8.0 / 8e6;
+        if (us < best_us) {
+            best_us = us;
+            best = tile;
         }
     }
     return best;
@@ -753,6 +842,7 @@ Operand operand(const Src& s, int tile, int64_t blocks) {
     o.kb = int(blocks);
     o.parts = s.col ? int(std::min<int64_t>(kMaxParts, std::max<int64_t>(1, s.C / 64))) : 1;
     o.width = s.col && s.bits != 32 ? s.groups : s.R;
+    o.blocks = o.rb * int(dgm::ceil_div(o.kb, 16));
     return o;
 }
 
@@ -772,91 +862,125 @@ MaxArg max_arg(const Operand& o) {
     return m;
 }
 
-// Where the pieces of a product lie in the plane buffer.
-struct Layout {
-    size_t planes_a, planes_b, exps_a, exps_b, max_a, max_b, scales, parts, bytes;
-};
-
-Layout layout(const Operand& a, const Operand& b, int cut, int splits, const Tile& t) {
-    Layout l{};
-    auto take = [&](int64_t bytes) {
-        const size_t at = l.bytes;
-        l.bytes += size_t(round_up(bytes, 256));
-        return at;
-    };
-    l.planes_a = take(int64_t(a.rb) * a.kb * 2048);
-    l.planes_b = take(int64_t(b.rb) * b.kb * 2048);
-    l.exps_a = take(int64_t(a.rb) * 128);
-    l.exps_b = take(int64_t(b.rb) * 128);
-    l.max_a = take(int64_t(a.parts) * a.width * 4);
-    l.max_b = take(int64_t(b.parts) * b.width * 4);
-    l.scales = take(int64_t(b.gpad) * b.rb * 128);
-    l.parts = take(int64_t(cut) * splits * t.tm * t.tn * 4);
-    return l;
-}
-
 // The forward keeps the codes as one plane where a stage of 32 c lies in one
-// group: 2 products instead of 3, and half the bytes of B's planes.
+// group: 2 products instead of 3, and half the bytes of B's planes. Same run, three
+// products first: 2048 x 14336 x 4096 in groups of 128 669 -> 457 us, 4096 x
+// 4096 x 4096 380 -> 263, in groups of 32 (a fold every stage) 388 -> 302, 517
+// x 4100 x 4128 in groups of 32 94 -> 77.
 bool one_plane(const Src& b) { return b.bits != 32 && !b.col && b.G % 32 == 0; }
 
-// out[M, N] (+)= A B^T (+ bias); kNotFused, launching nothing,
-// without a plane buffer.
-int run(dgm_gpu* g, const Src& sa, const Src& sb, const float* bias, float* out, bool accumulate) {
-    const bool code = one_plane(sb);
-    const int gps = code ? sb.G / 32 : 1, chunk = code ? gps : 2;
-    const int64_t blocks = code ? sa.C / 16 : round_up(dgm::ceil_div(sa.C, 16), 2);
-    const Plan plan = plan_for(sa.R, sb.R, blocks, code ? chunk * 2 : chunk, code ? 1.0 / gps : 0.0, g->num_cus);
-    if (plan.tiles > (1 << 24)) return dgm::kNotFused;   // 32-bit tile numbers
-    const Tile& tile = kTiles[plan.tile];
-    Operand a = operand(sa, tile.tm, blocks), b = operand(sb, tile.tn, blocks);
-    if (code) b.gpad = int(blocks / 2 / gps);
-    const int cut = int(plan.tiles - plan.full);
-    const Layout at = layout(a, b, cut, plan.splits, tile);
-    uint8_t* ws = dgm::planes_buffer(g, at.bytes);
-    if (!ws) return dgm::kNotFused;
-    a.planes = ws + at.planes_a;
-    b.planes = ws + at.planes_b;
-    a.exps = reinterpret_cast<int*>(ws + at.exps_a);
-    b.exps = reinterpret_cast<int*>(ws + at.exps_b);
-    a.part = reinterpret_cast<uint32_t*>(ws + at.max_a);
-    b.part = reinterpret_cast<uint32_t*>(ws + at.max_b);
-    if (code) b.scales = reinterpret_cast<float*>(ws + at.scales);
-    const MaxArg x = max_arg(a), y = max_arg(b);
-    hipLaunchKernelGGL(row_max_kernel, dim3(unsigned(x.blocks + y.blocks)), dim3(256), 0, g->stream, x, y);
-    const int ba = a.rb * int(dgm::ceil_div(a.kb, 16)), bb = b.rb * int(dgm::ceil_div(b.kb, 16));
-    hipLaunchKernelGGL(split_kernel, dim3(unsigned(ba + bb)), dim3(256), 0, g->stream, a, b, ba);
-    PlaneArgs p{};
-    p.A = a.planes;
-    p.B = b.planes;
-    p.ea = a.exps;
-    p.eb = b.exps;
-    p.sa = sa;
-    p.sb = sb;
-    p.bias = bias;
-    p.out = out;
-    p.M = sa.R;
-    p.N = sb.R;
-    p.stages = int(code ? blocks / 2 : blocks);
-    p.chunk = chunk;
-    p.scales = b.scales;
-    p.scale_ld = b.rb * 32;
-    p.gps = gps;
-    p.tiles_m = a.rb * 32 / tile.tm;
-    p.tiles_n = b.rb * 32 / tile.tn;
-    p.full = int(plan.full);
-    p.per_full = (p.full + 7) / 8;
-    p.splits = plan.splits;
-    p.per_part = (cut * plan.splits + 7) / 8;
-    p.part = reinterpret_cast<float*>(ws + at.parts);
-    p.accumulate = accumulate;
-    if (code) {
-        if (plan.tile == 0) return launch_gemm<CodeWide>(g, p);
-        if (plan.tile == 1) return launch_gemm<CodeTall>(g, p);
-        return launch_gemm<CodeSmall>(g, p);
+// out[M, N] (+)= A B^T (+ bias), columns from cols1 on in out2.
+struct Product {
+    Src a, b;
+    const float* bias;
+    float *out, *out2;
+    int ldo, cols1;
+    bool accumulate;
+};
+
+// One product, or two of two planes; kNotFused, launching nothing, without a
+// plane buffer. dry: only whether there is one.
+int run(dgm_gpu* g, const Product* q, int n, bool dry = false) {
+    const bool code = n == 1 && one_plane(q[0].b);
+    const int gps = code ? q[0].b.G / 32 : 1, chunk = code ? gps : 2;
+    int64_t blocks[2] = {}, M[2] = {}, N[2] = {}, tiles[2] = {}, full[2] = {};
+    int splits[2] = {1, 1}, t = 0;
+    for (int i = 0; i < n; ++i) {
+        M[i] = q[i].a.R;
+        N[i] = q[i].b.R;
+        blocks[i] = code ? q[i].a.C / 16 : round_up(dgm::ceil_div(q[i].a.C, 16), 2);
     }
-    if (plan.tile == 0) return launch_gemm<Wide>(g, p);
-    if (plan.tile == 1) return launch_gemm<Tall>(g, p);
-    return launch_gemm<Small>(g, p);
+    // The backward's products are cut alike in one call and in two.
+    const bool uniform = n == 2 || q[0].a.col || q[0].b.col;
+    for (int i = 0; i < n; ++i) {
+        const Plan plan = plan_for(M[i], N[i], blocks[i], code ? chunk * 2 : chunk, code ? 1.0 / gps : 0.0, uniform,
+                                   g->num_cus);
+        t = plan.tile;
+        full[i] = plan.full;
+        splits[i] = plan.splits;
+    }
+    if (n == 2) t = pair_tile(M, N, blocks, splits, g->num_cus);
+    const Tile& tile = kTiles[t];
+    Operands op{};
+    MaxArgs mx{};
+    PlaneArgs p[2] = {};
+    // Where the pieces lie in the plane buffer.
+    size_t bytes = 0, at[4][4] = {}, parts[2] = {};
+    auto take = [&](int64_t size) {
+        const size_t here = bytes;
+        bytes += size_t(round_up(size, 256));
+        return here;
+    };
+    for (int i = 0; i < n; ++i) {
+        tiles[i] = int64_t(dgm::ceil_div(M[i], tile.tm)) * dgm::ceil_div(N[i], tile.tn);
+        if (tiles[i] > (1 << 24)) return dgm::kNotFused;   // 32-bit tile numbers
+        if (n == 2) full[i] = splits[i] == 1 ? tiles[i] : 0;
+        op.o[2 * i] = operand(q[i].a, tile.tm, blocks[i]);
+        op.o[2 * i + 1] = operand(q[i].b, tile.tn, blocks[i]);
+        if (code) op.o[1].gpad = int(blocks[0] / 2 / gps);
+        for (int k = 2 * i; k < 2 * i + 2; ++k) {
+            const Operand& o = op.o[k];
+            at[k][0] = take(int64_t(o.rb) * o.kb * 2048);
+            at[k][1] = take(int64_t(o.rb) * 128);
+            at[k][2] = take(int64_t(o.parts) * o.width * 4);
+            at[k][3] = take(int64_t(o.gpad) * o.rb * 128);
+        }
+        parts[i] = take((tiles[i] - full[i]) * splits[i] * tile.tm * tile.tn * 4);
+    }
+    uint8_t* ws = dgm::planes_buffer(g, bytes);
+    if (!ws) return dgm::kNotFused;
+    if (dry) return DGM_OK;
+    unsigned max_blocks = 0, split_blocks = 0;
+    for (int k = 0; k < 2 * n; ++k) {
+        Operand& o = op.o[k];
+        o.planes = ws + at[k][0];
+        o.exps = reinterpret_cast<int*>(ws + at[k][1]);
+        o.part = reinterpret_cast<uint32_t*>(ws + at[k][2]);
+        if (o.gpad) o.scales = reinterpret_cast<float*>(ws + at[k][3]);
+        mx.m[k] = max_arg(o);
+        max_blocks += unsigned(mx.m[k].blocks);
+        split_blocks += unsigned(o.blocks);
+    }
+    hipLaunchKernelGGL(row_max_kernel, dim3(max_blocks), dim3(256), 0, g->stream, mx);
+    hipLaunchKernelGGL(split_kernel, dim3(split_blocks), dim3(256), 0, g->stream, op);
+    for (int i = 0; i < n; ++i) {
+        const Operand &a = op.o[2 * i], &b = op.o[2 * i + 1];
+        PlaneArgs& r = p[i];
+        r.A = a.planes;
+        r.B = b.planes;
+        r.ea = a.exps;
+        r.eb = b.exps;
+        r.sa = q[i].a;
+        r.sb = q[i].b;
+        r.bias = q[i].bias;
+        r.out = q[i].out;
+        r.out2 = q[i].out2;
+        r.ldo = q[i].ldo;
+        r.cols1 = q[i].cols1;
+        r.M = int(M[i]);
+        r.N = int(N[i]);
+        r.stages = int(code ? blocks[i] / 2 : blocks[i]);
+        r.chunk = chunk;
+        r.scales = b.scales;
+        r.scale_ld = b.rb * 32;
+        r.gps = gps;
+        r.tiles_m = a.rb * 32 / tile.tm;
+        r.tiles_n = b.rb * 32 / tile.tn;
+        r.full = int(full[i]);
+        r.per_full = (r.full + 7) / 8;
+        r.splits = splits[i];
+        r.per_part = (int(tiles[i] - full[i]) * splits[i] + 7) / 8;
+        r.part = reinterpret_cast<float*>(ws + parts[i]);
+        r.accumulate = q[i].accumulate;
+    }
+    if (code) {
+        if (t == 0) return launch_gemm<CodeWide>(g, p, n);
+        if (t == 1) return launch_gemm<CodeTall>(g, p, n);
+        return launch_gemm<CodeSmall>(g, p, n);
+    }
+    if (t == 0) return launch_gemm<Wide>(g, p, n);
+    if (t == 1) return launch_gemm<Tall>(g, p, n);
+    return launch_gemm<Small>(g, p, n);
 }
 
 Src dense(const float* p, int R, int C, int64_t ld, int col) {
@@ -905,19 +1029,21 @@ bool planes_pay(int64_t M, int64_t N, int64_t K) {
 }
 
 int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias,
-               float* Y, const dgm_GemmP* p) {
-    return run(g, dense(X, int(p->M), int(p->K), p->K, 0), weights(bits, W, scale, p, 0),
-               p->hasBias ? bias : nullptr, Y, false);
+               float* Y, const dgm_GemmP* p, float* Y2) {
+    const int N = int(p->N), cols1 = Y2 ? N / 2 : N;
+    const Product q{dense(X, int(p->M), int(p->K), p->K, 0), weights(bits, W, scale, p, 0), p->hasBias ? bias : nullptr,
+                    Y, Y2, cols1, cols1, false};
+    return run(g, &q, 1, X == nullptr);
 }
 
-int planes_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, float* dX,
-              const dgm_GemmP* p) {
-    return run(g, dense(dY, int(p->M), int(p->N), p->N, 0), weights(bits, W, scale, p, 1), nullptr, dX, false);
-}
-
-int planes_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p, bool accumulate) {
-    return run(g, dense(dY, int(p->N), int(p->M), p->N, 1), dense(X, int(p->K), int(p->M), p->K, 1), nullptr, dW,
-               accumulate);
+int planes_bwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, const float* X, float* dX,
+               float* dW, const dgm_GemmP* p, bool accumulate) {
+    const int M = int(p->M), N = int(p->N), K = int(p->K);
+    Product q[2];
+    int n = 0;
+    if (dX) q[n++] = Product{dense(dY, M, N, N, 0), weights(bits, W, scale, p, 1), nullptr, dX, nullptr, K, K, false};
+    if (dW) q[n++] = Product{dense(dY, N, M, N, 1), dense(X, K, M, K, 1), nullptr, dW, nullptr, K, K, accumulate};
+    return run(g, q, n, dY == nullptr);
 }
 
 }  // namespace dgm
