@@ -223,7 +223,9 @@ struct AttnArgs {
     int o_ld;
 };
 
-__global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
+// NT threads: 256, or 1024 where the head's LDS leaves a CU one workgroup.
+template <int NT>
+__global__ __launch_bounds__(NT) void attn_mfma_kernel(AttnArgs a) {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) float sm[];
     const int T = a.T, D = a.D, H = a.H;
@@ -233,9 +235,9 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
     float* vt = ks + T * qs_ld;          // [D][T+4]  (V transposed)
     float* ps = vt + D * vt_ld;          // [16][T+4]
     const int tiles = T >> 4;
-    const int tb = blockIdx.x % tiles;
-    const int h = (blockIdx.x / tiles) % H;
-    const int b = blockIdx.x / (tiles * H);
+    int bh, tb;
+    dgm_rows::head_block(int(blockIdx.x), a.B * H, tiles, bh, tb);
+    const int h = bh % H, b = bh / H;
     const int t0 = tb * 16;
     const int hk = a.kv_heads == 1 ? 0 : h;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -250,12 +252,13 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
     const int hc = cpr >> 1, half = D >> 1;        // chunk pairs per row
     const int np = (16 + T) * hc;                  // pairs: 16 q rows first, then T k rows
     const int nv = T * cpr;                        // v chunks
-    constexpr int PB = 2, VB = 3;                  // pairs / v chunks per thread per batch
-    for (int bp = 0, bv = 0; bp < np || bv < nv; bp += PB * kThreads, bv += VB * kThreads) {
+    constexpr int NW = NT / 64;
+    constexpr int PB = NT == 256 ? 2 : 3, VB = NT == 256 ? 3 : 4;                  // pairs / v chunks per thread per batch
+    for (int bp = 0, bv = 0; bp < np || bv < nv; bp += PB * NT, bv += VB * NT) {
         float4 x1[PB], x2[PB], c1[PB], c2[PB], s1[PB], s2[PB], vv[VB], fv[VB];
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
-            const int e = min(bp + u * kThreads + int(threadIdx.x), np - 1);
+            const int e = min(bp + u * NT + int(threadIdx.x), np - 1);
             const int row = e / hc, c = e - row * hc;
             const int t = row < 16 ? t0 + row : row - 16;
             const float* src = row < 16 ? a.q + size_t(b * T + t) * a.q_ld + h * D
@@ -271,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
         }
 #pragma unroll
         for (int u = 0; u < VB; ++u) {
-            const int e = min(bv + u * kThreads + int(threadIdx.x), nv - 1);
+            const int e = min(bv + u * NT + int(threadIdx.x), nv - 1);
             const int t = e / cpr, c = e - t * cpr;
             const size_t r = size_t(b * T + t);
             vv[u] = *reinterpret_cast<const float4*>(a.v + r * a.kv_ld + hk * D + 4 * c);
@@ -279,7 +282,7 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
         }
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
-            const int e = bp + u * kThreads + int(threadIdx.x);
+            const int e = bp + u * NT + int(threadIdx.x);
             if (e >= np) break;
             const int row = e / hc, c = e - row * hc;
             float* dst = row < 16 ? qs + row * qs_ld : ks + (row - 16) * qs_ld;
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
         }
 #pragma unroll
         for (int u = 0; u < VB; ++u) {
-            const int e = bv + u * kThreads + int(threadIdx.x);
+            const int e = bv + u * NT + int(threadIdx.x);
             if (e >= nv) break;
             const int t = e / cpr, c = e - t * cpr;
             float v4[4] = {vv[u].x, vv[u].y, vv[u].z, vv[u].w};
@@ -329,7 +332,7 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
     // -- training saves: this workgroup's 16 query rows of q, and the same 16
     // token rows of k and v for head h (all workgroups of (b, h) cover T).
     if (a.qo) {
-        for (int e = threadIdx.x; e < 16 * D; e += kThreads) {
+        for (int e = threadIdx.x; e < 16 * D; e += NT) {
             const int r = e / D, d = e - r * D;
             const size_t o = size_t(b * T + t0 + r) * a.o_ld + h * D + d;
             a.qo[o] = qs[r * qs_ld + d];
@@ -338,9 +341,9 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
         }
     }
 
-    // -- scores: wave w takes key tiles w, w+4, ...
+    // -- scores: wave w takes key tiles w, w + NW, ...
     const size_t srow0 = (size_t(b) * H + h) * T + t0;   // row index into [B,H,T,T]
-    for (int kt = wave; kt < tiles; kt += 4) {
+    for (int kt = wave; kt < tiles; kt += NW) {
         f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         const float* qa = qs + r16 * qs_ld + 4 * q4;
         const float* kb = ks + (kt * 16 + r16) * qs_ld + 4 * q4;
@@ -363,27 +366,29 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
     }
     __syncthreads();
 
-    // -- row softmax (max, sum of exp, normalize as attn_softmax does): wave w
-    // takes rows 4w .. 4w+3 at once, 16 lanes per row, each lane T/16 keys.
+    // -- row softmax (max, sum of exp, normalize as attn_softmax does): LPR
+    // lanes per row, 64 / LPR rows to a wave.
     {
-        const int t = 4 * wave + q4;
+        constexpr int LPR = NT / 16;
+        const int lr = lane % LPR;
+        const int t = wave * (64 / LPR) + lane / LPR;
         float* row = ps + t * vt_ld;
         float* so = a.scores + (srow0 + t) * T;
         float* po = a.probs + (srow0 + t) * T;
         float mx = -INFINITY;
-        for (int s2 = r16; s2 < T; s2 += 16) {
+        for (int s2 = lr; s2 < T; s2 += LPR) {
             const float v = row[s2];
             so[s2] = v;
             mx = fmaxf(mx, v);
         }
 #pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 16));
+        for (int off = LPR / 2; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, LPR));
         float sum = 0.0f;
-        for (int s2 = r16; s2 < T; s2 += 16) sum += expf(row[s2] - mx);
+        for (int s2 = lr; s2 < T; s2 += LPR) sum += expf(row[s2] - mx);
 #pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 16);
+        for (int off = LPR / 2; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, LPR);
         const float inv = 1.0f / sum;
-        for (int s2 = r16; s2 < T; s2 += 16) {
+        for (int s2 = lr; s2 < T; s2 += LPR) {
             const float pv = expf(row[s2] - mx) * inv;
             row[s2] = pv;
             po[s2] = pv;
@@ -391,8 +396,8 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
     }
     __syncthreads();
 
-    // -- av = probs . v: wave w takes d tiles w, w+4, ...
-    for (int dt = wave; dt < (D >> 4); dt += 4) {
+    // -- av = probs . v: wave w takes d tiles w, w + NW, ...
+    for (int dt = wave; dt < (D >> 4); dt += NW) {
         f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         const float* pa = ps + r16 * vt_ld + 4 * q4;
         const float* vb = vt + (dt * 16 + r16) * vt_ld + 4 * q4;
@@ -421,15 +426,22 @@ bool attn_mfma_ok(int T, int D) {
 }
 
 int launch_attn_mfma(dgm_gpu* g, const AttnArgs& a) {
+    // Above half of the LDS a CU holds one workgroup: 16 waves instead of 4
+    // stage, score and normalize (4 x 256 tokens, 8 heads of 64: 157 KB, 39 us
+    // with 4 waves, 26 with 16).
     const size_t lds = attn_mfma_lds_bytes(a.T, a.D);
+    const bool wide = lds > 80 * 1024;
+    const void* kern = wide ? reinterpret_cast<const void*>(attn_mfma_kernel<1024>)
+                            : reinterpret_cast<const void*>(attn_mfma_kernel<256>);
     if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_mfma_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+        hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess)
             return dgm::fail(g, DGM_ERR_HIP, "attn_fwd: cannot reserve %zu bytes of LDS: %s", lds,
                              hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(attn_mfma_kernel, dim3(unsigned(a.B * a.H * (a.T / 16))), dim3(kThreads), lds, g->stream, a);
+    const dim3 grid(unsigned(a.B * a.H * (a.T / 16)));
+    if (wide) hipLaunchKernelGGL(attn_mfma_kernel<1024>, grid, dim3(1024), lds, g->stream, a);
+    else hipLaunchKernelGGL(attn_mfma_kernel<256>, grid, dim3(256), lds, g->stream, a);
     return dgm::check_launch(g, "attn_fwd");
 }
 

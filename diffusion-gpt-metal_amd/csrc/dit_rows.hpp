@@ -8,6 +8,16 @@
 
 namespace dgm_rows {
 
+// Workgroup w of heads x blocks: which head and which of its blocks. Workgroups
+// w, w + 8, ... run on one XCD, so a head's blocks are dealt to one residue:
+// its keys and values are then fetched into one L2 instead of eight.
+__device__ __forceinline__ void head_block(int w, int heads, int blocks, int& head, int& block) {
+    const bool even = heads % 8 == 0;
+    const int i = even ? w >> 3 : w;
+    head = even ? (w & 7) + 8 * (i / blocks) : i / blocks;
+    block = i % blocks;
+}
+
 __device__ __forceinline__ float sum16(float v) {
 #pragma unroll
     for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 16);

@@ -32,6 +32,8 @@
 #include <cmath>
 
 #include "common.hpp"
+
+#include <type_traits>
 #include "dit_rows.hpp"
 
 #pragma clang fp contract(off)
@@ -48,9 +50,12 @@ constexpr int kDwWaves = 16;
 // ---- rmsnorm backward (metal/kernels.metal:827-868), dx and dweight in one launch --
 // Workgroups [0, ndx) take 16 rows each for dx: one wave per row, the row's
 // sum(dy*w*x) a wave reduction (fp32, a different order than the reference's
-// sequential loop). The others take 64 columns each for dweight += sum over
-// rows: wave w sums rows w, w+16, ... and the 16 partial sums are added in
-// wave order, then added into dweight (the weight is shared by every loop). With
+// sequential loop; up to 1024 columns a row stays in registers). The others
+// take 16 columns each for dweight += sum over rows: of 64 groups of 16 lanes,
+// group w sums rows w, w+64, ... and the 64 partial sums are added in order,
+// then added into dweight (the weight is shared by every loop). Both are bound
+// by the latency of their loads: 1024 x 512 9.3 us (10.6 with 64 columns to a
+// workgroup, 16 row groups and rows read twice). With
 // `add`, dx[r, c] = add[r, c] + the row's dx (an acc_f of the result; add may
 // alias dx).
 __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __restrict__ x,
@@ -59,23 +64,47 @@ __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __r
                                                                 const float* __restrict__ dy, float* dx,
                                                                 const float* add, float* __restrict__ dweight,
                                                                 int rows, int cols, int ndx) {
-    __shared__ float part[kDwWaves][64];
+    constexpr int GROUPS = 4 * kDwWaves;   // of 16 lanes
+    constexpr int PER = 16;                // columns a lane keeps
+    __shared__ float part[GROUPS][16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (int(blockIdx.x) < ndx) {
         const int row = blockIdx.x * kDwWaves + wave;
         if (row >= rows) return;
         const float* xr = x + size_t(row) * cols;
         const float* gr = dy + size_t(row) * cols;
+        const float* ad = add ? add + size_t(row) * cols : nullptr;
+        float* o = dx + size_t(row) * cols;
+        const float rs = rstd[row];
+        const float rs3 = rs * rs * rs;
         float pt = 0.0f;
+        if (cols <= 64 * PER) {
+            float xv[PER], dyhat[PER], av[PER];
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int c = lane + 64 * u;
+                const bool in = c < cols;
+                xv[u] = in ? xr[c] : 0.0f;
+                dyhat[u] = in ? gr[c] * w[c] : 0.0f;
+                av[u] = in && ad ? ad[c] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < PER; ++u) pt += dyhat[u] * xv[u];
+            const float meanDyX = wave_sum(pt) / float(cols);
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int c = lane + 64 * u;
+                if (c >= cols) continue;
+                const float v = rs * dyhat[u] - xv[u] * rs3 * meanDyX;
+                o[c] = ad ? av[u] + v : v;
+            }
+            return;
+        }
         for (int c = lane; c < cols; c += 64) {
             const float dyhat = gr[c] * w[c];
             pt += dyhat * xr[c];
         }
         const float meanDyX = wave_sum(pt) / float(cols);
-        const float rs = rstd[row];
-        const float rs3 = rs * rs * rs;
-        float* o = dx + size_t(row) * cols;
-        const float* ad = add ? add + size_t(row) * cols : nullptr;
         for (int c = lane; c < cols; c += 64) {
             const float dyhat = gr[c] * w[c];
             const float v = rs * dyhat - xr[c] * rs3 * meanDyX;
@@ -83,28 +112,29 @@ __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __r
         }
         return;
     }
-    const int c = (int(blockIdx.x) - ndx) * 64 + lane;
+    const int l16 = lane & 15, group = wave * 4 + (lane >> 4);
+    const int c = (int(blockIdx.x) - ndx) * 16 + l16;
     float acc = 0.0f;
     if (c < cols) {
-        int r = wave;
-        for (; r + 7 * kDwWaves < rows; r += 8 * kDwWaves) {
+        int r = group;
+        for (; r + 7 * GROUPS < rows; r += 8 * GROUPS) {
             float v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int rr = r + u * kDwWaves;
+                const int rr = r + u * GROUPS;
                 v[u] = dy[size_t(rr) * cols + c] * x[size_t(rr) * cols + c] * rstd[rr];
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u) acc += v[u];
         }
-        for (; r < rows; r += kDwWaves) acc += dy[size_t(r) * cols + c] * x[size_t(r) * cols + c] * rstd[r];
+        for (; r < rows; r += GROUPS) acc += dy[size_t(r) * cols + c] * x[size_t(r) * cols + c] * rstd[r];
     }
-    part[wave][lane] = acc;
+    part[group][l16] = acc;
     __syncthreads();
-    if (wave == 0 && c < cols) {
+    if (threadIdx.x < 16 && c < cols) {
         float tot = 0.0f;
 #pragma unroll
-        for (int w2 = 0; w2 < kDwWaves; ++w2) tot += part[w2][lane];
+        for (int g2 = 0; g2 < GROUPS; ++g2) tot += part[g2][l16];
         dweight[c] += tot;
     }
 }
@@ -689,8 +719,10 @@ bool attn_bwd_fused_ok(const AttnBwdArgs& a) {
 // a row is contiguous along it a lane takes four consecutive k in one 16-byte
 // load. What bounds them is moving K, V, Q and dO of the head from L2 into
 // each of its T / 16 workgroups (128 KB at T = 256, D = 64). 4 x 256 tokens,
-// 8 heads of 64 (1.07 GFLOP a call): 31 + 17 us; the five passes of one thread
-// per output, which still take the sizes left over, 89 + 443 + 194 + 88 + 88.
+// 8 heads of 64 (1.07 GFLOP a call): 23 + 14 us (31 + 17 while the compiler
+// left loads inside the loops over keys and rows one step ahead of their use);
+// the five passes of one thread per output, which still take the sizes left
+// over, 89 + 443 + 194 + 88 + 88.
 constexpr int kAmThreads = 256;
 constexpr int kAmMaxT = 960;    // 16 (T + 4) floats of LDS within 64 KB
 constexpr int kAmMaxD = 128;    // dO operands of a lane: D / 16 float4
@@ -701,49 +733,56 @@ bool attn_mfma_bwd_ok(const AttnBwdArgs& a) {
            dgm::aligned(a.dout, 16);
 }
 
+template <int ND>   // D / 16
 __global__ __launch_bounds__(kAmThreads) void attn_mfma_rows_kernel(AttnBwdArgs a) {
     extern __shared__ __align__(16) float lds[];
-    const int T = a.T, D = a.D, H = a.H, ld = T + 4;
+    constexpr int D = 16 * ND;
+    const int T = a.T, H = a.H, ld = T + 4;
     float* S = lds;               // dP, then dS: [16][ld]
     float* dots = S + 16 * ld;    // [4 waves][16], then the row dots in [0][..]
     const int nblk = T / 16;
-    const int bh = blockIdx.x / nblk, t0 = blockIdx.x % nblk * 16;
+    int bh, t0;
+    dgm_rows::head_block(int(blockIdx.x), a.B * H, nblk, bh, t0);
+    t0 *= 16;
     const int b = bh / H, h = bh % H;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, q4 = lane >> 4;
     const int64_t row = int64_t(H) * D;
     const int64_t head0 = (int64_t(b) * T * H + h) * D;
     const int64_t pm0 = (int64_t(bh) * T + t0) * T;
 
     // dP tiles of 16 keys: wave w takes w, w + 4, ...
-    f32x4 g[kAmMaxD / 16];
+    f32x4 g[ND];
     const float* gp = a.dout + head0 + (t0 + r16) * row + 4 * q4;
 #pragma unroll
-    for (int j = 0; j < kAmMaxD / 16; ++j)
-        if (j * 16 < D) g[j] = *reinterpret_cast<const f32x4*>(gp + j * 16);
+    for (int j = 0; j < ND; ++j) g[j] = *reinterpret_cast<const f32x4*>(gp + j * 16);
     float dot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s0 = wave * 16; s0 < T; s0 += 64) {
+    f32x4 v[ND], vn[ND];
+    float pr[4], pn[4];
+    auto load = [&](int s0, f32x4 (&x)[ND], float (&p)[4]) {
         const float* vp = a.v + head0 + (s0 + r16) * row + 4 * q4;
         const float* pp = a.probs + pm0 + int64_t(4 * q4) * T + s0 + r16;
-        f32x4 v[kAmMaxD / 16];
-        float pr[4];
 #pragma unroll
-        for (int j = 0; j < kAmMaxD / 16; ++j)
-            if (j * 16 < D) v[j] = *reinterpret_cast<const f32x4*>(vp + j * 16);
+        for (int j = 0; j < ND; ++j) x[j] = *reinterpret_cast<const f32x4*>(vp + j * 16);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pr[e] = pp[e * T];
+        for (int e = 0; e < 4; ++e) p[e] = pp[e * T];
+    };
+    if (wave * 16 < T) load(wave * 16, v, pr);
+    for (int s0 = wave * 16; s0 < T; s0 += 64) {
+        if (s0 + 64 < T) load(s0 + 64, vn, pn);   // the next tile while this one is multiplied
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < kAmMaxD / 16; ++j)
-            if (j * 16 < D) {
+        for (int j = 0; j < ND; ++j)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(g[j][u], v[j][u], acc, 0, 0, 0);
-            }
+            for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(g[j][u], v[j][u], acc, 0, 0, 0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             S[(4 * q4 + e) * ld + s0 + r16] = acc[e];
             if (a.keep_dp) a.dprobs[pm0 + int64_t(4 * q4 + e) * T + s0 + r16] = acc[e];
             dot[e] += acc[e] * pr[e];
+            pr[e] = pn[e];
         }
+#pragma unroll
+        for (int j = 0; j < ND; ++j) v[j] = vn[j];
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -752,26 +791,51 @@ __global__ __launch_bounds__(kAmThreads) void attn_mfma_rows_kernel(AttnBwdArgs 
         if (r16 == 0) dots[wave * 16 + 4 * q4 + e] = dot[e];
     }
     __syncthreads();
-    for (int i = tid; i < 16 * T; i += kAmThreads) {
-        const int r = i / T, s = i % T;
-        const float d = (dots[r] + dots[16 + r]) + (dots[32 + r] + dots[48 + r]);
-        const float ds = a.probs[pm0 + i] * (S[r * ld + s] - d);
-        S[r * ld + s] = ds;
-        a.dscores[pm0 + i] = ds;
+    {   // four rows to a wave
+        float d[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = wave * 4 + e;
+            d[e] = (dots[r] + dots[16 + r]) + (dots[32 + r] + dots[48 + r]);
+        }
+#pragma unroll 4
+        for (int s = lane; s < T; s += 64) {
+            float p[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p[e] = a.probs[pm0 + int64_t(wave * 4 + e) * T + s];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float* at = S + (wave * 4 + e) * ld + s;
+                const float ds = p[e] * (*at - d[e]);
+                *at = ds;
+                a.dscores[pm0 + int64_t(wave * 4 + e) * T + s] = ds;
+            }
+        }
     }
     __syncthreads();
     for (int d0 = wave * 16; d0 < D; d0 += 64) {
         const float* sp = S + r16 * ld + 4 * q4;
         const float* kp = a.k + head0 + int64_t(4 * q4) * row + d0 + r16;
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-        for (int s0 = 0; s0 < T; s0 += 16) {
+        int s0 = 0;
+        for (; s0 + 64 <= T; s0 += 64) {   // the loads of 64 keys in flight together
+            float y[4][4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) y[i][u] = kp[(s0 + 16 * i + u) * row];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(sp + s0 + 16 * i);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[i][u], acc, 0, 0, 0);
+            }
+        }
+        for (; s0 < T; s0 += 16) {
             const f32x4 x = *reinterpret_cast<const f32x4*>(sp + s0);
-            float y[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) y[u] = kp[(s0 + u) * row];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], acc, 0, 0, 0);
+            for (int u = 0; u < 4; ++u)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], kp[(s0 + u) * row], acc, 0, 0, 0);
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) a.dq[head0 + (t0 + 4 * q4 + e) * row + d0 + r16] = acc[e] * a.scale;
@@ -782,7 +846,9 @@ __global__ __launch_bounds__(kAmThreads) void attn_mfma_keys_kernel(AttnBwdArgs 
     __shared__ f32x4 part[3][8][64];   // waves 1 .. 3
     const int T = a.T, D = a.D, H = a.H;
     const int nblk = T / 16;
-    const int bh = blockIdx.x / nblk, s0 = blockIdx.x % nblk * 16;
+    int bh, s0;
+    dgm_rows::head_block(int(blockIdx.x), a.B * H, nblk, bh, s0);
+    s0 *= 16;
     const int b = bh / H, h = bh % H;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, q4 = lane >> 4;
     const int64_t row = int64_t(H) * D;
@@ -793,22 +859,33 @@ __global__ __launch_bounds__(kAmThreads) void attn_mfma_keys_kernel(AttnBwdArgs 
     f32x4 accv[4], acck[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) accv[j] = acck[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-    for (int t = wave * tq + q4; t < (wave + 1) * tq; t += 4) {
-        const float p = a.probs[pm0 + int64_t(t) * T], ds = a.dscores[pm0 + int64_t(t) * T];
-        const int64_t at = head0 + t * row + dbase + r16;
-        float x[4], y[4];
+    // STEPS steps of four t: their loads in flight together.
+    auto steps = [&](int t0, auto count) {
+        constexpr int STEPS = decltype(count)::value;
+        float p[STEPS], ds[STEPS], x[STEPS][4], y[STEPS][4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            x[j] = j < nd ? a.dout[at + j * 16] : 0.0f;
-            y[j] = j < nd ? a.q[at + j * 16] : 0.0f;
+        for (int i = 0; i < STEPS; ++i) {
+            const int t = t0 + 4 * i + q4;
+            p[i] = a.probs[pm0 + int64_t(t) * T];
+            ds[i] = a.dscores[pm0 + int64_t(t) * T];
+            const int64_t at = head0 + t * row + dbase + r16;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                x[i][j] = j < nd ? a.dout[at + j * 16] : 0.0f;
+                y[i][j] = j < nd ? a.q[at + j * 16] : 0.0f;
+            }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            accv[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, x[j], accv[j], 0, 0, 0);
-            acck[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ds, y[j], acck[j], 0, 0, 0);
-        }
-    }
+        for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                accv[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], x[i][j], accv[j], 0, 0, 0);
+                acck[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ds[i], y[i][j], acck[j], 0, 0, 0);
+            }
+    };
+    int t = wave * tq;
+    for (; t + 16 <= (wave + 1) * tq; t += 16) steps(t, std::integral_constant<int, 4>());
+    for (; t < (wave + 1) * tq; t += 4) steps(t, std::integral_constant<int, 1>());
     if (wave > 0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -968,7 +1045,7 @@ bool bad_count(int64_t n) { return n < 0 || n > dgm::kMaxIndex; }
 int launch_rms_bwd(dgm_gpu* g, const float* x, const float* rstd, const float* w, const float* dy, float* dx,
                    float* dweight, int64_t rows, int64_t cols, const float* add = nullptr) {
     if (rows == 0 || cols == 0) return DGM_OK;
-    const int ndx = int((rows + kDwWaves - 1) / kDwWaves), ndw = int((cols + 63) / 64);
+    const int ndx = int((rows + kDwWaves - 1) / kDwWaves), ndw = int((cols + 15) / 16);
     hipLaunchKernelGGL(rms_bwd_kernel, dim3(unsigned(ndx + ndw)), dim3(64 * kDwWaves), 0, g->stream, x, rstd, w, dy,
                        dx, add, dweight, int(rows), int(cols), ndx);
     return dgm::check_launch(g, "rms_bwd");
@@ -1008,8 +1085,14 @@ int launch_attn_bwd(dgm_gpu* g, const AttnBwdArgs& a) {
     }
     if (attn_mfma_bwd_ok(a)) {
         const unsigned grid = unsigned(a.B) * unsigned(a.H) * unsigned(a.T / 16);
-        hipLaunchKernelGGL(attn_mfma_rows_kernel, dim3(grid), dim3(kAmThreads),
-                           (size_t(16) * (a.T + 4) + 64) * sizeof(float), g->stream, a);
+        const size_t lds = (size_t(16) * (a.T + 4) + 64) * sizeof(float);
+        switch (a.D / 16) {
+#define DGM_AM_ROWS(ND) \
+    case ND: hipLaunchKernelGGL(attn_mfma_rows_kernel<ND>, dim3(grid), dim3(kAmThreads), lds, g->stream, a); break;
+            DGM_AM_ROWS(1) DGM_AM_ROWS(2) DGM_AM_ROWS(3) DGM_AM_ROWS(4)
+            DGM_AM_ROWS(5) DGM_AM_ROWS(6) DGM_AM_ROWS(7) DGM_AM_ROWS(8)
+#undef DGM_AM_ROWS
+        }
         hipLaunchKernelGGL(attn_mfma_keys_kernel, dim3(grid, unsigned((a.D + 63) / 64)), dim3(kAmThreads), 0, g->stream,
                            a);
         return dgm::check_launch(g, "attn_bwd");

@@ -288,16 +288,25 @@ __device__ __forceinline__ void split_part(const Operand& o, int block) {
     const int rb = block / chunks, chunk = block % chunks;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = rb * 32 + (lane & 31), h = lane >> 5;
-    const int at = BITS != 32 && COL ? r / o.s.G : r;
-    uint32_t m = 0;
-    if (r < o.s.R)
-        for (int i = 0; i < o.parts; ++i) m = max(m, o.part[int64_t(i) * o.width + at]);
-    const int e = row_exp(m, BITS == 32 ? 0 : (BITS == 8 ? 7 : 3));
-    if (chunk == 0 && wave == 0 && h == 0) o.exps[r] = e;
-    const float f = exp_factor(e);
     float v[4][8];
 #pragma unroll
     for (int u = 0; u < 4; ++u) load8<BITS, COL>(o.s, r, (chunk * 16 + u * 4 + wave) * 16 + 8 * h, v[u]);
+    const int at = BITS != 32 && COL ? r / o.s.G : r;
+    uint32_t m = 0;
+    if (r < o.s.R) {
+        if constexpr (COL) {
+            uint32_t p[kMaxParts];   // all in flight together
+#pragma unroll
+            for (int i = 0; i < kMaxParts; ++i) p[i] = o.part[int64_t(min(i, o.parts - 1)) * o.width + at];
+#pragma unroll
+            for (int i = 0; i < kMaxParts; ++i) m = max(m, p[i]);
+        } else {
+            m = o.part[r];
+        }
+    }
+    const int e = row_exp(m, BITS == 32 ? 0 : (BITS == 8 ? 7 : 3));
+    if (chunk == 0 && wave == 0 && h == 0) o.exps[r] = e;
+    const float f = exp_factor(e);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int kb = chunk * 16 + u * 4 + wave;
