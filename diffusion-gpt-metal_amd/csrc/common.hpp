@@ -216,9 +216,10 @@ int gemm_bwd_fold(dgm_gpu* g, const int8_t* codesT, const float* scalesT, const 
                   float* dW, int M, int N, int K, int G, bool accumulate, const float* sg_gate, const float* sg_up);
 
 // Large GEMMs on 16-bit MFMA over split operands (gemm_planes.hip): the
-// forward, dX and dW in the fp32 mode, where planes_pay says that they are
+// forward, dX and dW in the fp32 mode, where planes_pay_* say that they are
 // the faster way. Each product returns kNotFused, launching nothing, when planes_buffer has none.
-bool planes_pay(int64_t M, int64_t N, int64_t K);
+bool planes_pay_fwd(int64_t M, int64_t N, int64_t K);
+bool planes_pay_bwd(int64_t M, int64_t N, int64_t K);
 // Y2 (may be null): the upper half of the columns, Y and Y2 [M, N / 2]
 // (N % 64 == 0). X (dY) null: launches nothing, DGM_OK where the call would not
 // return kNotFused. dX or dW may be null: the other alone.

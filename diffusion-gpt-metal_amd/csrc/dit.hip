@@ -935,7 +935,13 @@ namespace {
 // that pays and the context has the buffer for it.
 int gate_up_planes(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_linear& L, const float* in, float* gate, float* up) {
     const int64_t M = int64_t(c->B) * c->T;
-    if (c->F % 32 != 0 || !planes_pay(M, 2 * int64_t(c->F), c->C)) return kNotFused;
+    // Against the one launch that also runs the row chain and SwiGLU, one block's
+    // forward in us, that launch and the planes: 2 x 256 x 512 -> 1536 (0.75 * 2^30
+    // products) 106.8 and 111.3, 8 x 256 x 256 -> 1024 (2^30) 107.9 and 104.9,
+    // 8 x 128 x 384 -> 1536 (1.12) 132.8 and 122.4, 4 x 256 x 512 -> 2048 (2) 170.8
+    // and 135.3.
+    if (c->F % 32 != 0 || M < 128 || c->C < 128 || double(M) * 2.0 * c->F * c->C < double(int64_t(7) << 27))
+        return kNotFused;
     const dgm_GemmP gp{uint32_t(M), uint32_t(2 * c->F), uint32_t(c->C), 0u, uint32_t(c->bits == 32 ? 0 : c->group),
                        0, 0, 0};
     return planes_fwd(g, c->bits, c->bits == 32 ? static_cast<const void*>(L.w) : L.q, L.scale, in, nullptr, gate, &gp,

@@ -1541,7 +1541,7 @@ int dgm_dit_backward(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w,
     // backward.
     auto large = [&](int64_t N, int64_t K) {
         const dgm_GemmP gp{uint32_t(M), uint32_t(N), uint32_t(K), 0u, uint32_t(bits == 32 ? 0 : G), 0, 0, 0};
-        return dgm::planes_pay(M, N, K) &&
+        return dgm::planes_pay_bwd(M, N, K) &&
                dgm::planes_bwd(g, bits, nullptr, nullptr, nullptr, nullptr, t1, t1, &gp, true) == DGM_OK;
     };
     // gemmBwd of stacked linear li (0 [wq; wk; wv], 1 wo, 2 [wgate; wup],

@@ -1613,7 +1613,7 @@ int gemm_f32_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const 
     // Larger M in the reduced-precision mode: bf16 MFMA with W dequantized in LDS.
     if (g->math == DGM_MATH_BF16 && bf16_ok(bits, W, X, scale, p))
         return bf16_fwd(g, bits, W, scale, X, bias, Y, p);
-    if (planes_pay(p->M, p->N, p->K)) {
+    if (planes_pay_fwd(p->M, p->N, p->K)) {
         const int rc = planes_fwd(g, bits, W, scale, X, bias, Y, p);
         if (rc != kNotFused) return rc;
     }
@@ -1653,7 +1653,7 @@ int gemm_f32_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const 
 
 int gemm_f32_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY,
                 float* dX, const dgm_GemmP* p) {
-    if (planes_pay(p->M, p->N, p->K)) {
+    if (planes_pay_bwd(p->M, p->N, p->K)) {
         const int rc = planes_bwd(g, bits, W, scale, dY, nullptr, dX, nullptr, p, false);
         if (rc != kNotFused) return rc;
     }
@@ -1683,7 +1683,7 @@ int gemm_f32_dx(dgm_gpu* g, int bits, const void* W, const float* scale, const f
 
 int gemm_f32_dw(dgm_gpu* g, const float* dY, const float* X, float* dW, const dgm_GemmP* p,
                 bool accumulate) {
-    if (planes_pay(p->M, p->N, p->K)) {
+    if (planes_pay_bwd(p->M, p->N, p->K)) {
         const int rc = planes_bwd(g, 32, nullptr, nullptr, dY, X, nullptr, dW, p, accumulate);
         if (rc != kNotFused) return rc;
     }
@@ -1710,7 +1710,7 @@ int gemm_f32_bwd_pair(dgm_gpu* g, int bits, const void* W, const float* scale, c
                       float* dX, float* dW, const dgm_GemmP* p, bool accumulate, bool* fused, const float* sg_gate,
                       const float* sg_up) {
     *fused = false;
-    if (!sg_gate && planes_pay(p->M, p->N, p->K)) {
+    if (!sg_gate && planes_pay_bwd(p->M, p->N, p->K)) {
         const int rc = planes_bwd(g, bits, W, scale, dY, X, dX, dW, p, accumulate);
         *fused = rc != kNotFused;
         if (*fused) return rc;

@@ -1027,14 +1027,29 @@ Src weights(int bits, const void* W, const float* scale, const dgm_GemmP* p, int
 
 namespace dgm {
 
-// Where three launches and the planes' traffic cost less than they save. The
-// fp32 MFMA kernels run at 43-57 TFLOP/s from about 2^28 products on; the
-// planes take 18 us and more before the first MFMA. Measured: 256 x 1024 x 1024
-// (2^28) 10.8 us against 23, 512 x 1024 x 768 dX + dW 37 against 62,
-// 1024 x 2048 x 512 (2^30) 35 against 26, 1024 x 512 x 2048 51 against 30,
-// 128 x 14336 x 4096 307 against 130.
-bool planes_pay(int64_t M, int64_t N, int64_t K) {
-    return M >= 128 && N >= 128 && K >= 128 && double(M) * double(N) * double(K) >= double(int64_t(7) << 27);
+// Where three or four launches and the planes' traffic cost less than they
+// save: the planes take 20 us and more before the last sum. Measured on int8
+// in groups of 32, us on the fp32 MFMA kernels and on these (G = 2^30 products):
+//   forward, K below 1280: 1024 x 768 x 768 (0.56 G) 24.7 and 27.7, 1100 x 1100 x
+//     576 (0.65 G) 27.8 and 31.7, 8192 x 192 x 480 (0.70 G) 34.8 and 33.4 (int4
+//     29.9 and 33.4), 256 x 4096 x 1024 (1 G) 45.5 and 30.6 (int4 38.4 and 29.1);
+//   forward, longer K, where those have few tiles: 256 x 512 x 2240 (0.27 G) 22.0
+//     and 28.8, 256 x 1024 x 2048 (0.5 G) 40.6 and 29.3 but fp32 24.9 and 27.5,
+//     128 x 2304 x 2048 (0.56 G) 58.0 and 30.9, fp32 35.2 and 31.3;
+//   up to 64 rows are the decode's; 70 x 4096 x 4096 110.6 and 55.7.
+bool planes_pay_fwd(int64_t M, int64_t N, int64_t K) {
+    return M > 64 && N >= 128 && K >= 128 &&
+           double(M) * double(N) * double(K) >= double(K >= 1280 ? int64_t(9) << 26 : int64_t(3) << 28);
+}
+
+// One line for dX, dW and both, which give the same bits (gemmBwd's promise),
+// where neither alone loses (in groups of 32, us as above: both, dX, dW):
+//   512 x 1024 x 1024 (0.5 G) 41.4 and 40.1, 21.6 and 33.7, 18.5 and 25.3;
+//   1024 x 768 x 768 (0.56 G) 48.8 and 39.3, 23.2 and 33.5, 24.7 and 26.0;
+//   640 x 1536 x 768 (0.70 G) 68.4 and 44.9, 35.6 and 35.1, 30.7 and 29.6;
+//   70 x 4096 x 4096 (1.09 G) 138 and 83, 70 and 58, 56 and 32.
+bool planes_pay_bwd(int64_t M, int64_t N, int64_t K) {
+    return M > 64 && N >= 128 && K >= 128 && double(M) * double(N) * double(K) >= double(int64_t(11) << 26);
 }
 
 int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias,

@@ -2,7 +2,7 @@
 
 Sizes sit at the edges of its tiles (128 and 256 rows), stages (16 and 32 of
 the contraction) and parts (tiles cut along the contraction), on both sides of
-where it is taken (7 * 2^27 products). The reference is the float64 product of
+where each is taken. The reference is the float64 product of
 the same operands. Bound per element, against the row's and column's 2-norms
 |a| |b| (every element of a split operand is within 2^-24 of its value, and a
 sum of n products, rounded once per 8, is within n/8 * 2^-24 of |a| |b| at
@@ -58,6 +58,10 @@ SHAPES = [   # bits, M, N, K, G
     (4, 2048, 4352, 256, 128),      # whole tiles and a cut last round
     (8, 1000, 1029, 960, 96),       # groups of three stages, an odd number of tiles cut
     (4, 300, 3000, 1056, 32),       # an odd number of stages
+    (8, 65, 2700, 4288, 32),        # fewest rows; all three just above their lines
+    (32, 67, 2305, 4000, 8),        # forward above its line for a long contraction, dX and dW below theirs
+    (4, 641, 1504, 768, 32),        # dX and dW above their line, forward below its
+    (8, 96, 8192, 960, 96),         # between those two lines, few rows
 ]
 
 
