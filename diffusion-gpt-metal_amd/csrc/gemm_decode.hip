@@ -104,7 +104,12 @@ struct DecShape {
 // the exponents the prepare pass writes, per (block, row), the fp32 term
 // -136 * sum over the block of bf16(x): the GEMM feeds the codes as
 // 128 + (code + 8), exact in bf16, and this term removes the offset 136.
-template <int BITS, int P>
+//
+// SPG > 0 (groups inside a block, see decode_kernel): step kk holds the
+// consecutive k 32 kk .. of the block, lane group q eight of them, and an
+// infinity or NaN keeps its place (the first piece holds it, the second 0; the
+// exponent is the finite elements'), so that it meets the codes as in fp32.
+template <int BITS, int P, int SPG>
 __global__ __launch_bounds__(256) void decode_prep_kernel(const float* __restrict__ X, _Float16* __restrict__ XP,
                                                           int8_t* __restrict__ ex, float* __restrict__ corr, int M,
                                                           int K, int MT) {
@@ -117,10 +122,11 @@ __global__ __launch_bounds__(256) void decode_prep_kernel(const float* __restric
     const int row = 16 * mt + c;
     float v[SH::KL];
     if (row < M) {
-        const float4* src = reinterpret_cast<const float4*>(X + size_t(row) * K + size_t(blk) * SH::KB + SH::KL * q);
+        const float4* src = reinterpret_cast<const float4*>(X + size_t(row) * K + size_t(blk) * SH::KB +
+                                                            (SPG ? 8 : SH::KL) * q);
 #pragma unroll
         for (int i = 0; i < SH::KL / 4; ++i) {
-            const float4 f = src[i];
+            const float4 f = src[SPG ? 8 * (i / 2) + i % 2 : i];
             v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
         }
     } else {
@@ -156,8 +162,8 @@ __global__ __launch_bounds__(256) void decode_prep_kernel(const float* __restric
     bool fin = true;
 #pragma unroll
     for (int i = 0; i < SH::KL; ++i) {
-        mx = fmaxf(mx, fabsf(v[i]));
-        fin = fin && __builtin_isfinite(v[i]);
+        mx = fmaxf(mx, SPG && !__builtin_isfinite(v[i]) ? 0.0f : fabsf(v[i]));
+        fin = fin && (SPG || __builtin_isfinite(v[i]));
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
@@ -187,7 +193,7 @@ __global__ __launch_bounds__(256) void decode_prep_kernel(const float* __restric
             const float xs = bad2 ? nan : v[frag_k<BITS>(0, kk, t)] * pw;
             const _Float16 h1 = _Float16(xs);
             h[0][t] = h1;
-            if constexpr (P == 2) h[1][t] = _Float16(xs - float(h1));
+            if constexpr (P == 2) h[1][t] = SPG && !__builtin_isfinite(xs) ? _Float16(0.0f) : _Float16(xs - float(h1));
         }
         const int s = blk * SH::SPB + kk;
 #pragma unroll
@@ -253,11 +259,27 @@ struct Schedule {
 // 0), transposed to [group][64 columns] behind the ring: a compute wave then
 // reads a block's 16 columns from LDS (16 consecutive words: no bank
 // conflict) instead of gathering them from 16 rows in HBM.
-template <int BITS, int MT, int P, int D, int MW, bool SL>
+//
+// SPG > 0: a group is SPG steps of a block rather than whole blocks (groups of
+// 32, and int4 groups of 64). The MFMA sums over its four lane groups, so a
+// step has to lie in one group: it takes 32 consecutive k, 4 (int8: 8) bytes of
+// codes to a lane instead of the 16 the lane reads at once otherwise, and every
+// group's partial is folded by itself. The scales go through a ring of their own
+// beside the weights': the producer reads four consecutive groups of each row
+// with one 16-byte direct-to-LDS load per lane.
+// Against the fp32 MFMA kernels (us): 1 x 14336 x 4096 int4 in groups of 32 73.2
+// -> 15.8, 24 rows 145.8 -> 21.8, 24 x 4096 x 14336 151.9 -> 26.8; int4 in groups of
+// 64 145.2 -> 18.6 for 24 x 14336 x 4096, int8 in groups of 32 144.7 -> 25.7. The
+// conversions and the folds bound it (VALU): the same with groups of 128 17.7.
+template <int BITS, int MT, int P, int D, int MW, bool SL, int SPG>
 __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecArgs a) {
     using SH = DecShape<BITS>;
     using SC = Schedule<BITS, MT, P, D, SL>;
     constexpr bool BF = SC::BF;   // reduced-precision int4: bf16 fragments, offset codes
+    static_assert(SPG == 0 || (SL && !BF), "groups inside a block: scales in LDS, f16 pieces");
+    constexpr int GPB = SPG ? SH::SPB / (SPG ? SPG : 1) : 0;   // groups per block
+    constexpr int SQ = 2 * GPB;     // scale loads per interval: 8 GPB groups, four to a load
+    constexpr int SSLOT = SQ * 1024;   // bytes of an interval's scales: [group / 4][64 columns][4]
     using XF = std::conditional_t<BF, bf16x8, f16x8>;
     static_assert(D >= 1 && D <= SH::SPB, "prefetch depth: at most one block ahead");
     // Activation ring: XR step slots, a power of two above D dividing SPC, so
@@ -297,6 +319,8 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
             doff[i] = uint32_t(min(n0 + r, a.N - 1)) * uint32_t(a.rowb) + 16u * uint32_t(piece);
         }
         const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(smem));
+        // Lane l moves the scales of row n0 + l (rows past N re-read row N - 1).
+        const uint32_t srow = uint32_t(min(n0 + lane, a.N - 1)) * uint32_t(a.groups) * 4u;
         auto dma_interval = [&](int t) {
 #pragma unroll
             for (int cw = 0; cw < 4; ++cw) {
@@ -314,13 +338,25 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
                                  : "memory", "m0");
 #pragma clang diagnostic pop
             }
+            if constexpr (SPG > 0) {
+                // Groups past the row's end (an interval that is not whole)
+                // re-read its last four; nothing uses them.
+                const int first = (ch0 + 4 * iv(t < T ? t : T - 1)) * 2 * GPB;
+                const uint32_t lds = lds0 + DEC_LDS + uint32_t(t % DEC_SLOTS) * SSLOT;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+#pragma unroll
+                for (int i = 0; i < SQ; ++i)
+                    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + i * 1024),
+                                 "v"(srow + 4u * uint32_t(min(first + 4 * i, a.groups - 4))), "s"(a.S)
+                                 : "memory", "m0");
+#pragma clang diagnostic pop
+            }
         };
         static_assert(DEC_SLOTS == 4, "the waits below count at most two intervals ahead");
         dma_interval(0);
-        if constexpr (SL) {
-            // Scales: one 4-byte gather per group, lane l = row n0 + l
-            // (rows past N re-read row N - 1).
-            const uint32_t srow = uint32_t(min(n0 + lane, a.N - 1)) * uint32_t(a.groups) * 4u;
+        if constexpr (SL && SPG == 0) {
+            // Scales: one 4-byte gather per group.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
             const int ng = ((2 * (ch0 + nch) - 1) >> a.gshift) - g0 + 1;
@@ -332,7 +368,7 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
         }
         for (int t = 1; t < DEC_SLOTS - 1 && t < T; ++t) dma_interval(t);
         for (int t = 0; t < T; ++t) {
-            // Interval t has landed once at most `ahead` newer intervals (32
+            // Interval t has landed once at most `ahead` newer intervals (32 + SQ
             // loads each, issued after it) are in flight; no interval past T
             // is ever issued. The counter holds at most 63, so with two ahead
             // this also waits for the first load of interval t + 1. The
@@ -341,7 +377,7 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
             if (ahead >= 2)
                 asm volatile("s_waitcnt vmcnt(63)" ::: "memory");
             else if (ahead == 1)
-                asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(32 + SQ) : "memory");
             else
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
@@ -415,7 +451,8 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct) acc[mt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    u32x4 wc[4];   // the lane's 16-byte code piece of the current block, per column tile
+    u32x4 wc[4];   // the lane's 16 bytes of codes of the current block, per column tile
+    float gs[4][SPG ? GPB : 1];   // the block's scales (SPG > 0)
 
     if (cnt > 0) {
 #pragma unroll
@@ -454,10 +491,34 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
 #pragma unroll
                 for (int ct = 0; ct < 4; ++ct) {
                     const int r = 16 * ct + c;
-                    const int sl = (4 * hb + q) ^ (r & 7);
-                    wc[ct] = *reinterpret_cast<const u32x4*>(cs + r * 128 + sl * 16);
+                    if constexpr (SPG == 0) {
+                        const int sl = (4 * hb + q) ^ (r & 7);
+                        wc[ct] = *reinterpret_cast<const u32x4*>(cs + r * 128 + sl * 16);
+                    } else if constexpr (BITS == 4) {
+                        // Dword q of each of the block's four pieces.
+#pragma unroll
+                        for (int p = 0; p < 4; ++p)
+                            wc[ct][p] = *reinterpret_cast<const uint32_t*>(cs + r * 128 + ((4 * hb + p) ^ (r & 7)) * 16 + 4 * q);
+                    } else {
+                        // Bytes 8 q .. of each two pieces.
+#pragma unroll
+                        for (int p = 0; p < 2; ++p) {
+                            const u32x2 d = *reinterpret_cast<const u32x2*>(
+                                cs + r * 128 + ((4 * hb + 2 * p + (q >> 1)) ^ (r & 7)) * 16 + 8 * (q & 1));
+                            wc[ct][2 * p] = d[0];
+                            wc[ct][2 * p + 1] = d[1];
+                        }
+                    }
                 }
-                if constexpr (SL) {
+                if constexpr (SPG > 0) {
+                    const int gl = (2 * kw + hb) * GPB;   // in the interval: a multiple of GPB (4 or 2)
+                    const float* sc = reinterpret_cast<const float*>(smem + DEC_LDS + (j % DEC_SLOTS) * SSLOT) +
+                                      (gl >> 2) * 256 + (gl & 3) + 4 * c;
+#pragma unroll
+                    for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+                        for (int e = 0; e < GPB; ++e) gs[ct][e] = sc[64 * ct + e];
+                } else if constexpr (SL) {
                     const int g = ((2 * (ch0 + kw + 4 * iv(j)) + hb) >> a.gshift) - g0;
                     const float* sc = reinterpret_cast<const float*>(smem + DEC_LDS) + g * 64 + c;
 #pragma unroll
@@ -488,7 +549,7 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
                     const f16x8 b = {h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) {
-                        f32x4 t0 = kk == 0 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : tmp[mt][ct];
+                        f32x4 t0 = (SPG ? kk % (SPG ? SPG : 1) == 0 : kk == 0) ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : tmp[mt][ct];
 #pragma unroll
                         for (int p = 0; p < P; ++p)
                             t0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[slot][mt][p], b, t0, 0, 0, 0);
@@ -496,7 +557,25 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
                     }
                 }
             }
-            if (kk == SH::SPB - 1) {
+            if constexpr (SPG > 0) {
+                // Group done: as below, with the group's own scale.
+                if (kk == 0) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(be[hb][mt]));
+                }
+                if ((kk + 1) % SPG == 0) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float inv =
+                                __builtin_bit_cast(float, uint32_t(127 - int(int8_t(be[hb][mt] >> (8 * r)))) << 23);
+#pragma unroll
+                            for (int ct = 0; ct < 4; ++ct)
+                                acc[mt][ct][r] = __builtin_fmaf(tmp[mt][ct][r] * inv, gs[ct][kk / SPG], acc[mt][ct][r]);
+                        }
+                }
+            } else if (kk == SH::SPB - 1) {
                 const int bslot = (i / SH::SPB) & 1;
                 asm volatile("" : "+v"(bs[bslot][0]), "+v"(bs[bslot][1]), "+v"(bs[bslot][2]), "+v"(bs[bslot][3]));
                 if constexpr (BF) {
@@ -539,7 +618,8 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
             for (int p = 0; p < P; ++p) asm volatile("" : "+v"(xa[sl][mt][p]));
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
-        asm volatile("" : "+v"(bs[sl][0]), "+v"(bs[sl][1]), "+v"(bs[sl][2]), "+v"(bs[sl][3]));
+        if constexpr (SPG == 0)
+            asm volatile("" : "+v"(bs[sl][0]), "+v"(bs[sl][1]), "+v"(bs[sl][2]), "+v"(bs[sl][3]));
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             if constexpr (BF)
@@ -965,10 +1045,10 @@ int launch_decode_small(dgm_gpu* g, const DecArgs& a0, const float* X) {
 // (160 KB - DEC_LDS) / 256 = 128 groups; more keep the per-block gathers.
 constexpr int DEC_SL_MAX = (160 * 1024 - DEC_LDS) / 256;
 
-template <int BITS, int MT, int P, int D, int MW, bool SL>
+template <int BITS, int MT, int P, int D, int MW, bool SL, int SPG>
 int launch_decode_sl(dgm_gpu* g, const DecArgs& a) {
-    auto kern = decode_kernel<BITS, MT, P, D, MW, SL>;
-    const int lds = DEC_LDS + (SL ? 256 * a.groups : 0);
+    auto kern = decode_kernel<BITS, MT, P, D, MW, SL, SPG>;
+    const int lds = DEC_LDS + (SPG ? DEC_SLOTS * 2048 * (DecShape<BITS>::SPB / (SPG ? SPG : 1)) : SL ? 256 * a.groups : 0);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess)
@@ -979,10 +1059,12 @@ int launch_decode_sl(dgm_gpu* g, const DecArgs& a) {
     return DGM_OK;
 }
 
-template <int BITS, int MT, int P, int D, int MW = 1>
+template <int BITS, int MT, int P, int D, int MW, int SPG>
 int launch_decode(dgm_gpu* g, const DecArgs& a) {
-    return a.groups <= DEC_SL_MAX ? launch_decode_sl<BITS, MT, P, D, MW, true>(g, a)
-                                  : launch_decode_sl<BITS, MT, P, D, MW, false>(g, a);
+    if constexpr (SPG > 0) return launch_decode_sl<BITS, MT, P, D, MW, true, SPG>(g, a);
+    else
+        return a.groups <= DEC_SL_MAX ? launch_decode_sl<BITS, MT, P, D, MW, true, 0>(g, a)
+                                      : launch_decode_sl<BITS, MT, P, D, MW, false, 0>(g, a);
 }
 
 // The one-launch kernel's domain: M <= 16, the scales of 64 rows in LDS (at
@@ -1000,10 +1082,12 @@ constexpr bool DEC_ONE_GROUP = BITS == 4 && P == 1;
 template <int BITS, int P>
 constexpr int DEC_D2 = P == 2 ? 1 : 2;
 
-template <int BITS, int P>
+template <int BITS, int P, int SPG = 0>
 int decode_dispatch(dgm_gpu* g, DecArgs& a, const float* X) {
     using SH = DecShape<BITS>;
-    if (small_ok(a.M, a.K, a.groups)) return launch_decode_small<BITS, P>(g, a, X);
+    if constexpr (SPG == 0) {
+        if (small_ok(a.M, a.K, a.groups)) return launch_decode_small<BITS, P>(g, a, X);
+    }
     // Row tiles of the prepared pieces: for the two-group kernel three are
     // padded to four (zero rows), which it covers as 2 x 2.
     const int MT = (a.M <= 32 || DEC_ONE_GROUP<BITS, P>) ? (a.M + 15) / 16 : 4;
@@ -1026,14 +1110,16 @@ int decode_dispatch(dgm_gpu* g, DecArgs& a, const float* X) {
     if (ws) a.part = reinterpret_cast<float*>(ws + own);
     else {
         a.slices = 1;
-        ws = static_cast<uint8_t*>(dgm::workspace(g, xp_bytes + ex_bytes + 256));
+        // Groups inside a block have kernels without staging to go back to.
+        ws = static_cast<uint8_t*>(SPG ? dgm::workspace_if(g, xp_bytes + ex_bytes + 256)
+                                       : dgm::workspace(g, xp_bytes + ex_bytes + 256));
     }
-    if (!ws) return dgm::ws_error(g);
+    if (!ws) return SPG ? dgm::kNotFused : dgm::ws_error(g);
     _Float16* xp = reinterpret_cast<_Float16*>(ws);
     int8_t* ex = reinterpret_cast<int8_t*>(ws + xp_bytes);
     float* corr = reinterpret_cast<float*>(ws + xp_bytes);
     const unsigned jobs = unsigned(MT * nblk);
-    hipLaunchKernelGGL((decode_prep_kernel<BITS, P>), dim3((jobs + 3) / 4), dim3(256), 0, g->stream, X, xp, ex, corr,
+    hipLaunchKernelGGL((decode_prep_kernel<BITS, P, SPG>), dim3((jobs + 3) / 4), dim3(256), 0, g->stream, X, xp, ex, corr,
                        a.M, a.K, MT);
     a.XP = xp;
     a.ex = ex;
@@ -1047,14 +1133,14 @@ int decode_dispatch(dgm_gpu* g, DecArgs& a, const float* X) {
     // would be copied before it holds the data. build.py checks this.
     constexpr int SPB = SH::SPB;
     switch (MT) {
-        case 1: return launch_decode<BITS, 1, P, SPB>(g, a);
-        case 2: return launch_decode<BITS, 2, P, (SPB > 2 ? SPB / 2 : 1)>(g, a);
+        case 1: return launch_decode<BITS, 1, P, SPB, 1, SPG>(g, a);
+        case 2: return launch_decode<BITS, 2, P, (SPB > 2 ? SPB / 2 : 1), 1, SPG>(g, a);
         default: break;
     }
     if constexpr (DEC_ONE_GROUP<BITS, P>)
-        return MT == 3 ? launch_decode<BITS, 3, P, 2>(g, a) : launch_decode<BITS, 4, P, 1>(g, a);
+        return MT == 3 ? launch_decode<BITS, 3, P, 2, 1, SPG>(g, a) : launch_decode<BITS, 4, P, 1, 1, SPG>(g, a);
     else
-        return launch_decode<BITS, 2, P, DEC_D2<BITS, P>, 2>(g, a);
+        return launch_decode<BITS, 2, P, DEC_D2<BITS, P>, 2, SPG>(g, a);
 }
 
 }  // namespace
@@ -1095,6 +1181,28 @@ bool decode_ok(int bits, const void* W, const float* X, const float* S, const dg
     return aligned(W, 16) && aligned(X, 16) && aligned(S, 4);
 }
 
+// Groups inside a block: groups of 32, and int4 groups of 64, whole chunks,
+// 32-bit byte offsets, aligned buffers (16 bytes the scales too).
+// The two launches take 8 to 17 us at least, the fp32 MFMA kernels 5 us and up
+// (us, those and this, int4 in groups of 32 unless noted): K below 2048, where N x
+// K is small: 1 x 4096 x 1024 6.2 and 8.6, 16 x 16384 x 768 7.7 and 8.2, 16 x
+// 16384 x 1024 11.3 and 8.8, 64 x 16384 x 768 25.0 and 11.9 (left on the line); from
+// 2048 on 1 x 64 x 2048 11.2 and 9.6, 20 x 64 x 2048 14.5 and 12.5, but 64 rows
+// 64 x 1024 x 2048 15.2 and 16.7, 64 x 1024 x 4096 28.2 and 26.5.
+bool decode_groups_ok(int bits, const void* W, const float* X, const float* S, const dgm_GemmP* p) {
+    if (bits != 4 && bits != 8) return false;
+    if (p->M < 1 || p->M > 64 || p->K == 0 || p->N == 0) return false;
+    if (p->qGroup != 32 && !(bits == 4 && p->qGroup == 64)) return false;
+    if (p->K % (bits == 4 ? 256 : 128) != 0) return false;
+    const int64_t nk = int64_t(p->N) * p->K;
+    if (p->K >= 2048 ? p->M > 32 && nk < (int64_t(1) << 22) : nk < (int64_t(1) << 24)) return false;
+    const int64_t rowb = bits == 4 ? p->K / 2 : p->K;
+    if (int64_t(p->N) * rowb >= (int64_t(1) << 32) || int64_t(p->N) * (p->K / p->qGroup) * 4 >= (int64_t(1) << 32))
+        return false;
+    if (int64_t(p->K / 32) * 4 * 2 * 1024 >= (int64_t(1) << 32)) return false;
+    return aligned(W, 16) && aligned(X, 16) && aligned(S, 16);
+}
+
 int decode_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias, float* Y,
                const dgm_GemmP* p) {
     DecArgs a{};
@@ -1106,10 +1214,15 @@ int decode_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const fl
     a.N = int(p->N);
     a.K = int(p->K);
     a.groups = int(p->K / p->qGroup);
-    a.gshift = __builtin_ctz(p->qGroup / (bits == 4 ? 128u : 64u));
+    const uint32_t kb = bits == 4 ? 128 : 64;
+    a.gshift = p->qGroup < kb ? 0 : __builtin_ctz(p->qGroup / kb);   // groups inside a block: not used
     a.rowb = bits == 4 ? a.K / 2 : a.K;
     a.nchunk = a.rowb / 128;
     a.has_bias = p->hasBias != 0;
+    if (p->qGroup < kb) {   // both modes: the precision these shapes had without this kernel
+        if (bits == 8) return decode_dispatch<8, 2, 1>(g, a, X);
+        return p->qGroup == 32 ? decode_dispatch<4, 2, 1>(g, a, X) : decode_dispatch<4, 2, 2>(g, a, X);
+    }
     const bool exact = g->math == DGM_MATH_FP32;
     if (bits == 4) return exact ? decode_dispatch<4, 2>(g, a, X) : decode_dispatch<4, 1>(g, a, X);
     return exact ? decode_dispatch<8, 2>(g, a, X) : decode_dispatch<8, 1>(g, a, X);

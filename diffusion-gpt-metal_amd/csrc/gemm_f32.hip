@@ -1581,6 +1581,7 @@ namespace dgm {
 bool skinny_ok(int bits, const void* W, const float* X, const dgm_GemmP* p);
 bool skinny_fused_ok(dgm_gpu* g, int bits, const void* W, const float* X, const dgm_GemmP* p);
 bool decode_ok(int bits, const void* W, const float* X, const float* S, const dgm_GemmP* p);
+bool decode_groups_ok(int bits, const void* W, const float* X, const float* S, const dgm_GemmP* p);
 int decode_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias, float* Y,
                const dgm_GemmP* p);
 int skinny_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X,
@@ -1604,12 +1605,17 @@ int gemm_f32_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const 
     // rows; up to 16 rows (8 in the reduced mode) split K over workgroups on
     // the same arithmetic when the weights are large (gemm_slab.hip); more
     // rows take f16 MFMA over exact f16 activation pieces (gemm_decode.hip),
-    // or the int8-MFMA kernel outside those domains.
+    // or the int8-MFMA kernel outside those domains. Groups of 32, and int4
+    // groups of 64, take that f16 kernel too where it pays and has staging.
     if (stream_ok(g, bits, W, X, scale, p)) return stream_fwd(g, bits, W, scale, X, bias, Y, p);
     if (slab_ok(g, bits, W, X, scale, p)) return slab_fwd(g, bits, W, scale, X, bias, Y, p);
     if (skinny_fused_ok(g, bits, W, X, p)) return skinny_fwd(g, bits, W, scale, X, bias, Y, p);
     if (decode_ok(bits, W, X, scale, p)) return decode_fwd(g, bits, W, scale, X, bias, Y, p);
     if (skinny_ok(bits, W, X, p)) return skinny_fwd(g, bits, W, scale, X, bias, Y, p);
+    if (decode_groups_ok(bits, W, X, scale, p)) {
+        const int rc = decode_fwd(g, bits, W, scale, X, bias, Y, p);
+        if (rc != kNotFused) return rc;
+    }
     // Larger M in the reduced-precision mode: bf16 MFMA with W dequantized in LDS.
     if (g->math == DGM_MATH_BF16 && bf16_ok(bits, W, X, scale, p))
         return bf16_fwd(g, bits, W, scale, X, bias, Y, p);
