@@ -54,10 +54,14 @@ constexpr int kDwWaves = 16;
 // take 16 columns each for dweight += sum over rows: of 64 groups of 16 lanes,
 // group w sums rows w, w+64, ... and the 64 partial sums are added in order,
 // then added into dweight (the weight is shared by every loop). Both are bound
-// by the latency of their loads: 1024 x 512 9.3 us (10.6 with 64 columns to a
-// workgroup, 16 row groups and rows read twice). With
+// by the latency of their loads, so all loads of a row (4, 8 or 16 to a lane
+// and operand, for up to 256, 512 or 1024 columns) and of 16 rows of a group
+// are issued together: 1024 x 512 7.3 us (9.3 with a branch at each load and 8
+// rows at a time; 10.6 with 64 columns to a workgroup, 16 row groups and rows
+// read twice), same bits. With
 // `add`, dx[r, c] = add[r, c] + the row's dx (an acc_f of the result; add may
 // alias dx).
+template <int PER>   // columns a lane keeps (cols <= 64 PER), 0: none
 __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __restrict__ x,
                                                                 const float* __restrict__ rstd,
                                                                 const float* __restrict__ w,
@@ -65,7 +69,6 @@ __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __r
                                                                 const float* add, float* __restrict__ dweight,
                                                                 int rows, int cols, int ndx) {
     constexpr int GROUPS = 4 * kDwWaves;   // of 16 lanes
-    constexpr int PER = 16;                // columns a lane keeps
     __shared__ float part[GROUPS][16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (int(blockIdx.x) < ndx) {
@@ -78,15 +81,24 @@ __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __r
         const float rs = rstd[row];
         const float rs3 = rs * rs * rs;
         float pt = 0.0f;
-        if (cols <= 64 * PER) {
-            float xv[PER], dyhat[PER], av[PER];
+        if constexpr (PER > 0) {
+            // Loads past the row re-read its last element, so that all of them
+            // are issued without a branch between.
+            const float* src = ad ? ad : xr;
+            float xv[PER], dyhat[PER], av[PER], wv[PER];
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
-                const int c = lane + 64 * u;
-                const bool in = c < cols;
-                xv[u] = in ? xr[c] : 0.0f;
-                dyhat[u] = in ? gr[c] * w[c] : 0.0f;
-                av[u] = in && ad ? ad[c] : 0.0f;
+                const int c = min(lane + 64 * u, cols - 1);
+                xv[u] = xr[c];
+                dyhat[u] = gr[c];
+                wv[u] = w[c];
+                av[u] = src[c];
+            }
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const bool in = lane + 64 * u < cols;
+                xv[u] = in ? xv[u] : 0.0f;
+                dyhat[u] = in ? dyhat[u] * wv[u] : 0.0f;
             }
 #pragma unroll
             for (int u = 0; u < PER; ++u) pt += dyhat[u] * xv[u];
@@ -114,9 +126,22 @@ __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __r
     }
     const int l16 = lane & 15, group = wave * 4 + (lane >> 4);
     const int c = (int(blockIdx.x) - ndx) * 16 + l16;
+    const float before = threadIdx.x < 16 && c < cols ? dweight[c] : 0.0f;
     float acc = 0.0f;
     if (c < cols) {
         int r = group;
+        for (; r + 15 * GROUPS < rows; r += 16 * GROUPS) {
+            float d[16], y[16], q[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const int rr = r + u * GROUPS;
+                d[u] = dy[size_t(rr) * cols + c];
+                y[u] = x[size_t(rr) * cols + c];
+                q[u] = rstd[rr];
+            }
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc += d[u] * y[u] * q[u];
+        }
         for (; r + 7 * GROUPS < rows; r += 8 * GROUPS) {
             float v[8];
 #pragma unroll
@@ -135,7 +160,7 @@ __global__ __launch_bounds__(64 * kDwWaves) void rms_bwd_kernel(const float* __r
         float tot = 0.0f;
 #pragma unroll
         for (int g2 = 0; g2 < GROUPS; ++g2) tot += part[g2][l16];
-        dweight[c] += tot;
+        dweight[c] = before + tot;
     }
 }
 
@@ -1046,8 +1071,12 @@ int launch_rms_bwd(dgm_gpu* g, const float* x, const float* rstd, const float* w
                    float* dweight, int64_t rows, int64_t cols, const float* add = nullptr) {
     if (rows == 0 || cols == 0) return DGM_OK;
     const int ndx = int((rows + kDwWaves - 1) / kDwWaves), ndw = int((cols + 15) / 16);
-    hipLaunchKernelGGL(rms_bwd_kernel, dim3(unsigned(ndx + ndw)), dim3(64 * kDwWaves), 0, g->stream, x, rstd, w, dy,
-                       dx, add, dweight, int(rows), int(cols), ndx);
+    auto* const kern = cols <= 256    ? rms_bwd_kernel<4>
+                       : cols <= 512  ? rms_bwd_kernel<8>
+                       : cols <= 1024 ? rms_bwd_kernel<16>
+                                      : rms_bwd_kernel<0>;
+    hipLaunchKernelGGL(kern, dim3(unsigned(ndx + ndw)), dim3(64 * kDwWaves), 0, g->stream, x, rstd, w, dy, dx, add,
+                       dweight, int(rows), int(cols), ndx);
     return dgm::check_launch(g, "rms_bwd");
 }
 

@@ -39,6 +39,14 @@ def test_rms_bwd(gpu, orc, rows, cols):
     assert gpu.lastKernel == "rmsnorm_bwd"
 
 
+# Columns on both sides of each register row (256, 512, 1024), rows on both
+# sides of the weight gradient's batches (64 groups: 8 and 16 of their rows).
+@pytest.mark.parametrize("rows,cols", [(511, 256), (513, 257), (961, 512), (1024, 513), (1540, 511), (1025, 1024),
+                                       (960, 1025), (17, 1)])
+def test_rms_bwd_edges(gpu, orc, rows, cols):
+    test_rms_bwd(gpu, orc, rows, cols)
+
+
 # T % 8 == 0: the two-launch split kernels; T % 4 == 0 (12): the one-workgroup-
 # per-head kernel; others: the five passes.
 @pytest.mark.parametrize("B,T,H,D", [(8, 64, 4, 48), (2, 32, 2, 12), (2, 12, 3, 8), (2, 5, 3, 4), (1, 17, 2, 10)])
