@@ -547,19 +547,26 @@ int check_bthd(dgm_gpu* g, const char* name, int64_t B, int64_t T, int64_t H, in
 //   mid  = res + rms(a) * w1          (rmsnorm_fwd + add_f)
 //   out2 = rms(mid) * w2              (rmsnorm_fwd)
 //   out3 = rms(out2) * w3             (rmsnorm_fwd; when w3 != nullptr)
+// Bound by the latency of the loads: the row's, res's and the weights' are
+// issued together, before the first reduction, 4, 8 or 16 to a lane (up to
+// 256, 512 or 1024 columns; loads past the row re-read its last element).
+// 1024 x 512 4.9 us, 8.8 with a branch at each load and res and the weights
+// loaded where they are used.
 constexpr int kRowMax = 16;   // columns per lane: cols <= 1024
 
-__device__ __forceinline__ float row_rstd(const float (&v)[kRowMax], int lane, int cols, float eps) {
+template <int PER>
+__device__ __forceinline__ float row_rstd(const float (&v)[PER], int lane, int cols, float eps) {
 #pragma clang fp contract(off)
     float ss = 0.0f;
 #pragma unroll
-    for (int u = 0; u < kRowMax; ++u)
+    for (int u = 0; u < PER; ++u)
         if (lane + 64 * u < cols) ss += v[u] * v[u];
     ss = wave_sum(ss);
     const float mean = ss / float(cols);
     return 1.0f / sqrtf(mean + eps);
 }
 
+template <int PER>   // columns of a lane: cols <= 64 PER
 __global__ __launch_bounds__(kThreads) void row_fuse_kernel(const float* __restrict__ a, const float* __restrict__ res,
                                                             float* __restrict__ mid, float* __restrict__ out2,
                                                             float* __restrict__ out3, const float* __restrict__ w1,
@@ -571,35 +578,45 @@ __global__ __launch_bounds__(kThreads) void row_fuse_kernel(const float* __restr
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
     const size_t base = size_t(row) * cols;
-    float v[kRowMax];
+    const float* w3s = w3 ? w3 : w2;
+    float v[PER], rv[PER], g1[PER], g2[PER], g3[PER];
 #pragma unroll
-    for (int u = 0; u < kRowMax; ++u) v[u] = lane + 64 * u < cols ? a[base + lane + 64 * u] : 0.0f;
+    for (int u = 0; u < PER; ++u) {
+        const int c = min(lane + 64 * u, cols - 1);
+        v[u] = a[base + c];
+        rv[u] = res[base + c];
+        g1[u] = w1[c];
+        g2[u] = w2[c];
+        g3[u] = w3s[c];
+    }
+#pragma unroll
+    for (int u = 0; u < PER; ++u) v[u] = lane + 64 * u < cols ? v[u] : 0.0f;
     float rs = row_rstd(v, lane, cols, eps);
     if (lane == 0 && rstd1) rstd1[row] = rs;
 #pragma unroll
-    for (int u = 0; u < kRowMax; ++u) {
+    for (int u = 0; u < PER; ++u) {
         const int c = lane + 64 * u;
         if (c < cols) {
-            const float t1 = (v[u] * rs) * w1[c];
-            v[u] = res[base + c] + t1;
+            const float t1 = (v[u] * rs) * g1[u];
+            v[u] = rv[u] + t1;
             if (mid) mid[base + c] = v[u];
         }
     }
     rs = row_rstd(v, lane, cols, eps);
 #pragma unroll
-    for (int u = 0; u < kRowMax; ++u) {
+    for (int u = 0; u < PER; ++u) {
         const int c = lane + 64 * u;
         if (c < cols) {
-            v[u] = (v[u] * rs) * w2[c];
+            v[u] = (v[u] * rs) * g2[u];
             out2[base + c] = v[u];
         }
     }
     if (w3) {
         rs = row_rstd(v, lane, cols, eps);
 #pragma unroll
-        for (int u = 0; u < kRowMax; ++u) {
+        for (int u = 0; u < PER; ++u) {
             const int c = lane + 64 * u;
-            if (c < cols) out3[base + c] = (v[u] * rs) * w3[c];
+            if (c < cols) out3[base + c] = (v[u] * rs) * g3[u];
         }
     }
     if (lane == 0 && rstd) rstd[row] = rs;
@@ -891,8 +908,9 @@ int launch_row_fuse(dgm_gpu* g, const float* a, const float* res, float* mid, fl
                     const float* w1, const float* w2, const float* w3, float* rstd, int64_t rows, int64_t cols,
                     float eps, float* rstd1 = nullptr) {
     if (rows == 0 || cols == 0) return DGM_OK;
-    hipLaunchKernelGGL(row_fuse_kernel, dim3(unsigned((rows + 3) / 4)), dim3(kThreads), 0, g->stream, a, res, mid,
-                       out2, out3, w1, w2, w3, rstd, rstd1, int(rows), int(cols), eps);
+    auto* const kern = cols <= 256 ? row_fuse_kernel<4> : cols <= 512 ? row_fuse_kernel<8> : row_fuse_kernel<kRowMax>;
+    hipLaunchKernelGGL(kern, dim3(unsigned((rows + 3) / 4)), dim3(kThreads), 0, g->stream, a, res, mid, out2, out3, w1,
+                       w2, w3, rstd, rstd1, int(rows), int(cols), eps);
     return dgm::check_launch(g, "dit_forward row_fuse");
 }
 
