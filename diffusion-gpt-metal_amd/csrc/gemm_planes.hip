@@ -418,9 +418,10 @@ __device__ __forceinline__ void tile_at(const PlaneArgs& a, int L, int& ti, int&
     tj = within / gm;
 }
 
-// Stores one 32 x 32 tile of sums at (r0, c0). Lane l holds column l % 32,
+// Stores one 32 x 32 tile of sums at (r0, c0), but for the elements of flagged
+// rows and columns; true where there are any. Lane l holds column l % 32,
 // rows 8 (e / 4) + 4 (l / 32) + e % 4. ea: the rows' exponents from r0.
-__device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r0, int c0, const int* ea, int eb) {
+__device__ __forceinline__ bool store_tile(const PlaneArgs& a, f32x16 acc, int r0, int c0, const int* ea, int eb) {
     const int lane = threadIdx.x & 63, q = lane >> 5;
     const int M = a.M, N = a.N, ld = a.ldo, c = c0 + (lane & 31);
     float* const base = c0 < a.cols1 ? a.out : a.out2 - a.cols1;   // cols1 is a multiple of 32, or N
@@ -445,7 +446,7 @@ __device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r
         }
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[int64_t(8 * (e >> 2) + (e & 3)) * ld] = acc[e];
-        return;
+        return false;
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -455,14 +456,56 @@ __device__ __forceinline__ void store_tile(const PlaneArgs& a, f32x16 acc, int r
             *at = a.accumulate ? *at + acc[e] : acc[e];
         }
     }
-    if (!__any(odd) || c >= N) return;
-    for (int e = 0; e < 16; ++e) {   // from the operands, in fp32
+    return __any(odd);
+}
+
+__device__ __forceinline__ void load_any(const Src& s, int r, int c, float (&v)[8]) {
+    if (s.col) {
+        if (s.bits == 32) load8<32, 1>(s, r, c, v);
+        else if (s.bits == 8) load8<8, 1>(s, r, c, v);
+        else load8<4, 1>(s, r, c, v);
+    } else {
+        if (s.bits == 32) load8<32, 0>(s, r, c, v);
+        else if (s.bits == 8) load8<8, 0>(s, r, c, v);
+        else load8<4, 0>(s, r, c, v);
+    }
+}
+
+// The flagged elements of one 32 x 32 tile, from the operands in fp32
+// (v_mfma_f32_32x32x2_f32, a lane 8 consecutive c of its row and column). One
+// token of NaN gradients flags every row of dW, so this has to run at about the
+// rate of the fp32 MFMA kernels: dX + dW of 2048 x 2048 x 2048 with such a token
+// 859 us, those kernels 659, a chain of scalar fmas per element 42810.
+__device__ __forceinline__ void exact_tile(const PlaneArgs& a, int r0, int c0, const int* ea, int eb) {
+    const int lane = threadIdx.x & 63, q = lane >> 5;
+    f32x16 acc = {};
+    for (int k = 0; k < a.sa.C; k += 32) {
+        float x[2][8], y[2][8];
+        // Kept opaque: the addresses of every form that load_any has would
+        // otherwise be computed before the loop, in registers that the
+        // kernel's other waves then go without.
+        int rx = r0 + (lane & 31), ry = c0 + (lane & 31);
+        asm volatile("" : "+v"(rx), "+v"(ry));
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            load_any(a.sa, rx, k + 16 * u + 8 * q, x[u]);
+            load_any(a.sb, ry, k + 16 * u + 8 * q, y[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u][j], y[u][j], acc, 0, 0, 0);
+    }
+    const int c = c0 + (lane & 31);
+    if (c >= a.N) return;
+    float* const o = (c0 < a.cols1 ? a.out : a.out2 - a.cols1) + c;
+    const float bv = a.bias ? a.bias[c] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
         const int lr = 8 * (e >> 2) + 4 * q + (e & 3), r = r0 + lr;
-        if (r >= M || (ea[lr] != kFlag && eb != kFlag)) continue;
-        float v = 0.0f;
-        for (int k = 0; k < a.sa.C; ++k) v = __builtin_fmaf(elem(a.sa, r, k), elem(a.sb, c, k), v);
-        v += bv;
-        float* at = base + int64_t(r) * ld + c;
+        if (r >= a.M || (ea[lr] != kFlag && eb != kFlag)) continue;
+        float* at = o + int64_t(r) * a.ldo;
+        const float v = acc[e] + bv;
         *at = a.accumulate ? *at + v : v;
     }
 }
@@ -656,6 +699,7 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g)
     // No direct-to-LDS load may outlive the workgroup's LDS.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
+    uint32_t odd = 0;   // tiles with flagged elements
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -663,7 +707,8 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g)
             if constexpr (!CODE) acc[i][j] += low[i][j];
             if (whole) {
                 const int lr = (wm * MT + i) * 32, lc = (wn * NT + j) * 32;
-                store_tile(a, acc[i][j], m0 + lr, n0 + lc, exps + lr, exps[T::TM + lc + (lane & 31)]);
+                if (store_tile(a, acc[i][j], m0 + lr, n0 + lc, exps + lr, exps[T::TM + lc + (lane & 31)]))
+                    odd |= 1u << (i * NT + j);
             } else {
                 f32x4* o = reinterpret_cast<f32x4*>(a.part) +
                            ((int64_t(L - a.full) * a.splits + part) * T::WAVES + wave) * (MT * NT * 4 * 64) +
@@ -674,11 +719,15 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g)
                                       acc[i][j][4 * e + 3]};
             }
         }
+    for (; odd; odd &= odd - 1) {
+        const int k = __builtin_ctz(odd), lr = (wm * MT + k / NT) * 32, lc = (wn * NT + k % NT) * 32;
+        exact_tile(a, m0 + lr, n0 + lc, exps + lr, exps[T::TM + lc + (lane & 31)]);
+    }
 }
 
 // The parts of the split tiles, added in order: one wave per 32 x 32 tile.
 template <typename T>
-__global__ __launch_bounds__(256) void part_sum_kernel(PlaneGroup g) {
+__global__ __launch_bounds__(256, 7) void part_sum_kernel(PlaneGroup g) {
     constexpr int SUB = T::MT * T::NT;
     const bool second = int(blockIdx.x) >= g.first;
     const PlaneArgs& a = args_of(second);
@@ -701,7 +750,8 @@ __global__ __launch_bounds__(256) void part_sum_kernel(PlaneGroup g) {
             for (int k = 0; k < 4; ++k) acc[4 * e + k] = p == 0 ? v[k] : acc[4 * e + k] + v[k];
         }
     }
-    store_tile(a, acc, r0, c0, a.ea + r0, a.eb[c0 + (lane & 31)]);
+    const int eb = a.eb[c0 + (lane & 31)];
+    if (store_tile(a, acc, r0, c0, a.ea + r0, eb)) exact_tile(a, r0, c0, a.ea + r0, eb);
 }
 
 template <typename T>

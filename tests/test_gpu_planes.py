@@ -121,7 +121,7 @@ def test_unaligned_buffers(gpu, bits, M, N, K, G):
         assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
-@pytest.mark.parametrize("kind", ["nonfinite", "rows", "tiny", "zeros"])
+@pytest.mark.parametrize("kind", ["nonfinite", "token", "rows", "tiny", "zeros"])
 def test_values(gpu, kind):
     """Infinities and NaN land where the products of the operands put them;
     rows of very different size each keep their own precision."""
@@ -131,6 +131,8 @@ def test_values(gpu, kind):
     if kind == "nonfinite":
         x[3, 5], x[7, 9], x[11, 2], dy[4, 6], dy[1029, 999] = float("inf"), -float("inf"), float("nan"), float("inf"), \
             float("nan")
+    elif kind == "token":      # a token whose gradients overflowed: every row of dW
+        dy[517], x[13] = float("nan"), float("inf")
     elif kind == "rows":
         x *= torch.exp2(torch.randint(-60, 60, (M, 1), device="cuda").float())
         dy *= torch.exp2(torch.randint(-30, 30, (1, N), device="cuda").float())
@@ -149,7 +151,7 @@ def test_values(gpu, kind):
     for got, a, b, n in ((y, xd, wd, K), (dx, dyd, wd.T.contiguous(), N),
                          (dw, dyd.T.contiguous(), xd.T.contiguous(), M)):
         ref = a @ b.T
-        if kind == "nonfinite":
+        if kind in ("nonfinite", "token"):
             assert torch.equal(torch.isnan(got), torch.isnan(ref))
             inf = torch.isinf(ref)
             assert torch.equal(torch.isinf(got), inf) and torch.equal(got[inf].double(), ref[inf])
@@ -225,3 +227,44 @@ def test_buffer_capture_and_streams(dgm, gpu, torch_cuda):
     finally:
         torch.cuda.synchronize()
         g.close()
+
+
+def test_time_of_nonfinite(dgm, torch_cuda):
+    """A token of NaN gradients flags every row of dW and one of dX. The call
+    then takes what the fp32 MFMA kernels take for all of it (a context whose
+    reserve leaves no room for the pieces runs those), not a multiple: less
+    than three times that."""
+    torch = torch_cuda
+    M, N, K, G = 2048, 2048, 2048, 32
+    st = torch.cuda.Stream()
+    a, b = dgm.GPU(stream=st), dgm.GPU(stream=st)
+    try:
+        x, dy, w, q, s, _, _ = _inputs(a, 8, M, N, K, G, 21)
+        dx, dw = torch.empty(M, K, device="cuda"), torch.empty(N, K, device="cuda")
+        dy[100] = float("nan")
+        b.reserve(1 << 20)
+        torch.cuda.synchronize()
+
+        def us(g):
+            times = []
+            for _ in range(4):
+                e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+                g.begin()
+                e[0].record(st)
+                g.gemmBwd(8, w, q, s, dy, x, dx, dw, M, N, K, G)
+                e[1].record(st)
+                g.end()
+                times.append(e[0].elapsed_time(e[1]) * 1e3)
+            return min(times[1:])
+        fp32 = us(b)
+        assert torch.isnan(dw).all()
+        dw.zero_()
+        torch.cuda.synchronize()
+        pieces = us(a)
+        assert torch.isnan(dw).all() and int(torch.isnan(dx).sum()) == K
+        print(f"fp32 kernels {fp32:.0f} us, pieces with a NaN token {pieces:.0f} us")
+        assert pieces < 3 * fp32
+    finally:
+        torch.cuda.synchronize()
+        a.close()
+        b.close()
