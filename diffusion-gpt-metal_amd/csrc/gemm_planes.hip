@@ -7,11 +7,21 @@
 // element (row, c) of an operand lies differs (struct Src).
 //
 // Every operand row is scaled by a power of two that brings its largest
-// element into [2^14, 2^15), and split into two f16 pieces x = h + l with
-// h = f16(x), l = f16(x - h): 22 bits and a sign, an error of at most
-// 2^-24 |x| for elements down to 2^-15 of the row's largest (below that 2^-40
-// of the largest). The product is hh + hl + lh on v_mfma_f32_32x32x16_f16 with
-// fp32 accumulation; the omitted ll is below 2^-24 of the product. Products of
+// element into [2^14, 2^15), and split into two f16 pieces x = h + 2^-12 l with
+// h = f16(x), l = f16(2^12 (x - h)): 22 bits and a sign, an error of at most
+// 2^-23 |x| for elements down to 2^-27 of the row's largest, 2^-20 |x| down to
+// 2^-31, and 2^-51 of the largest below that (l unscaled: 2^-39 of the largest below
+// 2^-15). Rows of which more than one nonzero element in 16 lies below 2^-31 of
+// the largest are flagged: their outputs are computed from the original
+// operands in fp32. So a row keeps fp32's error where one huge element meets
+// zeros, or where the factors of the other operand grow as the row's elements
+// fall. What is left out: a row with few such elements against one that is zero
+// at nearly all others; its sum, below 2^-31 of what the row can give, then has
+// their error. (Every such element counted, the products of three
+// normal values that a SwiGLU backward returns would flag a row in most calls, at
+// 130 us each.)
+// The product is hh + hl + lh on v_mfma_f32_32x32x16_f16 with
+// fp32 accumulation; the omitted ll is below 2^-22 of the product. Products of
 // f16 pieces are exact, and the matrix unit rounds its sum once per 8 of them
 // (measured: 4.0e-7 in the 2-norm over 4096 random products, the figure of a
 // CPU chain rounded every 8), so hh, summed by itself, has half the roundings
@@ -24,8 +34,9 @@
 // summed per group, and the sum goes to the accumulator times the group's
 // scale. Two products instead of three, and no rounding of code * scale: 1.4e-7
 // for the first case above.
-// Rows with an infinity or NaN are computed from the original operands in
-// fp32 (an infinity times a low piece of the other sign would be NaN).
+// There l stays against the codes times 2^-12 (exact in f16).
+// Rows with an infinity or NaN are flagged too (an infinity times a low piece
+// of the other sign would be NaN).
 //
 // What it gains: v_mfma_f32_16x16x4_f32 peaks at 157 TFLOP/s and its kernels
 // here ran at 50-57; three f16 products per fp32 product at 2.5 PFLOP/s peak at
@@ -65,7 +76,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kFlag = 1 << 30;      // exps[]: the row holds an infinity or NaN
+constexpr int kFlag = 1 << 30;      // an exponent: the row's elements do not fit the pieces
+constexpr float kLow = 1.0f / 4096.0f;   // of l
 constexpr int kMaxParts = 16;       // row chunks of a column-maximum pass
 
 // One operand: element (r, c) of R x C.
@@ -83,9 +95,10 @@ struct Src {
 struct Operand {
     Src s;
     uint8_t* planes;
-    uint32_t* part;       // largest |element| (its bits) of each row: parts x width
+    uint32_t* part;       // largest |element| (its bits) of each row: parts x width; then how many are not zero
     int parts, width;
-    int* exps;            // row scale 2^e, or kFlag
+    int* exps;            // row scale 2^e, or kFlag; then (each [32 rb]) the row's elements below
+                          // 2^-31 of its largest but not zero, and how many it may have
     int rb, kb;           // 32-row blocks and 16-c blocks written (padded)
     float* scales;        // codes kept as one plane: their scales 2^e, [group][32 rb]
     int gpad;             // groups written there (padded)
@@ -105,7 +118,7 @@ __device__ __forceinline__ float elem(const Src& s, int r, int c) {
     return code_at(s.p, s.bits, i) * s.scale[si];
 }
 
-// ---- launch 1: largest |element| of each row ---------------------------------------
+// ---- launch 1: largest |element| of each row, and its nonzero ones ----------------
 // One pass over fp32 data (X, dY, W, or the scales that bound the codes'
 // weights). Rows stored contiguously: lpr lanes per row. Rows stored across:
 // a block takes 64 of them and one of `parts` chunks of c.
@@ -113,15 +126,19 @@ struct MaxArg {
     const float* p;
     int64_t ld;
     int R, C, col, lpr, parts, blocks;
-    uint32_t* out;
+    uint32_t* out;   // [parts][R] largest; then nonzero
+    int* far;        // cleared for the split: `rows` of them
+    int rows;
 };
 
 __device__ __forceinline__ void max_part(const MaxArg& a, int block) {
     const int t = threadIdx.x;
+    uint32_t* const nonzero = a.out + int64_t(a.parts) * a.R;
+    for (int i = block * 256 + t; i < a.rows; i += a.blocks * 256) a.far[i] = 0;
     if (!a.col) {
         const int per = 256 / a.lpr;
         const int r = block * per + t / a.lpr, l = t % a.lpr;
-        uint32_t m = 0;
+        uint32_t m = 0, n = 0;
         if (r < a.R) {
             const float* row = a.p + int64_t(r) * a.ld;
             const bool vec = (a.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(a.p) & 15) == 0;
@@ -132,29 +149,47 @@ __device__ __forceinline__ void max_part(const MaxArg& a, int block) {
                 for (int i = l; i < n4; i += a.lpr) {
                     const u32x4 v = reinterpret_cast<const u32x4*>(row)[i] & 0x7fffffffu;
                     m = max(max(m, max(v[0], v[1])), max(v[2], v[3]));
+                    n += min(v[0], 1u) + min(v[1], 1u) + min(v[2], 1u) + min(v[3], 1u);
                 }
                 c = n4 << 2;
             }
-            for (int i = c + l; i < a.C; i += a.lpr) m = max(m, __float_as_uint(row[i]) & 0x7fffffffu);
+            for (int i = c + l; i < a.C; i += a.lpr) {
+                const uint32_t v = __float_as_uint(row[i]) & 0x7fffffffu;
+                m = max(m, v);
+                n += min(v, 1u);
+            }
         }
-        for (int off = a.lpr >> 1; off >= 1; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off)));
-        if (r < a.R && l == 0) a.out[r] = m;
+        for (int off = a.lpr >> 1; off >= 1; off >>= 1) {
+            m = max(m, uint32_t(__shfl_xor(int(m), off)));
+            n += uint32_t(__shfl_xor(int(n), off));
+        }
+        if (r < a.R && l == 0) {
+            a.out[r] = m;
+            nonzero[r] = n;
+        }
         return;
     }
-    __shared__ uint32_t sh[4][64];
+    __shared__ uint32_t sh[2][4][64];
     const int nb = (a.R + 63) / 64;
     const int r = (block % nb) * 64 + (t & 63), part = block / nb;
     const int64_t chunk = (int64_t(a.C) + a.parts - 1) / a.parts;
     const int64_t c1 = min(int64_t(a.C), (part + 1) * chunk);
-    uint32_t m = 0;
+    uint32_t m = 0, n = 0;
     if (r < a.R) {
 #pragma unroll 8
-        for (int64_t c = part * chunk + (t >> 6); c < c1; c += 4)
-            m = max(m, __float_as_uint(a.p[c * a.ld + r]) & 0x7fffffffu);
+        for (int64_t c = part * chunk + (t >> 6); c < c1; c += 4) {
+            const uint32_t v = __float_as_uint(a.p[c * a.ld + r]) & 0x7fffffffu;
+            m = max(m, v);
+            n += min(v, 1u);
+        }
     }
-    sh[t >> 6][t & 63] = m;
+    sh[0][t >> 6][t & 63] = m;
+    sh[1][t >> 6][t & 63] = n;
     __syncthreads();
-    if (t < 64 && r < a.R) a.out[int64_t(part) * a.R + r] = max(max(sh[0][t], sh[1][t]), max(sh[2][t], sh[3][t]));
+    if (t < 64 && r < a.R) {
+        a.out[int64_t(part) * a.R + r] = max(max(sh[0][0][t], sh[0][1][t]), max(sh[0][2][t], sh[0][3][t]));
+        nonzero[int64_t(part) * a.R + r] = sh[1][0][t] + sh[1][1][t] + sh[1][2][t] + sh[1][3][t];
+    }
 }
 
 // The operands of up to two products.
@@ -275,7 +310,10 @@ __device__ __forceinline__ void codes_part(const Operand& o, int block) {
     }
     if (chunk != 0) return;
     const int e = row_exp(r < o.s.R ? o.part[r] : 0u, BITS == 8 ? 7 : 3);
-    if (wave == 0 && h == 0) o.exps[r] = e;
+    if (wave == 0 && h == 0) {
+        o.exps[r] = e;
+        o.exps[2 * 32 * o.rb + r] = INT32_MAX;   // codes are exact
+    }
     const float f = exp_factor(e);
     for (int g = threadIdx.x >> 5; g < o.gpad; g += 8)
         o.scales[int64_t(g) * (o.rb * 32) + r] =
@@ -305,23 +343,44 @@ __device__ __forceinline__ void split_part(const Operand& o, int block) {
         }
     }
     const int e = row_exp(m, BITS == 32 ? 0 : (BITS == 8 ? 7 : 3));
-    if (chunk == 0 && wave == 0 && h == 0) o.exps[r] = e;
+    if (chunk == 0 && wave == 0 && h == 0) {
+        // How many elements may lie far below the largest (rows past the end:
+        // any). Of codes every one counts as not zero.
+        int limit = INT32_MAX;
+        if (r < o.s.R) {
+            limit = BITS == 32 ? 0 : o.s.C;
+            if constexpr (BITS == 32)
+                for (int i = 0; i < o.parts; ++i) limit += int(o.part[int64_t(o.parts + i) * o.width + r]);
+            limit /= 16;
+        }
+        o.exps[r] = e;
+        o.exps[2 * 32 * o.rb + r] = limit;
+    }
     const float f = exp_factor(e);
+    int far = 0;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int kb = chunk * 16 + u * 4 + wave;
         if (kb >= o.kb) continue;
         f16x8 hi, lo;
+        uint32_t least = ~0u;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const float x = v[u][j] * f;
+            least = min(least, (__float_as_uint(x) << 1) - 1);   // a zero gives the largest
             hi[j] = _Float16(x);
-            lo[j] = _Float16(x - float(hi[j]));
+            lo[j] = _Float16((x - float(hi[j])) * (1.0f / kLow));
         }
         uint8_t* out = o.planes + (int64_t(rb) * o.kb + kb) * 2048 + lane * 16;
         *reinterpret_cast<f16x8*>(out) = hi;
         *reinterpret_cast<f16x8*>(out + 1024) = lo;
+        if (least < 2 * 0x37000000u - 1) {   // below 2^-17
+#pragma unroll
+            for (int j = 0; j < 8; ++j) far += v[u][j] != 0.0f && fabsf(v[u][j] * f) < 0x1p-17f;
+        }
     }
+    // From e = 114 on, fp32's own last bit (2^-149) is a multiple of l's (2^-36).
+    if (far && e < 114) atomicAdd(o.exps + 32 * o.rb + r, far);
 }
 
 __device__ __forceinline__ void split_any(const Operand& o, int block) {
@@ -353,8 +412,9 @@ __global__ __launch_bounds__(256) void split_kernel(Operands a) {
 // ---- launch 3: the GEMM ----------------------------------------------------------------
 struct PlaneArgs {
     const uint8_t *A, *B;
-    const int *ea, *eb;
-    Src sa, sb;           // the original operands, for rows with an infinity or NaN
+    const int *ea, *eb;   // as Operand::exps, of rows_a and rows_b rows
+    int rows_a, rows_b;
+    Src sa, sb;           // the original operands, for flagged rows
     const float* bias;
     float *out, *out2;    // columns from cols1 on go to out2; rows of ldo floats
     int ldo, cols1;
@@ -395,6 +455,11 @@ __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
                                                   0);
 }
 
+// Codes times kLow.
+__device__ __forceinline__ u32x4 lowered(u32x4 b) {
+    return __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, b) * _Float16(kLow));
+}
+
 // Up to two products in one launch: the workgroups of the first, then those
 // of the second, which fill what the first leaves idle.
 struct PlaneGroup {
@@ -406,6 +471,11 @@ struct PlaneGroup {
 // chosen one would keep 50 more scalar registers than there are).
 __device__ __forceinline__ const PlaneArgs& args_of(bool second) {
     return ((const PlaneArgs*)__builtin_amdgcn_kernarg_segment_ptr())[second ? 1 : 0];
+}
+
+// The exponent of row r, or kFlag.
+__device__ __forceinline__ int row_scale(const int* exps, int rows, int r) {
+    return exps[rows + r] > exps[2 * rows + r] ? kFlag : exps[r];
 }
 
 // Tile L of the order: groups of GROUP_M tile rows, column after column, so
@@ -544,7 +614,7 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g)
     const int m0 = ti * T::TM, n0 = tj * T::TN;
 
     for (int i = t; i < T::TM + T::TN; i += 64 * T::WAVES)
-        exps[i] = i < T::TM ? a.ea[m0 + i] : a.eb[n0 + i - T::TM];
+        exps[i] = i < T::TM ? row_scale(a.ea, a.rows_a, m0 + i) : row_scale(a.eb, a.rows_b, n0 + i - T::TM);
 
     // This wave's loads of a stage: units wave * UPW ..; first A's (AU to a
     // 32-row block), then B's. A stage further is AU or BU KB further.
@@ -599,7 +669,8 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g)
                     st + (T::TM / 32 * T::AU + (wn * NT + j) * T::BU + kb + p) * 1024);
     };
     // The matrix unit rounds once per 8 products. Two planes: hh is summed
-    // apart from hl + lh, whose roundings are then 2^-11 of those of the sum.
+    // apart from hl + lh (2^12 too large), whose roundings are then 2^-11 of
+    // those of the sum.
     // CODE: `low` is the sum of the group, x as h and l against the codes, and
     // goes to acc times the group's scale.
     f32x16 acc[MT][NT], low[MT][NT];
@@ -616,7 +687,8 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g)
                 for (int i = 0; i < MT; ++i)
 #pragma unroll
                     for (int j = 0; j < NT; ++j)
-                        low[i][j] = mfma(f.a[i][p], f.b[j][0], fresh && p == 0 ? zero : low[i][j]);
+                        low[i][j] = mfma(f.a[i][p], p == 0 ? f.b[j][0] : lowered(f.b[j][0]),
+                                         fresh && p == 0 ? zero : low[i][j]);
         } else {
 #pragma unroll
             for (int i = 0; i < MT; ++i)
@@ -704,7 +776,10 @@ __global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g)
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            if constexpr (!CODE) acc[i][j] += low[i][j];
+            if constexpr (!CODE) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = __builtin_fmaf(low[i][j][e], kLow, acc[i][j][e]);
+            }
             if (whole) {
                 const int lr = (wm * MT + i) * 32, lc = (wn * NT + j) * 32;
                 if (store_tile(a, acc[i][j], m0 + lr, n0 + lc, exps + lr, exps[T::TM + lc + (lane & 31)]))
@@ -739,6 +814,8 @@ __global__ __launch_bounds__(256, 7) void part_sum_kernel(PlaneGroup g) {
     const int r0 = ti * T::TM + (wave / T::WN * T::MT + sub / T::NT) * 32;
     const int c0 = tj * T::TN + (wave % T::WN * T::NT + sub % T::NT) * 32;
     if (r0 >= a.M || c0 >= a.N) return;
+    const int row_e = row_scale(a.ea, a.rows_a, r0 + (lane & 31));   // used after the sums
+    const int eb = row_scale(a.eb, a.rows_b, c0 + (lane & 31));
     f32x16 acc;
     for (int p = 0; p < a.splits; ++p) {
         const f32x4* o = reinterpret_cast<const f32x4*>(a.part) +
@@ -750,8 +827,12 @@ __global__ __launch_bounds__(256, 7) void part_sum_kernel(PlaneGroup g) {
             for (int k = 0; k < 4; ++k) acc[4 * e + k] = p == 0 ? v[k] : acc[4 * e + k] + v[k];
         }
     }
-    const int eb = a.eb[c0 + (lane & 31)];
-    if (store_tile(a, acc, r0, c0, a.ea + r0, eb)) exact_tile(a, r0, c0, a.ea + r0, eb);
+    __shared__ int exps[4][32];   // a wave's own
+    int* const ea = exps[threadIdx.x >> 6];
+    if (lane < 32) ea[lane] = row_e;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (store_tile(a, acc, r0, c0, ea, eb)) exact_tile(a, r0, c0, ea, eb);
 }
 
 template <typename T>
@@ -914,6 +995,8 @@ MaxArg max_arg(const Operand& o) {
     m.col = s.col;
     m.parts = o.parts;
     m.out = o.part;
+    m.far = o.exps + 32 * o.rb;
+    m.rows = s.R;
     m.R = o.width;
     m.C = codes && !s.col ? s.groups : s.C;
     m.lpr = m.C >= 512 ? 64 : m.C >= 128 ? 16 : 8;
@@ -980,8 +1063,8 @@ int run(dgm_gpu* g, const Product* q, int n, bool dry = false) {
         for (int k = 2 * i; k < 2 * i + 2; ++k) {
             const Operand& o = op.o[k];
             at[k][0] = take(int64_t(o.rb) * o.kb * 2048);
-            at[k][1] = take(int64_t(o.rb) * 128);
-            at[k][2] = take(int64_t(o.parts) * o.width * 4);
+            at[k][1] = take(int64_t(o.rb) * 3 * 128);
+            at[k][2] = take(int64_t(o.parts) * o.width * 8);
             at[k][3] = take(int64_t(o.gpad) * o.rb * 128);
         }
         parts[i] = take((tiles[i] - full[i]) * splits[i] * tile.tm * tile.tn * 4);
@@ -1009,6 +1092,8 @@ int run(dgm_gpu* g, const Product* q, int n, bool dry = false) {
         r.B = b.planes;
         r.ea = a.exps;
         r.eb = b.exps;
+        r.rows_a = a.rb * 32;
+        r.rows_b = b.rb * 32;
         r.sa = q[i].a;
         r.sb = q[i].b;
         r.bias = q[i].bias;

@@ -47,8 +47,13 @@ extern "C" {
  * over an exact split of the activations into four int8 pieces against a
  * power of two per row and k-range (2^-27 of its maximum); other forwards up
  * to M = 64 on f16 MFMA over two f16 pieces per activation against a power
- * of two per (row, 128-k block) (2^-22 of each element); the rest accumulate
- * fp32 products of fp32 operands.
+ * of two per (row, 128-k block) (2^-22 of each element); large products (from
+ * about 0.6 * 2^30 on: the forward, dX and dW) take two f16 pieces of every
+ * operand element against a power of two per row of the contraction (2^-23 of
+ * each element, and 2^-22 of each product; 2^-20 of an element 2^31 below its
+ * row's largest; rows with more than a sixteenth of their nonzero elements
+ * below that, or with an infinity or NaN, run on fp32 operands); the rest
+ * accumulate fp32 products of fp32 operands.
  * BF16: the int8-piece kernels take two pieces (up to M = 8 when K is
  * split); otherwise up to M = 64, int4 codes
  * meet bf16(x) and int8 codes one f16 piece; larger M (with K % 128 == 0 and

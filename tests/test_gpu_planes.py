@@ -4,7 +4,8 @@ Sizes sit at the edges of its tiles (128 and 256 rows), stages (16 and 32 of
 the contraction) and parts (tiles cut along the contraction), on both sides of
 where each is taken. The reference is the float64 product of
 the same operands. Bound per element, against the row's and column's 2-norms
-|a| |b| (every element of a split operand is within 2^-24 of its value, and a
+|a| |b| (every element of a split operand is within 2^-23 of its value and the
+product of the low pieces within 2^-22 at worst, mostly a quarter of both, and a
 sum of n products, rounded once per 8, is within n/8 * 2^-24 of |a| |b| at
 worst): (2 + n / 8) * 2^-24 |a| |b|.
 """
@@ -163,6 +164,103 @@ def test_values(gpu, kind):
                          b.norm(dim=1)[None, :] + 2.0 ** -148).all())
         else:
             assert _within(got, ref, a, b, n)
+
+
+# 2-norm of the error over that of the result where an element far below its
+# row's largest carries the sum. It is held to 2^-20 of itself (or its row goes to
+# the fp32 kernel): 2^-19 for one such operand with the product of the low pieces,
+# 2^-18 for two, the sums' own 5e-7 within that.
+FAR_ONE, FAR_BOTH = 2.0 ** -19, 2.0 ** -18
+
+
+@pytest.mark.parametrize("bits,G", [(4, 32), (8, 8), (32, 8)])
+@pytest.mark.parametrize("ratio", [1e4, 1e6, 1e8, 1e9, 1e12, 1e30])
+def test_outlier_channel_against_zeros(gpu, bits, G, ratio):
+    """One channel of X (one output of dY) far above the others meets weights of
+    zero: the others are the whole product and keep their precision."""
+    import torch
+    M, N, K = 512, 1536, 1024
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x, dy = torch.randn(M, K, generator=g, device="cuda"), torch.randn(M, N, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda") * 0.02
+    x[:, 100] *= ratio
+    dy[:, 7] *= ratio
+    w[:, 100] = 0
+    w[7] = 0
+    q = s = None
+    wd = w.double()
+    if bits != 32:
+        q = torch.empty(N * K // (2 if bits == 4 else 1), dtype=torch.uint8, device="cuda")
+        s = torch.empty(N * (K // G), device="cuda")
+        torch.cuda.synchronize()
+        gpu.begin()
+        gpu.quantize(w, q, s, N, K, bits, G)
+        gpu.end()
+        codes = q.view(torch.int8).double() if bits == 8 else torch.stack(
+            [(q << 4).view(torch.int8) >> 4, q.view(torch.int8) >> 4], dim=1).reshape(-1).double()
+        wd = (codes.reshape(N, K // G, G) * s.double().reshape(N, K // G, 1)).reshape(N, K)
+    y, dx = torch.empty(M, N, device="cuda"), torch.empty(M, K, device="cuda")
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.gemmNT(bits, w, q, s, x, None, y, M, N, K, G)
+    gpu.gemmDX(bits, w, q, s, dy, dx, M, N, K, G)
+    gpu.end()
+    for got, ref in ((y, x.double() @ wd.T), (dx, dy.double() @ wd)):
+        err = float((got.double() - ref).norm() / ref.norm())
+        assert err <= FAR_ONE, err
+
+
+@pytest.mark.parametrize("spread", [8, 16, 24, 40, 60])
+def test_tokens_scaled_against_each_other(gpu, spread):
+    """Tokens whose X is 2^s as large and whose dY is 2^-s: every product of dW
+    matters alike, however far the elements lie below their column's largest."""
+    import torch
+    M, N, K = 1024, 1024, 1024
+    g = torch.Generator(device="cuda").manual_seed(spread)
+    x, dy = torch.randn(M, K, generator=g, device="cuda"), torch.randn(M, N, generator=g, device="cuda")
+    f = torch.exp2(torch.randint(0, spread + 1, (M, 1), generator=g, device="cuda").float())
+    x, dy = x * f, dy / f
+    dw = torch.empty(N, K, device="cuda")
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.gemmDW(dy, x, dw, M, N, K)
+    gpu.end()
+    ref = dy.double().T.contiguous() @ x.double()
+    err = float((dw.double() - ref).norm() / ref.norm())
+    assert err <= FAR_BOTH, err
+
+
+@pytest.mark.parametrize("bits,G", [(4, 32), (8, 8), (32, 8)])
+@pytest.mark.parametrize("spread", [16, 24, 60])
+def test_outputs_scaled_against_each_other(gpu, bits, G, spread):
+    """The same along the contraction of dX: rows of W 2^s as large (their
+    codes' scales, for quantized weights), outputs of dY 2^-s."""
+    import torch
+    M, N, K = 512, 1536, 1024
+    g = torch.Generator(device="cuda").manual_seed(spread)
+    f = torch.exp2(torch.randint(0, spread + 1, (N,), generator=g, device="cuda").float())
+    w = torch.randn(N, K, generator=g, device="cuda") * f[:, None]
+    dy = torch.randn(M, N, generator=g, device="cuda") / f
+    q = s = None
+    wd = w.double()
+    if bits != 32:
+        q = torch.empty(N * K // (2 if bits == 4 else 1), dtype=torch.uint8, device="cuda")
+        s = torch.empty(N * (K // G), device="cuda")
+        torch.cuda.synchronize()
+        gpu.begin()
+        gpu.quantize(w, q, s, N, K, bits, G)
+        gpu.end()
+        codes = q.view(torch.int8).double() if bits == 8 else torch.stack(
+            [(q << 4).view(torch.int8) >> 4, q.view(torch.int8) >> 4], dim=1).reshape(-1).double()
+        wd = (codes.reshape(N, K // G, G) * s.double().reshape(N, K // G, 1)).reshape(N, K)
+    dx = torch.empty(M, K, device="cuda")
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.gemmDX(bits, w, q, s, dy, dx, M, N, K, G)
+    gpu.end()
+    ref = dy.double() @ wd
+    err = float((dx.double() - ref).norm() / ref.norm())
+    assert err <= FAR_BOTH, err
 
 
 def test_buffer_capture_and_streams(dgm, gpu, torch_cuda):
