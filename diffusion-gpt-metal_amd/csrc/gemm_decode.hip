@@ -84,6 +84,8 @@ constexpr int DEC_CHUNK = DEC_COLS * 128;    // bytes of one chunk (64 rows x 12
 constexpr int DEC_KW = 4;                    // compute waves splitting K
 constexpr int DEC_LDS = DEC_SLOTS * 4 * DEC_CHUNK;   // 128 KB
 
+constexpr int kPoison = -128;                // no block's exponent (decode_prep_kernel)
+
 template <int BITS>
 struct DecShape {
     static constexpr int KB = BITS == 4 ? 128 : 64;   // k per 64-byte block of a weight row
@@ -109,6 +111,11 @@ struct DecShape {
 // consecutive k 32 kk .. of the block, lane group q eight of them, and an
 // infinity or NaN keeps its place (the first piece holds it, the second 0; the
 // exponent is the finite elements'), so that it meets the codes as in fp32.
+// The second piece is 2^12 larger (the codes meet it as code * 2^-12, exact):
+// an element is then held to 2^-20 of itself down to 2^-31 of its block's
+// largest. A block row of which more than one nonzero element in 16 lies below that
+// gets the exponent kPoison, whose factor 2^-e is an infinity: its outputs
+// leave the block sums as infinities or NaN and are computed from X.
 template <int BITS, int P, int SPG>
 __global__ __launch_bounds__(256) void decode_prep_kernel(const float* __restrict__ X, _Float16* __restrict__ XP,
                                                           int8_t* __restrict__ ex, float* __restrict__ corr, int M,
@@ -182,8 +189,28 @@ __global__ __launch_bounds__(256) void decode_prep_kernel(const float* __restric
         }
         e = min(126, max(-126, 141 - E));
     }
-    if (q == 0) ex[size_t(blk) * (16 * MT) + row] = int8_t(e);
     const float pw = __builtin_bit_cast(float, uint32_t(e + 127) << 23);   // 2^e
+    int stored = e;
+    if constexpr (SPG > 0) {
+        uint32_t least = ~0u;   // a zero gives the largest
+#pragma unroll
+        for (int i = 0; i < SH::KL; ++i) least = min(least, (__builtin_bit_cast(uint32_t, v[i] * pw) << 1) - 1);
+        int far = 0, nonzero = 0;
+        if (__any(least < 2 * 0x37000000u - 1)) {   // below 2^-17
+#pragma unroll
+            for (int i = 0; i < SH::KL; ++i) {
+                nonzero += v[i] != 0.0f;
+                far += v[i] != 0.0f && fabsf(v[i] * pw) < 0x1p-17f;
+            }
+            far += __shfl_xor(far, 16);
+            far += __shfl_xor(far, 32);
+            nonzero += __shfl_xor(nonzero, 16);
+            nonzero += __shfl_xor(nonzero, 32);
+        }
+        // From e = 114 on, fp32's own last bit is a multiple of the second piece's.
+        if (16 * far > nonzero && e < 114) stored = kPoison;
+    }
+    if (q == 0) ex[size_t(blk) * (16 * MT) + row] = int8_t(stored);
     const float nan = __builtin_nanf("");
 #pragma unroll
     for (int kk = 0; kk < SH::SPB; ++kk) {
@@ -193,7 +220,9 @@ __global__ __launch_bounds__(256) void decode_prep_kernel(const float* __restric
             const float xs = bad2 ? nan : v[frag_k<BITS>(0, kk, t)] * pw;
             const _Float16 h1 = _Float16(xs);
             h[0][t] = h1;
-            if constexpr (P == 2) h[1][t] = SPG && !__builtin_isfinite(xs) ? _Float16(0.0f) : _Float16(xs - float(h1));
+            if constexpr (P == 2)
+                h[1][t] = SPG && !__builtin_isfinite(xs) ? _Float16(0.0f)
+                                                         : _Float16((xs - float(h1)) * (SPG ? 4096.0f : 1.0f));
         }
         const int s = blk * SH::SPB + kk;
 #pragma unroll
@@ -218,6 +247,7 @@ struct DecArgs {
     const float* corr;     // offset terms [blocks][16 MT] (bf16 path)
     const float* bias;
     float* Y;
+    const float* X;        // groups inside a block: for the outputs that the pieces do not give
     int M, N, K, groups, gshift, rowb, nchunk, has_bias;
     int mtp;     // row tiles of the prepared pieces and exponents
     int mt0;     // first row tile this launch handles (its MT tiles)
@@ -246,6 +276,37 @@ struct Schedule {
 };
 
 
+// Rows m .. m + 3 (those past M repeat row M - 1) against weight row n over
+// chunks ch0 .. ch0 + nch - 1 in fp32, code * scale rounded as dequantization does.
+// Bound by the latency of the loads of X and the codes (eight 16-byte pieces at
+// a time instead of one: no faster): all rows so, 1 x 14336 x 4096 int4 in groups of
+// 32 143 us, 24 rows 265, where the fp32 MFMA kernels take 73 and 146.
+template <int BITS>
+__device__ __forceinline__ f32x4 direct_rows(const DecArgs& a, int n, int m, int ch0, int nch) {
+    constexpr int KP = 128 / BITS;   // k of 16 bytes; groups are of 32 k at least
+    f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+    const uint8_t* w = a.W + size_t(n) * a.rowb;
+    const float* s = a.S + size_t(n) * a.groups;
+    const int G = a.K / a.groups;
+    const float* x[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = a.X + size_t(min(m + r, a.M - 1)) * a.K;
+    for (int p = ch0 * 8; p < (ch0 + nch) * 8; ++p) {
+        const u32x4 q = *reinterpret_cast<const u32x4*>(w + size_t(p) * 16);
+        const float sc = s[p * KP / G];
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int j = 0; j < 32 / BITS; ++j) {
+                const float c = float(int(q[d] << (32 - BITS - BITS * j)) >> (32 - BITS)) * sc;
+                const int k = p * KP + d * (32 / BITS) + j;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[r] = __builtin_fmaf(c, x[r][k], z[r]);
+            }
+    }
+    return z;
+}
+
 // 4 MW + 1 waves: compute wave w takes chunks kw, kw + 4, ... (kw = w % 4;
 // interval t holds chunks 4t .. 4t + 3) for row tiles MT mh .. MT mh + MT - 1
 // (mh = w / 4); wave 4 MW streams the weight chunks into a ring of DEC_SLOTS
@@ -270,7 +331,9 @@ struct Schedule {
 // Against the fp32 MFMA kernels (us): 1 x 14336 x 4096 int4 in groups of 32 73.2
 // -> 15.8, 24 rows 145.8 -> 21.8, 24 x 4096 x 14336 151.9 -> 26.8; int4 in groups of
 // 64 145.2 -> 18.6 for 24 x 14336 x 4096, int8 in groups of 32 144.7 -> 25.7. The
-// conversions and the folds bound it (VALU): the same with groups of 128 17.7.
+// conversions and the folds bound it (VALU): the same with groups of 128 17.7. The
+// second piece at 2^12 costs a packed multiply per code pair: 24 rows 22.6 -> 24.4,
+// 64 rows 30.1 -> 33.6.
 template <int BITS, int MT, int P, int D, int MW, bool SL, int SPG>
 __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecArgs a) {
     using SH = DecShape<BITS>;
@@ -547,12 +610,13 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
                         codes_to_f16<8>(wc[ct][2 * kk + 1], h + 2);
                     }
                     const f16x8 b = {h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
+                    const f16x8 b2 = SPG ? b * _Float16(1.0f / 4096.0f) : b;   // of the second piece
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) {
                         f32x4 t0 = (SPG ? kk % (SPG ? SPG : 1) == 0 : kk == 0) ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : tmp[mt][ct];
 #pragma unroll
                         for (int p = 0; p < P; ++p)
-                            t0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[slot][mt][p], b, t0, 0, 0, 0);
+                            t0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[slot][mt][p], p == 0 ? b : b2, t0, 0, 0, 0);
                         tmp[mt][ct] = t0;
                     }
                 }
@@ -659,6 +723,18 @@ __global__ __launch_bounds__(64 * (DEC_KW * MW + 1), 1) void decode_kernel(DecAr
 #pragma unroll
         for (int v = 1; v < 4; ++v) y += *reinterpret_cast<const f32x4*>(red + (v * 64 + col) * RP + 4 * m4);
         if (bias) y += bv;
+        if constexpr (SPG > 0) {
+            // Poisoned rows, infinities and NaN of the operands, a block sum
+            // beyond fp32 before its scale: from X and the weights in fp32.
+            const bool odd = !(__builtin_isfinite(y[0]) && __builtin_isfinite(y[1]) && __builtin_isfinite(y[2]) &&
+                               __builtin_isfinite(y[3]));
+            if (__any(odd)) {
+                const f32x4 z = direct_rows<BITS>(a, n, 16 * a.mt0 + 4 * m4, ch0, nch);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (!__builtin_isfinite(y[r])) y[r] = z[r] + bv;
+            }
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = 4 * m4 + r;
@@ -1121,6 +1197,7 @@ int decode_dispatch(dgm_gpu* g, DecArgs& a, const float* X) {
     const unsigned jobs = unsigned(MT * nblk);
     hipLaunchKernelGGL((decode_prep_kernel<BITS, P, SPG>), dim3((jobs + 3) / 4), dim3(256), 0, g->stream, X, xp, ex, corr,
                        a.M, a.K, MT);
+    a.X = X;
     a.XP = xp;
     a.ex = ex;
     a.corr = corr;

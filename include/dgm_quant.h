@@ -47,7 +47,10 @@ extern "C" {
  * over an exact split of the activations into four int8 pieces against a
  * power of two per row and k-range (2^-27 of its maximum); other forwards up
  * to M = 64 on f16 MFMA over two f16 pieces per activation against a power
- * of two per (row, 128-k block) (2^-22 of each element); large products (from
+ * of two per (row, 128-k block) (2^-22 of each element; with groups of 32, and
+ * int4 groups of 64, also of an element 2^27 below its block's largest, 2^-20
+ * at 2^31, and a row of which more than a sixteenth of a block lies below that
+ * runs on fp32 operands); large products (from
  * about 0.6 * 2^30 on: the forward, dX and dW) take two f16 pieces of every
  * operand element against a power of two per row of the contraction (2^-23 of
  * each element, and 2^-22 of each product; 2^-20 of an element 2^31 below its

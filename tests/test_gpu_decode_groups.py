@@ -112,3 +112,51 @@ def test_values(gpu, bits, M, N, K, G):
         inf = torch.isinf(ref)
         assert torch.equal(torch.isinf(y), inf) and torch.equal(y[inf].double(), ref[inf])
         assert _within(y[3:], ref[3:], x[3:], wd, K) if M > 3 else True
+
+
+@pytest.mark.parametrize("bits,M,N,K,G", [(4, 20, 100, 2048, 32), (8, 3, 2100, 2048, 32), (4, 40, 2100, 2048, 64),
+                                          (8, 64, 1100, 4096, 32)])
+@pytest.mark.parametrize("ratio", [1e4, 1e6, 1e8, 1e9, 1e12, 1e30])
+def test_outlier_channels_against_zeros(gpu, bits, M, N, K, G, ratio):
+    """One channel of each block far above the others meets weights of zero: the
+    others are the whole product. Each is held to 2^-20 of itself, or its row is
+    computed in fp32: 2^-19 of the result's 2-norm, the sums' 5e-7 within that."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda") * 0.02
+    x[:, 7::64] *= ratio
+    w[:, 7::64] = 0
+    q = torch.empty(N * K // (2 if bits == 4 else 1), dtype=torch.uint8, device="cuda")
+    s = torch.empty(N * (K // G), device="cuda")
+    y = torch.empty(M, N, device="cuda")
+    bias = torch.randn(N, generator=g, device="cuda")
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.quantize(w, q, s, N, K, bits, G)
+    gpu.gemmNT(bits, None, q, s, x, bias, y, M, N, K, G)
+    gpu.end()
+    codes = q.view(torch.int8).double() if bits == 8 else torch.stack(
+        [(q << 4).view(torch.int8) >> 4, q.view(torch.int8) >> 4], dim=1).reshape(-1).double()
+    wd = (codes.reshape(N, K // G, G) * s.double().reshape(N, K // G, 1)).reshape(N, K)
+    ref = x.double() @ wd.T + bias.double()
+    err = float((y.double() - ref).norm() / ref.norm())
+    assert err <= 2.0 ** -19, err
+
+
+@pytest.mark.parametrize("bits,G", [(4, 32), (4, 64), (8, 32)])
+def test_sums_of_codes_beyond_fp32(gpu, bits, G):
+    """A sum of codes * x over a group may pass fp32's largest number where the
+    scale brings the result back: the result is finite."""
+    import torch
+    M, N, K = 18, 200, 2048
+    x, bias, q, s, wd = _operands(gpu, bits, M, N, K, G, 8)
+    x[:9] *= 1e35
+    y = torch.empty(M, N, device="cuda")
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.gemmNT(bits, None, q, s, x, bias, y, M, N, K, G)
+    gpu.end()
+    ref = x.double() @ wd.T + bias.double()
+    assert float(ref.abs().max()) < 3.4e38 and torch.isfinite(y).all()
+    assert _within(y, ref, x, wd, K)
