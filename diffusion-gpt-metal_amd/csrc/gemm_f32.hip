@@ -1720,6 +1720,11 @@ int gemm_f32_bwd_pair(dgm_gpu* g, int bits, const void* W, const float* scale, c
         const int rc = planes_bwd(g, bits, W, scale, dY, X, dX, dW, p, accumulate);
         *fused = rc != kNotFused;
         if (*fused) return rc;
+        // No room for the pieces of both products: where there is for those of
+        // one, that call alone takes them, so the two calls it is.
+        if (planes_bwd(g, bits, nullptr, nullptr, nullptr, nullptr, dX, nullptr, p, false) == DGM_OK ||
+            planes_bwd(g, 32, nullptr, nullptr, nullptr, nullptr, nullptr, dW, p, accumulate) == DGM_OK)
+            return DGM_OK;
     }
     GemmArgs ax{};
     ax.A = dY; ax.B = W; ax.scale = scale; ax.out = dX;

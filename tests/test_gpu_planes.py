@@ -327,6 +327,28 @@ def test_buffer_capture_and_streams(dgm, gpu, torch_cuda):
         g.close()
 
 
+@pytest.mark.parametrize("mib", [1, 5, 8, 20, 24, 64])
+@pytest.mark.parametrize("bits,M,N,K,G", [(8, 2048, 256, 2048, 32), (4, 1024, 1024, 1024, 32), (32, 2048, 384, 1024, 8)])
+def test_pair_under_a_reserve(dgm, torch_cuda, mib, bits, M, N, K, G):
+    """gemmBwd is bitwise the two calls also where the reserve holds the pieces
+    of neither product, of one, of each but not of both, or of both."""
+    torch = torch_cuda
+    c = dgm.GPU(stream=torch.cuda.current_stream())
+    try:
+        x, dy, w, q, s, _, _ = _inputs(c, bits, M, N, K, G, 4)
+        c.reserve(mib << 20)
+        outs = [[torch.zeros(sh, device="cuda") for sh in ((M, K), (N, K))] for _ in range(2)]
+        torch.cuda.synchronize()
+        c.begin()
+        c.gemmDX(bits, w, q, s, dy, outs[0][0], M, N, K, G)
+        c.gemmDW(dy, x, outs[0][1], M, N, K)
+        c.gemmBwd(bits, w, q, s, dy, x, *outs[1], M, N, K, G)
+        c.end()
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    finally:
+        c.close()
+
+
 def test_time_of_nonfinite(dgm, torch_cuda):
     """A token of NaN gradients flags every row of dW and one of dX. The call
     then takes what the fp32 MFMA kernels take for all of it (a context whose
