@@ -86,6 +86,11 @@ int ws_error(dgm_gpu* g);
 // dgm_gemmNT_noalloc, when dgm_gpu_reserve fixed a smaller one, or when the
 // memory is not there: the caller then takes the kernels that need no planes.
 uint8_t* planes_buffer(dgm_gpu* g, size_t bytes);
+// Makes that buffer hold `bytes` (more than it does), whatever was reserved;
+// false, recording nothing, without the memory.
+bool grow_planes(dgm_gpu* g, size_t bytes);
+// Whether the stream is capturing a graph (or cannot be asked).
+bool capturing(hipStream_t s);
 // After a synchronize: records an error on g if a decode kernel gave up a
 // bounded in-workgroup wait since the last check (gemm_decode.hip), and
 // clears the device's flag.

@@ -135,28 +135,33 @@ void* workspace_if(dgm_gpu* g, size_t bytes) {
     return p;
 }
 
-uint8_t* planes_buffer(dgm_gpu* g, size_t bytes) {
-    if (g->use_scratch) return nullptr;
+bool capturing(hipStream_t s) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(g->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+    const bool none = hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    if (!none) (void)hipGetLastError();
+    return !none;
+}
+
+bool grow_planes(dgm_gpu* g, size_t bytes) {
+    if (g->n_planes_retired == dgm_gpu::kMaxRetired) return false;
+    void* p = nullptr;
+    const size_t want = std::max(bytes, std::min(2 * g->planes_bytes, bytes + (size_t(256) << 20)));
+    if (hipMalloc(&p, want) != hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
+        return false;
     }
-    if (bytes > g->planes_bytes) {
-        if (g->reserved || g->n_planes_retired == dgm_gpu::kMaxRetired) return nullptr;
-        void* p = nullptr;
-        const size_t want = std::max(bytes, std::min(2 * g->planes_bytes, bytes + (size_t(256) << 20)));
-        if (hipMalloc(&p, want) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        if (g->planes) g->planes_retired[g->n_planes_retired++] = g->planes;
-        g->planes = p;
-        g->planes_bytes = want;
-        g->planes_stream = nullptr;   // nothing has used this one
-    }
+    if (g->planes) g->planes_retired[g->n_planes_retired++] = g->planes;
+    g->planes = p;
+    g->planes_bytes = want;
+    g->planes_stream = nullptr;   // nothing has used this one
+    return true;
+}
+
+uint8_t* planes_buffer(dgm_gpu* g, size_t bytes) {
+    if (g->use_scratch || capturing(g->stream)) return nullptr;
+    if (bytes > g->planes_bytes && (g->reserved || !grow_planes(g, bytes))) return nullptr;
     if (g->planes_stream && g->planes_stream != g->stream) {
-        if (hipStreamIsCapturing(g->planes_stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
+        if (capturing(g->planes_stream) ||
             (!g->planes_event && hipEventCreateWithFlags(&g->planes_event, hipEventDisableTiming) != hipSuccess) ||
             hipEventRecord(g->planes_event, g->planes_stream) != hipSuccess ||
             hipStreamWaitEvent(g->stream, g->planes_event, 0) != hipSuccess) {

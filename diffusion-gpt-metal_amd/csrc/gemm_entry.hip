@@ -156,11 +156,16 @@ int64_t dgm_gemmNT_workspace_bound(int64_t M, int64_t N, int64_t K) {
 
 int dgm_gpu_reserve(dgm_gpu* g, int64_t bytes) {
     if (!g || bytes < 0) return DGM_ERR_ARG;
+    if (bytes == 0) return DGM_OK;   // asks for nothing, and fixes nothing
     if (size_t(bytes) > g->ws_bytes && !dgm::workspace(g, size_t(bytes))) return dgm::ws_error(g);
     // The plane buffer too, which from now on grows here only: a call that
     // finds it too small runs without it.
-    g->reserved = false;
-    if (size_t(bytes) > g->planes_bytes) (void)dgm::planes_buffer(g, size_t(bytes));
+    if (size_t(bytes) > g->planes_bytes) {
+        if (dgm::capturing(g->stream))
+            return dgm::fail(g, DGM_ERR_UNSUPPORTED, "reserve of %lld bytes during graph capture", (long long)bytes);
+        if (!dgm::grow_planes(g, size_t(bytes)))
+            return dgm::fail(g, DGM_ERR_HIP, "reserve of %lld bytes for operand pieces failed", (long long)bytes);
+    }
     g->reserved = true;
     return DGM_OK;
 }

@@ -212,3 +212,38 @@ def test_reserve_is_monotone_and_refused_under_capture(dgm, torch_cuda):
         assert err.value.code == dgm.DGM_ERR_ARG
     finally:
         g.close()
+
+
+def test_reserve_reports_what_it_cannot_do(dgm, gpu, torch_cuda):
+    """Under graph capture a reserve that either buffer would have to grow for is
+    refused, also where the workspace alone holds it; a refused one, and one
+    of nothing, leave the context as it was: large products still take f16
+    pieces, with the bits of a fresh context."""
+    torch = torch_cuda
+    M, N, K, G = 512, 1536, 1024, 32
+    x, q, s = _case(gpu, M, N, K, G, 4, 12)
+    st = torch.cuda.Stream()
+    contexts = [dgm.GPU(stream=st) for _ in range(4)]
+    fresh, zero, refused, small = contexts
+    try:
+        torch.cuda.synchronize()
+        want = _forward(fresh, dgm, "fp32", 4, q, s, x, M, N, K, G)
+        zero.reserve(0)
+        assert np.array_equal(want, _forward(zero, dgm, "fp32", 4, q, s, x, M, N, K, G))
+        _forward(refused, dgm, "bf16", 4, q, s, x, M, N, K, G)      # the workspace holds X in bf16, 1 MiB
+        t = torch.zeros(16, device="cuda")
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            t.add_(1.0)
+            with pytest.raises(dgm.DgmError) as err:
+                refused.reserve(1 << 20)
+            assert err.value.code == dgm.DGM_ERR_UNSUPPORTED
+        del graph
+        assert np.array_equal(want, _forward(refused, dgm, "fp32", 4, q, s, x, M, N, K, G))
+        small.reserve(1 << 20)                                      # too small for the pieces: other kernels
+        assert not np.array_equal(want, _forward(small, dgm, "fp32", 4, q, s, x, M, N, K, G))
+    finally:
+        torch.cuda.synchronize()
+        for c in contexts:
+            c.close()
