@@ -144,9 +144,16 @@ bool capturing(hipStream_t s) {
 
 bool grow_planes(dgm_gpu* g, size_t bytes) {
     if (g->n_planes_retired == dgm_gpu::kMaxRetired) return false;
+    // At least double, so that the retired buffers (queued work may use them)
+    // total less than the live one; what is asked for where that much is not to be had.
+    size_t want = std::max(bytes, 2 * g->planes_bytes);
     void* p = nullptr;
-    const size_t want = std::max(bytes, std::min(2 * g->planes_bytes, bytes + (size_t(256) << 20)));
-    if (hipMalloc(&p, want) != hipSuccess) {
+    hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess && want > bytes) {
+        want = bytes;
+        e = hipMalloc(&p, want);
+    }
+    if (e != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }

@@ -349,6 +349,28 @@ def test_pair_under_a_reserve(dgm, torch_cuda, mib, bits, M, N, K, G):
         c.close()
 
 
+def test_buffer_doubles(dgm, torch_cuda):
+    """The buffer of the pieces at least doubles when it grows, as the workspace
+    does, so that what it keeps until the context goes is less than what it
+    uses, however many sizes a program runs through."""
+    torch = torch_cuda
+    c = dgm.GPU(stream=torch.cuda.current_stream())
+    try:
+        sizes = []
+        for M in (32768, 33792, 34816):
+            x, w = torch.ones(M, 4096, device="cuda"), torch.ones(2048, 4096, device="cuda")
+            y = torch.empty(M, 2048, device="cuda")
+            torch.cuda.synchronize()
+            c.begin()
+            c.gemmNT(32, w, None, None, x, None, y, M, 2048, 4096, 8)
+            c.end()
+            assert bool((y == 4096).all())
+            sizes.append(c.workspaceBytes())
+        assert sizes[0] > 256 << 20 and sizes[1] >= 2 * sizes[0] and sizes[2] == sizes[1]
+    finally:
+        c.close()
+
+
 def test_time_of_nonfinite(dgm, torch_cuda):
     """A token of NaN gradients flags every row of dW and one of dX. The call
     then takes what the fp32 MFMA kernels take for all of it (a context whose
