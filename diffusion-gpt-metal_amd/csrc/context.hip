@@ -168,12 +168,20 @@ uint8_t* planes_buffer(dgm_gpu* g, size_t bytes) {
     if (g->use_scratch || capturing(g->stream)) return nullptr;
     if (bytes > g->planes_bytes && (g->reserved || !grow_planes(g, bytes))) return nullptr;
     if (g->planes_stream && g->planes_stream != g->stream) {
-        if (capturing(g->planes_stream) ||
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        const bool asked = hipStreamIsCapturing(g->planes_stream, &cs) == hipSuccess;
+        if (asked && cs != hipStreamCaptureStatusNone) return nullptr;
+        if (!asked ||
             (!g->planes_event && hipEventCreateWithFlags(&g->planes_event, hipEventDisableTiming) != hipSuccess) ||
             hipEventRecord(g->planes_event, g->planes_stream) != hipSuccess ||
             hipStreamWaitEvent(g->stream, g->planes_event, 0) != hipSuccess) {
+            // A stream that is gone (against dgm_gpu_destroy's condition): its
+            // work is over once the device is idle, and the buffer free again.
             (void)hipGetLastError();
-            return nullptr;
+            if (hipDeviceSynchronize() != hipSuccess) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
         }
     }
     g->planes_stream = g->stream;
