@@ -164,6 +164,7 @@ PROTOTYPES = {
     "dgm_gemm_dw_acc": (_I, [_P, _P, _P, _P, _GP]),
     "dgm_quantize": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _I64]),
     "dgm_gemmNT": (_I, [_P, _I64, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64]),
+    "dgm_gemm_staging_bound": (_I64, [_I64, _I64, _I64]),
     "dgm_gemmNT_noalloc": (_I, [_P, _I64, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64]),
     "dgm_gemmNT_workspace_bound": (_I64, [_I64, _I64, _I64]),
     "dgm_gpu_reserve": (_I, [_P, _I64]),

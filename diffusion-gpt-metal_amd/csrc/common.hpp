@@ -14,7 +14,7 @@
 // Context behind the opaque dgm_gpu handle (mirrors class GPU, src/GPU.swift:91-198).
 struct dgm_gpu {
     int device = 0;
-    int num_cus = 256;
+    int num_cus = 256;   // dgm::kCus
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
     bool begun = false;
@@ -232,6 +232,13 @@ int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const fl
                float* Y, const dgm_GemmP* p, float* Y2 = nullptr);
 int planes_bwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, const float* X, float* dX,
                float* dW, const dgm_GemmP* p, bool accumulate);
+
+// Bytes of plane buffer that any of these calls of a linear [N, K] over M rows
+// takes on `cus` CUs (0: none takes these kernels).
+size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus);
+// Slices of K that a decode forward is cut into, at most (gemm_decode.hip).
+int64_t decode_slices(int bits, int64_t N, int64_t K, int cus);
+constexpr int kCus = 256;   // of an MI355X
 
 // Y[m, n] = part[0][m][n] + part[1][m][n] + ... + bias[n] (gemm_slab.hip).
 void slab_sum(dgm_gpu* g, const float* part, const float* bias, float* Y, int slices, int M, int N);

@@ -1177,8 +1177,7 @@ int decode_dispatch(dgm_gpu* g, DecArgs& a, const float* X) {
     // 4096 x 14336 int8 55.0 -> 26.8 us, int4 43.0 -> 23.3, 64 rows 64.9 -> 31.6;
     // 16 workgroups, 20 x 1024 x 4096 int8 in two 19.5 -> 15.0. Where no
     // workspace is to be had for the sums, K stays whole.
-    const int64_t wgs = dgm::ceil_div(a.N, DEC_COLS), intervals = (a.nchunk + 3) / 4;
-    a.slices = int(std::max<int64_t>(1, std::min<int64_t>(g->num_cus / wgs, intervals / 3)));
+    a.slices = int(dgm::decode_slices(BITS, a.N, a.K, g->num_cus));
     const size_t own = (xp_bytes + ex_bytes + 511) & ~size_t(255);
     uint8_t* ws = nullptr;
     if (a.slices > 1)
@@ -1241,6 +1240,11 @@ void decode_wait_check(dgm_gpu* g) {
 // The decode kernel's domain: quantized weights, 1 <= M <= 64, blocks inside
 // groups (G a multiple of 128 for int4, 64 for int8), whole chunks (K a
 // multiple of 256 / 128), 32-bit byte offsets, aligned buffers.
+int64_t decode_slices(int bits, int64_t N, int64_t K, int cus) {
+    const int64_t wgs = ceil_div(N, DEC_COLS), chunks = K * bits / 8 / 128, intervals = (chunks + 3) / 4;
+    return std::max<int64_t>(1, std::min<int64_t>(cus / std::max<int64_t>(wgs, 1), intervals / 3));
+}
+
 bool decode_ok(int bits, const void* W, const float* X, const float* S, const dgm_GemmP* p) {
     if (bits != 4 && bits != 8) return false;
     if (p->M < 1 || p->M > 64 || p->K == 0 || p->N == 0) return false;

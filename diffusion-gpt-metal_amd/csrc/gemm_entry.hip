@@ -154,6 +154,18 @@ int64_t dgm_gemmNT_workspace_bound(int64_t M, int64_t N, int64_t K) {
     return b;
 }
 
+int64_t dgm_gemm_staging_bound(int64_t M, int64_t N, int64_t K) {
+    int64_t b = dgm_gemmNT_workspace_bound(M, N, K);
+    if (b < 0) return b;
+    // Pieces and the sums of slices of K (int8 has the most) of the decode
+    // kernel.
+    if (M <= 64) b = std::max(b, 260 * K + 1024 + dgm::decode_slices(8, N, K, dgm::kCus) * M * N * 4);
+    // Operand pieces of large products: this shape's forward, dX and dW.
+    if (M <= dgm::kMaxIndex && N <= dgm::kMaxIndex && K <= dgm::kMaxIndex)
+        b = std::max(b, int64_t(dgm::planes_bytes(M, N, K, dgm::kCus)));
+    return b;
+}
+
 int dgm_gpu_reserve(dgm_gpu* g, int64_t bytes) {
     if (!g || bytes < 0) return DGM_ERR_ARG;
     if (bytes == 0) return DGM_OK;   // asks for nothing, and fixes nothing
@@ -170,7 +182,10 @@ int dgm_gpu_reserve(dgm_gpu* g, int64_t bytes) {
     return DGM_OK;
 }
 
-int64_t dgm_gpu_workspace_bytes(const dgm_gpu* g) { return g ? int64_t(g->ws_bytes + g->planes_bytes) : -1; }
+// The larger of the two buffers: what a reserve of that size makes of both.
+int64_t dgm_gpu_workspace_bytes(const dgm_gpu* g) {
+    return g ? int64_t(std::max(g->ws_bytes, g->planes_bytes)) : -1;
+}
 
 int dgm_gemmDX(dgm_gpu* g, int64_t bits, const float* w, const void* q, const float* scale,
                const float* dy, float* dx, int64_t M, int64_t N, int64_t K, int64_t qGroup) {

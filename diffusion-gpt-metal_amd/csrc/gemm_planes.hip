@@ -1020,65 +1020,82 @@ struct Product {
     bool accumulate;
 };
 
-// One product, or two of two planes; kNotFused, launching nothing, without a
-// plane buffer. dry: only whether there is one.
-int run(dgm_gpu* g, const Product* q, int n, bool dry = false) {
-    const bool code = n == 1 && one_plane(q[0].b);
-    const int gps = code ? q[0].b.G / 32 : 1, chunk = code ? gps : 2;
-    int64_t blocks[2] = {}, M[2] = {}, N[2] = {}, tiles[2] = {}, full[2] = {};
-    int splits[2] = {1, 1}, t = 0;
+// How one product, or two of two planes, are cut, and where their pieces lie
+// in the plane buffer.
+struct Layout {
+    bool code;             // one product, its B one plane
+    int gps, chunk, t;     // t: of kTiles
+    int64_t M[2], N[2], blocks[2], tiles[2], full[2];
+    int splits[2];
+    Operands op;
+    size_t bytes, at[4][4], parts[2];
+};
+
+// False: not for these kernels.
+bool layout(const Product* q, int n, int cus, Layout& l) {
+    l = Layout{};
+    const bool code = l.code = n == 1 && one_plane(q[0].b);
+    l.gps = code ? q[0].b.G / 32 : 1;
+    l.chunk = code ? l.gps : 2;
     for (int i = 0; i < n; ++i) {
-        M[i] = q[i].a.R;
-        N[i] = q[i].b.R;
-        blocks[i] = code ? q[i].a.C / 16 : round_up(dgm::ceil_div(q[i].a.C, 16), 2);
+        l.M[i] = q[i].a.R;
+        l.N[i] = q[i].b.R;
+        l.blocks[i] = code ? q[i].a.C / 16 : round_up(dgm::ceil_div(q[i].a.C, 16), 2);
     }
     // The backward's products are cut alike in one call and in two.
     const bool uniform = n == 2 || q[0].a.col || q[0].b.col;
     for (int i = 0; i < n; ++i) {
-        const Plan plan = plan_for(M[i], N[i], blocks[i], code ? chunk * 2 : chunk, code ? 1.0 / gps : 0.0, uniform,
-                                   g->num_cus);
-        t = plan.tile;
-        full[i] = plan.full;
-        splits[i] = plan.splits;
+        const Plan plan = plan_for(l.M[i], l.N[i], l.blocks[i], code ? l.chunk * 2 : l.chunk, code ? 1.0 / l.gps : 0.0,
+                                   uniform, cus);
+        l.t = plan.tile;
+        l.full[i] = plan.full;
+        l.splits[i] = plan.splits;
     }
-    if (n == 2) t = pair_tile(M, N, blocks, splits, g->num_cus);
-    const Tile& tile = kTiles[t];
-    Operands op{};
-    MaxArgs mx{};
-    PlaneArgs p[2] = {};
-    // Where the pieces lie in the plane buffer.
-    size_t bytes = 0, at[4][4] = {}, parts[2] = {};
+    if (n == 2) l.t = pair_tile(l.M, l.N, l.blocks, l.splits, cus);
+    const Tile& tile = kTiles[l.t];
     auto take = [&](int64_t size) {
-        const size_t here = bytes;
-        bytes += size_t(round_up(size, 256));
+        const size_t here = l.bytes;
+        l.bytes += size_t(round_up(size, 256));
         return here;
     };
     for (int i = 0; i < n; ++i) {
-        tiles[i] = int64_t(dgm::ceil_div(M[i], tile.tm)) * dgm::ceil_div(N[i], tile.tn);
-        if (tiles[i] > (1 << 24)) return dgm::kNotFused;   // 32-bit tile numbers
-        if (n == 2) full[i] = splits[i] == 1 ? tiles[i] : 0;
-        op.o[2 * i] = operand(q[i].a, tile.tm, blocks[i]);
-        op.o[2 * i + 1] = operand(q[i].b, tile.tn, blocks[i]);
-        if (code) op.o[1].gpad = int(blocks[0] / 2 / gps);
+        l.tiles[i] = int64_t(dgm::ceil_div(l.M[i], tile.tm)) * dgm::ceil_div(l.N[i], tile.tn);
+        if (l.tiles[i] > (1 << 24)) return false;   // 32-bit tile numbers
+        if (n == 2) l.full[i] = l.splits[i] == 1 ? l.tiles[i] : 0;
+        l.op.o[2 * i] = operand(q[i].a, tile.tm, l.blocks[i]);
+        l.op.o[2 * i + 1] = operand(q[i].b, tile.tn, l.blocks[i]);
+        if (code) l.op.o[1].gpad = int(l.blocks[0] / 2 / l.gps);
         for (int k = 2 * i; k < 2 * i + 2; ++k) {
-            const Operand& o = op.o[k];
-            at[k][0] = take(int64_t(o.rb) * o.kb * 2048);
-            at[k][1] = take(int64_t(o.rb) * 3 * 128);
-            at[k][2] = take(int64_t(o.parts) * o.width * 8);
-            at[k][3] = take(int64_t(o.gpad) * o.rb * 128);
+            const Operand& o = l.op.o[k];
+            l.at[k][0] = take(int64_t(o.rb) * o.kb * 2048);
+            l.at[k][1] = take(int64_t(o.rb) * 3 * 128);
+            l.at[k][2] = take(int64_t(o.parts) * o.width * 8);
+            l.at[k][3] = take(int64_t(o.gpad) * o.rb * 128);
         }
-        parts[i] = take((tiles[i] - full[i]) * splits[i] * tile.tm * tile.tn * 4);
+        l.parts[i] = take((l.tiles[i] - l.full[i]) * l.splits[i] * tile.tm * tile.tn * 4);
     }
-    uint8_t* ws = dgm::planes_buffer(g, bytes);
+    return true;
+}
+
+// kNotFused, launching nothing, without a plane buffer. dry: only whether
+// there is one.
+int run(dgm_gpu* g, const Product* q, int n, bool dry = false) {
+    Layout l;
+    if (!layout(q, n, g->num_cus, l)) return dgm::kNotFused;
+    uint8_t* ws = dgm::planes_buffer(g, l.bytes);
     if (!ws) return dgm::kNotFused;
     if (dry) return DGM_OK;
+    const Tile& tile = kTiles[l.t];
+    Operands& op = l.op;
+    MaxArgs mx{};
+    PlaneArgs p[2] = {};
     unsigned max_blocks = 0, split_blocks = 0;
     for (int k = 0; k < 2 * n; ++k) {
         Operand& o = op.o[k];
-        o.planes = ws + at[k][0];
-        o.exps = reinterpret_cast<int*>(ws + at[k][1]);
-        o.part = reinterpret_cast<uint32_t*>(ws + at[k][2]);
-        if (o.gpad) o.scales = reinterpret_cast<float*>(ws + at[k][3]);
+        o.planes = ws + l.at[k][0];
+        o.exps = reinterpret_cast<int*>(ws + l.at[k][1]);
+        o.part = reinterpret_cast<uint32_t*>(ws + l.at[k][2]);
+        if (o.gpad) o.scales = reinterpret_cast<float*>(ws + l.at[k][3]);
         mx.m[k] = max_arg(o);
         max_blocks += unsigned(mx.m[k].blocks);
         split_blocks += unsigned(o.blocks);
@@ -1101,29 +1118,29 @@ int run(dgm_gpu* g, const Product* q, int n, bool dry = false) {
         r.out2 = q[i].out2;
         r.ldo = q[i].ldo;
         r.cols1 = q[i].cols1;
-        r.M = int(M[i]);
-        r.N = int(N[i]);
-        r.stages = int(code ? blocks[i] / 2 : blocks[i]);
-        r.chunk = chunk;
+        r.M = int(l.M[i]);
+        r.N = int(l.N[i]);
+        r.stages = int(l.code ? l.blocks[i] / 2 : l.blocks[i]);
+        r.chunk = l.chunk;
         r.scales = b.scales;
         r.scale_ld = b.rb * 32;
-        r.gps = gps;
+        r.gps = l.gps;
         r.tiles_m = a.rb * 32 / tile.tm;
         r.tiles_n = b.rb * 32 / tile.tn;
-        r.full = int(full[i]);
+        r.full = int(l.full[i]);
         r.per_full = (r.full + 7) / 8;
-        r.splits = splits[i];
-        r.per_part = (int(tiles[i] - full[i]) * splits[i] + 7) / 8;
-        r.part = reinterpret_cast<float*>(ws + parts[i]);
+        r.splits = l.splits[i];
+        r.per_part = (int(l.tiles[i] - l.full[i]) * l.splits[i] + 7) / 8;
+        r.part = reinterpret_cast<float*>(ws + l.parts[i]);
         r.accumulate = q[i].accumulate;
     }
-    if (code) {
-        if (t == 0) return launch_gemm<CodeWide>(g, p, n);
-        if (t == 1) return launch_gemm<CodeTall>(g, p, n);
+    if (l.code) {
+        if (l.t == 0) return launch_gemm<CodeWide>(g, p, n);
+        if (l.t == 1) return launch_gemm<CodeTall>(g, p, n);
         return launch_gemm<CodeSmall>(g, p, n);
     }
-    if (t == 0) return launch_gemm<Wide>(g, p, n);
-    if (t == 1) return launch_gemm<Tall>(g, p, n);
+    if (l.t == 0) return launch_gemm<Wide>(g, p, n);
+    if (l.t == 1) return launch_gemm<Tall>(g, p, n);
     return launch_gemm<Small>(g, p, n);
 }
 
@@ -1187,21 +1204,68 @@ bool planes_pay_bwd(int64_t M, int64_t N, int64_t K) {
     return M > 64 && N >= 128 && K >= 128 && double(M) * double(N) * double(K) >= double(int64_t(11) << 26);
 }
 
+namespace {
+
+// Y [M, N], or Y and Y2 [M, N / 2].
+Product forward_of(int bits, const void* W, const float* scale, const float* X, const float* bias, float* Y,
+                   const dgm_GemmP* p, float* Y2) {
+    const int N = int(p->N), cols1 = Y2 ? N / 2 : N;
+    return Product{dense(X, int(p->M), int(p->K), p->K, 0), weights(bits, W, scale, p, 0), p->hasBias ? bias : nullptr,
+                   Y, Y2, cols1, cols1, false};
+}
+
+int backward_of(Product* q, int bits, const void* W, const float* scale, const float* dY, const float* X, float* dX,
+                float* dW, const dgm_GemmP* p, bool accumulate) {
+    const int M = int(p->M), N = int(p->N), K = int(p->K);
+    int n = 0;
+    if (dX) q[n++] = Product{dense(dY, M, N, N, 0), weights(bits, W, scale, p, 1), nullptr, dX, nullptr, K, K, false};
+    if (dW) q[n++] = Product{dense(dY, N, M, N, 1), dense(X, K, M, K, 1), nullptr, dW, nullptr, K, K, accumulate};
+    return n;
+}
+
+size_t layout_bytes(const Product* q, int n, int cus) {
+    Layout l;
+    return layout(q, n, cus, l) ? l.bytes : 0;
+}
+
+}  // namespace
+
+size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus) {
+    const dgm_GemmP p{uint32_t(M), uint32_t(N), uint32_t(K), 0u, 1u, 0u, 0u, 0u};
+    size_t b = 0;
+    Product q[2];
+    if (planes_pay_fwd(M, N, K)) {
+        q[0] = forward_of(32, nullptr, nullptr, nullptr, nullptr, nullptr, &p, nullptr);   // two planes of any weights
+        b = layout_bytes(q, 1, cus);
+        for (int64_t stages = K / 32, gps = 1; K % 32 == 0 && gps <= stages; ++gps) {   // one plane, every group
+            if (stages % gps != 0) continue;
+            dgm_GemmP pg = p;
+            pg.qGroup = uint32_t(32 * gps);
+            q[0] = forward_of(8, nullptr, nullptr, nullptr, nullptr, nullptr, &pg, nullptr);
+            b = std::max(b, layout_bytes(q, 1, cus));
+        }
+    }
+    if (planes_pay_bwd(M, N, K)) {
+        float* const some = reinterpret_cast<float*>(16);   // asked for, never read
+        for (int both = 0; both < 3; ++both) {
+            const int n = backward_of(q, 32, nullptr, nullptr, nullptr, nullptr, both != 1 ? some : nullptr,
+                                      both != 0 ? some : nullptr, &p, false);
+            b = std::max(b, layout_bytes(q, n, cus));
+        }
+    }
+    return b;
+}
+
 int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* X, const float* bias,
                float* Y, const dgm_GemmP* p, float* Y2) {
-    const int N = int(p->N), cols1 = Y2 ? N / 2 : N;
-    const Product q{dense(X, int(p->M), int(p->K), p->K, 0), weights(bits, W, scale, p, 0), p->hasBias ? bias : nullptr,
-                    Y, Y2, cols1, cols1, false};
+    const Product q = forward_of(bits, W, scale, X, bias, Y, p, Y2);
     return run(g, &q, 1, X == nullptr);
 }
 
 int planes_bwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, const float* X, float* dX,
                float* dW, const dgm_GemmP* p, bool accumulate) {
-    const int M = int(p->M), N = int(p->N), K = int(p->K);
     Product q[2];
-    int n = 0;
-    if (dX) q[n++] = Product{dense(dY, M, N, N, 0), weights(bits, W, scale, p, 1), nullptr, dX, nullptr, K, K, false};
-    if (dW) q[n++] = Product{dense(dY, N, M, N, 1), dense(X, K, M, K, 1), nullptr, dW, nullptr, K, K, accumulate};
+    const int n = backward_of(q, bits, W, scale, dY, X, dX, dW, p, accumulate);
     return run(g, q, n, dY == nullptr);
 }
 

@@ -122,6 +122,11 @@ class GPU:
         counterpart in the reference, whose buffers are all made at setup)."""
         return int(self.lib.dgm_gemmNT_workspace_bound(M, N, K))
 
+    def gemm_staging_bound(self, M: int, N: int, K: int) -> int:
+        """Bytes of workspace with which gemmNT, gemmDX, gemmDW and gemmBwd of
+        this shape run as fast as on a context that allocates as it goes."""
+        return int(self.lib.dgm_gemm_staging_bound(M, N, K))
+
     def reserve(self, nbytes: int) -> None:
         """Grow the context's workspace to at least nbytes now, so that later
         calls within it allocate nothing."""

@@ -194,19 +194,22 @@ int dgm_gemmNT_noalloc(dgm_gpu* g, int64_t bits, const float* w, const void* q,
  * second buffer of the context, which calls under graph capture do not use
  * (they, and calls for which no memory is left, take the kernels that stage
  * nothing). A call on another stream than the last one to use that buffer
- * waits for that one. dgm_gemmNT_workspace_bound returns bytes that cover every path a
- * dgm_gemmNT call of that shape can take, in either math mode (-1 for
- * negative sizes); dgm_gpu_reserve grows both buffers to at least `bytes`
- * now (DGM_ERR_UNSUPPORTED during a graph capture), so that later calls whose
- * bound it covers allocate nothing (the bound leaves out what a call can do
- * without: after a reserve, large products whose f16 pieces do not fit the
- * reserved bytes take the kernels that stage nothing, and calls of 17 to 64
- * rows whose slice sums do not fit keep K whole; the pieces need 4 bytes for
- * each element of both operands, rows padded to 256, and some tens of MB of
- * partial sums, the slices 4 M N bytes each, 256 / ceil(N / 64) of them at most);
- * dgm_gpu_workspace_bytes returns the size of both (0 before anything was
- * allocated). */
+ * waits for that one. dgm_gemmNT_workspace_bound returns bytes that cover what
+ * a dgm_gemmNT call of that shape cannot do without, on any path, in either
+ * math mode; dgm_gemm_staging_bound (never less) also what makes it, and
+ * dgm_gemmDX, dgm_gemmDW and dgm_gemmBwd of the shape, faster: the f16 pieces of large
+ * products and, at up to 64 rows, the sums of slices of K (both -1 for negative
+ * sizes). dgm_gpu_reserve grows both buffers to at least `bytes` now, and then
+ * they grow by a reserve only, but for staging that a call cannot do without:
+ * later calls whose bound it covers allocate nothing, and those whose staging
+ * bound it covers run the kernels that they run on a context without a reserve;
+ * the others take kernels that stage less (for large products the fp32 ones,
+ * several times slower). A reserve that cannot grow a buffer leaves the context as it
+ * was: DGM_ERR_UNSUPPORTED during a graph capture, DGM_ERR_HIP without the
+ * memory; one of 0 bytes does nothing. dgm_gpu_workspace_bytes returns the size
+ * of the larger buffer (0 before anything was allocated). */
 int64_t dgm_gemmNT_workspace_bound(int64_t M, int64_t N, int64_t K);
+int64_t dgm_gemm_staging_bound(int64_t M, int64_t N, int64_t K);
 int dgm_gpu_reserve(dgm_gpu* g, int64_t bytes);
 int64_t dgm_gpu_workspace_bytes(const dgm_gpu* g);
 /* GPU.gemmDX (src/GPU.swift:245-260). */

@@ -78,3 +78,19 @@ def test_workspace_bound_closed_forms(dgm):
     assert f(65, 10, 100) == 260 * 100 + 512                       # 2 M K = 13,000 is smaller
     assert f(0, 0, 0) == 512
     assert f(-1, 4, 4) == -1 and f(4, -1, 4) == -1 and f(4, 4, -1) == -1
+
+
+def test_staging_bound(dgm):
+    """dgm_gemm_staging_bound adds the slices' sums of the decode kernel (256
+    CUs over ceil(N / 64) workgroups, a third of K / 512 at most) and the operand
+    pieces of large products: 4 bytes an element and more, 2 for codes in one
+    plane, which rows padded to tiles and the cut tiles' sums come on top of."""
+    lib = dgm.load_library()
+    f, least = lib.dgm_gemm_staging_bound, lib.dgm_gemmNT_workspace_bound
+    assert f(24, 4096, 14336) == 260 * 14336 + 1024 + 4 * 24 * 4096 * 4
+    assert f(1, 14336, 4096) == 260 * 4096 + 1024 + 14336 * 4
+    assert f(1024, 512, 128) == least(1024, 512, 128)            # too small for pieces
+    M, N, K = 2048, 4096, 4096
+    pair = 4 * (2 * M * N + N * K + M * K)                       # dY in both orders, W, X
+    assert pair < f(M, N, K) < 1.25 * pair
+    assert f(-1, 4, 4) == -1 and f(4, -1, 4) == -1 and f(4, 4, -1) == -1

@@ -312,7 +312,7 @@ def test_buffer_capture_and_streams(dgm, gpu, torch_cuda):
         assert torch.equal(yn, yc)
         assert g.workspaceBytes() == held
         small = dgm.GPU(stream=st[0])
-        small.reserve(small.gemmNT_workspace_bound(M, N, K))
+        small.reserve(2 * M * K)     # less than the pieces
         held = small.workspaceBytes()
         ys[1].zero_()
         torch.cuda.synchronize()

@@ -117,7 +117,8 @@ def test_growth_during_capture_is_refused(dgm, orc, torch_cuda):
 
 # (math, bits, (M, N, K, G)): stream (M = 1), K-sliced (fp32 M = 16, int4 and int8), one-launch
 # decode (reduced M = 16), decode pieces (M = 64 both modes, M = 33), int8
-# skinny (M = 24 int8 fp32), bf16 prefill (M = 256 reduced), fp32 tiles (M = 256).
+# skinny (M = 24 int8 fp32), bf16 prefill (M = 256 reduced), fp32 tiles
+# (M = 256).
 CASES = [
     ("fp32", 4, (1, 14336, 4096, 128)),
     ("fp32", 4, (16, 14336, 4096, 128)),
@@ -129,6 +130,17 @@ CASES = [
     ("fp32", 8, (24, 4096, 2048, 64)),
     ("bf16", 4, (256, 2048, 1024, 128)),
     ("fp32", 4, (256, 2048, 1024, 128)),
+]
+
+
+# Staging that a call can do without: sums of slices of K, operand pieces.
+FASTER = [
+    ("fp32", 8, (24, 4096, 14336, 128)),     # slices of K: their sums
+    ("bf16", 4, (33, 2048, 8192, 128)),
+    ("fp32", 4, (20, 1024, 8192, 32)),       # groups inside a block, sliced
+    ("fp32", 4, (2048, 4096, 1024, 128)),    # operand pieces, codes in one plane
+    ("fp32", 8, (517, 1000, 4128, 8)),       # and in two
+    ("fp32", 8, (300, 2500, 3168, 96)),
 ]
 
 
@@ -177,6 +189,62 @@ def test_reserve_covers_the_call(dgm, torch_cuda, gpu, math, bits, shape):
         assert np.all(np.isfinite(y0))
         assert np.array_equal(y0.view(np.uint32), y1.view(np.uint32))
         assert np.array_equal(y1.view(np.uint32), y2.view(np.uint32))
+    finally:
+        lazy.close()
+        eager.close()
+
+
+@pytest.mark.parametrize("math,bits,shape", FASTER)
+def test_reserve_of_the_staging_bound(dgm, torch_cuda, gpu, math, bits, shape):
+    """A context that reserved the staging bound of a shape allocates nothing
+    for it and runs it with the bits, so on the kernels, of one without a
+    reserve; with the smaller workspace bound it allocates nothing either."""
+    M, N, K, G = shape
+    x, q, s = _case(gpu, M, N, K, G, bits, M + K)
+    st = torch_cuda.cuda.current_stream()
+    contexts = [dgm.GPU(stream=st) for _ in range(3)]
+    lazy, eager, least = contexts
+    try:
+        want = _forward(lazy, dgm, math, bits, q, s, x, M, N, K, G)
+        bound, staging = gpu.gemmNT_workspace_bound(M, N, K), gpu.gemm_staging_bound(M, N, K)
+        assert staging > bound
+        for c, b in ((eager, staging), (least, bound)):
+            c.reserve(b)
+            held = c.workspaceBytes()
+            y = _forward(c, dgm, math, bits, q, s, x, M, N, K, G)
+            assert c.workspaceBytes() == held >= b
+            if c is eager or M > 64:     # the pieces of few rows leave room for the sums
+                assert np.array_equal(want.view(np.uint32), y.view(np.uint32)) == (c is eager)
+        assert lazy.workspaceBytes() <= max(eager.workspaceBytes(), 1 << 20)
+    finally:
+        for c in contexts:
+            c.close()
+
+
+@pytest.mark.parametrize("bits,M,N,K,G", [(8, 1024, 2048, 1024, 32), (4, 300, 3000, 1056, 32), (32, 3072, 1536, 384, 8)])
+def test_reserve_covers_the_backward(dgm, gpu, torch_cuda, bits, M, N, K, G):
+    """The staging bound of a shape covers dX, dW and gemmBwd of it too."""
+    torch = torch_cuda
+    x, q, s = _case(gpu, M, N, K, G, bits, 3) if bits != 32 else (torch.randn(M * K, device="cuda"), None, None)
+    w = torch.randn(N * K, device="cuda") if bits == 32 else None
+    dy = torch.randn(M * N, device="cuda")
+    st = torch.cuda.current_stream()
+    lazy, eager = dgm.GPU(stream=st), dgm.GPU(stream=st)
+    try:
+        eager.reserve(eager.gemm_staging_bound(M, N, K))
+        held = eager.workspaceBytes()
+        outs = []
+        for c in (lazy, eager):
+            dx, dw, dx2, dw2 = (torch.zeros(n, device="cuda") for n in (M * K, N * K, M * K, N * K))
+            c.begin()
+            c.gemmBwd(bits, w, q, s, dy, x, dx, dw, M, N, K, G)
+            c.gemmDX(bits, w, q, s, dy, dx2, M, N, K, G)
+            c.gemmDW(dy, x, dw2, M, N, K)
+            c.end()
+            outs.append([from_dev(t).view(np.uint32) for t in (dx, dw, dx2, dw2)])
+        assert eager.workspaceBytes() == held and 0 < lazy.workspaceBytes() <= held
+        for a, b in zip(*outs):
+            assert np.array_equal(a, b)
     finally:
         lazy.close()
         eager.close()
