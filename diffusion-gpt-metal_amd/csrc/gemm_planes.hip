@@ -1067,7 +1067,7 @@ bool layout(const Product* q, int n, int cus, Layout& l) {
         if (code) l.op.o[1].gpad = int(l.blocks[0] / 2 / l.gps);
         for (int k = 2 * i; k < 2 * i + 2; ++k) {
             const Operand& o = l.op.o[k];
-            l.at[k][0] = take(int64_t(o.rb) * o.kb * 2048);
+            l.at[k][0] = take(int64_t(o.rb) * o.kb * (o.gpad ? 1024 : 2048));
             l.at[k][1] = take(int64_t(o.rb) * 3 * 128);
             l.at[k][2] = take(int64_t(o.parts) * o.width * 8);
             l.at[k][3] = take(int64_t(o.gpad) * o.rb * 128);

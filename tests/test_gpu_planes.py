@@ -371,6 +371,25 @@ def test_buffer_doubles(dgm, torch_cuda):
         c.close()
 
 
+def test_codes_of_one_plane_take_half(dgm, torch_cuda):
+    """A forward whose codes are kept as one plane takes 2 bytes for each, not the
+    4 of two planes (scales and X come to less than another byte here)."""
+    torch = torch_cuda
+    M, N, K, G = 128, 14336, 4096, 128
+    c = dgm.GPU(stream=torch.cuda.current_stream())
+    try:
+        x, _, w, q, s, wd, _ = _inputs(c, 4, M, N, K, G, 2)
+        y = torch.empty(M, N, device="cuda")
+        torch.cuda.synchronize()
+        c.begin()
+        c.gemmNT(4, w, q, s, x, None, y, M, N, K, G)
+        c.end()
+        assert _within(y, x.double() @ wd.T, x.double(), wd, K)
+        assert c.workspaceBytes() < 3 * N * K
+    finally:
+        c.close()
+
+
 def test_time_of_nonfinite(dgm, torch_cuda):
     """A token of NaN gradients flags every row of dW and one of dX. The call
     then takes what the fp32 MFMA kernels take for all of it (a context whose
