@@ -1067,6 +1067,10 @@ bool layout(const Product* q, int n, int cus, Layout& l) {
         if (code) l.op.o[1].gpad = int(l.blocks[0] / 2 / l.gps);
         for (int k = 2 * i; k < 2 * i + 2; ++k) {
             const Operand& o = l.op.o[k];
+            // The GEMM's 32-bit offsets of a stage (of two planes, 2 KB to a
+            // 16-c block) and of a group's scales.
+            if (int64_t(o.kb) * 2048 > (int64_t(1) << 32) || int64_t(o.gpad) * o.rb * 128 > (int64_t(1) << 32))
+                return false;
             l.at[k][0] = take(int64_t(o.rb) * o.kb * (o.gpad ? 1024 : 2048));
             l.at[k][1] = take(int64_t(o.rb) * 3 * 128);
             l.at[k][2] = take(int64_t(o.parts) * o.width * 8);

@@ -93,4 +93,8 @@ def test_staging_bound(dgm):
     M, N, K = 2048, 4096, 4096
     pair = 4 * (2 * M * N + N * K + M * K)                       # dY in both orders, W, X
     assert pair < f(M, N, K) < 1.25 * pair
+    # Contractions beyond 2^25 pass the 32-bit offsets of the pieces' kernels:
+    # dW of so many rows is left to others, and dX takes dY's pieces alone.
+    M, rows = 1 << 25, 4 * 128 << 25
+    assert f(M, 128, 128) > 4 * rows and f(M + 32, 128, 128) < 1.25 * rows
     assert f(-1, 4, 4) == -1 and f(4, -1, 4) == -1 and f(4, 4, -1) == -1
