@@ -56,6 +56,12 @@ struct dgm_gpu {
     bool reserved = false;                 // dgm_gpu_reserve was called: staging that a call can do without grows no more
     hipStream_t planes_stream = nullptr;   // of the last use
     hipEvent_t planes_event = nullptr;
+    // While a block entry point runs (dgm::Lend): room in the caller's workspace
+    // for the planes instead, and nothing of the context's grows that the call
+    // can do without.
+    bool lending = false;
+    uint8_t* lent = nullptr;
+    size_t lent_bytes = 0;
 };
 
 namespace dgm {
@@ -82,8 +88,8 @@ void* workspace_if(dgm_gpu* g, size_t bytes);
 // The status a caller returns when workspace() gave nullptr.
 int ws_error(dgm_gpu* g);
 // The buffer of the large GEMMs' operand planes, at least `bytes`, ordered
-// after its last use. nullptr (recording nothing) under graph capture, in
-// dgm_gemmNT_noalloc, when dgm_gpu_reserve fixed a smaller one, or when the
+// after its last use; while `lending`, the caller's room if it is that large.
+// nullptr (recording nothing) under graph capture, in dgm_gemmNT_noalloc, when dgm_gpu_reserve fixed a smaller one, or when the
 // memory is not there: the caller then takes the kernels that need no planes.
 uint8_t* planes_buffer(dgm_gpu* g, size_t bytes);
 // Makes that buffer hold `bytes` (more than it does), whatever was reserved;
@@ -91,6 +97,21 @@ uint8_t* planes_buffer(dgm_gpu* g, size_t bytes);
 bool grow_planes(dgm_gpu* g, size_t bytes);
 // Whether the stream is capturing a graph (or cannot be asked).
 bool capturing(hipStream_t s);
+// For a scope: the planes go to `floats` floats at `p` (16-byte aligned or not;
+// at least 0), memory that belongs to the call.
+struct Lend {
+    dgm_gpu* const g;
+    Lend(dgm_gpu* g_, float* p, int64_t floats) : g(g_) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(p), end = at + size_t(floats) * 4;
+        const uintptr_t first = (at + 255) & ~uintptr_t(255);
+        g->lending = true;
+        g->lent = reinterpret_cast<uint8_t*>(first);
+        g->lent_bytes = first < end ? end - first : 0;
+    }
+    ~Lend() { g->lending = false; }
+    Lend(const Lend&) = delete;
+    Lend& operator=(const Lend&) = delete;
+};
 // After a synchronize: records an error on g if a decode kernel gave up a
 // bounded in-workgroup wait since the last check (gemm_decode.hip), and
 // clears the device's flag.
@@ -233,9 +254,12 @@ int planes_fwd(dgm_gpu* g, int bits, const void* W, const float* scale, const fl
 int planes_bwd(dgm_gpu* g, int bits, const void* W, const float* scale, const float* dY, const float* X, float* dX,
                float* dW, const dgm_GemmP* p, bool accumulate);
 
-// Bytes of plane buffer that any of these calls of a linear [N, K] over M rows
-// takes on `cus` CUs (0: none takes these kernels).
-size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus);
+// Bytes of plane buffer that any of these calls (the forward; dX, dW and both)
+// of a linear [N, K] over M rows takes on `cus` CUs (0: none takes these kernels).
+size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus, bool forward = true, bool backward = true);
+// Floats that the block's forward (or its backward) adds to its workspace for
+// the planes of its linears, 0 where none is large enough.
+int64_t dit_planes_floats(const dgm_dit_cfg* c, bool backward);
 // Slices of K that a decode forward is cut into, at most (gemm_decode.hip).
 int64_t decode_slices(int bits, int64_t N, int64_t K, int cus);
 constexpr int kCus = 256;   // of an MI355X

@@ -118,7 +118,7 @@ void* workspace_if(dgm_gpu* g, size_t bytes) {
     if (g->use_scratch) return g->scratch && bytes <= kScratchBytes ? g->scratch : nullptr;
     if (bytes <= g->ws_bytes) return g->ws;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (g->reserved || g->n_retired == dgm_gpu::kMaxRetired || hipStreamIsCapturing(g->stream, &cs) != hipSuccess ||
+    if (g->reserved || g->lending || g->n_retired == dgm_gpu::kMaxRetired || hipStreamIsCapturing(g->stream, &cs) != hipSuccess ||
         cs != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return nullptr;
@@ -165,6 +165,7 @@ bool grow_planes(dgm_gpu* g, size_t bytes) {
 }
 
 uint8_t* planes_buffer(dgm_gpu* g, size_t bytes) {
+    if (g->lending) return bytes <= g->lent_bytes ? g->lent : nullptr;
     if (g->use_scratch || capturing(g->stream)) return nullptr;
     if (bytes > g->planes_bytes && (g->reserved || !grow_planes(g, bytes))) return nullptr;
     if (g->planes_stream && g->planes_stream != g->stream) {

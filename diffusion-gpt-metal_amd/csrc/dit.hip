@@ -947,10 +947,21 @@ int64_t dit_train_scratch_floats(const dgm_dit_cfg* c) {
     return 2 * ((M * QKV + 63) & ~int64_t(63)) + int64_t(c->B) * c->H * c->T * c->T;
 }
 
+int64_t dit_planes_floats(const dgm_dit_cfg* c, bool backward) {
+    if (!c || c->B <= 0 || c->T <= 0 || c->C <= 0 || c->F <= 0 || c->D <= 0) return 0;
+    const int64_t M = int64_t(c->B) * c->T, C = c->C, F = c->F, KV = c->D;
+    const int64_t nk[6][2] = {{C + 2 * KV, C}, {C, C}, {KV, C}, {2 * F, C}, {F, C}, {C, F}};
+    size_t b = 0;
+    for (const auto& l : nk)
+        if (l[0] <= kMaxIndex && l[1] <= kMaxIndex && M <= kMaxIndex)
+            b = std::max(b, planes_bytes(M, l[0], l[1], kCus, !backward, backward));
+    return b ? int64_t(b / 4) + 64 : 0;   // and what aligning them takes
+}
+
 namespace {
 // Gate and up of the stacked [wgate; wup] as one large product on split
 // operands (gemm_planes.hip), gate and up [M, F] each. With in null: whether
-// that pays and the context has the buffer for it.
+// that pays and the caller's workspace has room for it.
 int gate_up_planes(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_linear& L, const float* in, float* gate, float* up) {
     const int64_t M = int64_t(c->B) * c->T;
     // Against the one launch that also runs the row chain and SwiGLU, one block's
@@ -1169,7 +1180,9 @@ int dgm_ropeTables(int64_t maxT, int64_t dim, float theta, float* cos_t, float* 
 
 // ---- block forward ------------------------------------------------------------------
 
-int64_t dgm_dit_workspace_floats(const dgm_dit_cfg* c) { return c ? dit_workspace_floats(c) : -1; }
+int64_t dgm_dit_workspace_floats(const dgm_dit_cfg* c) {
+    return c ? dit_workspace_floats(c) + dgm::dit_planes_floats(c, false) : -1;
+}
 
 int dgm_dit_forward(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w, const float* cosv,
                     const float* sinv, float* x, float* ws, int64_t ws_floats) {
@@ -1200,6 +1213,7 @@ int dgm_dit_forward(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w, 
         if (c->bits == 32 ? !L->w : (!L->q || !L->scale)) return dgm::fail(g, DGM_ERR_ARG, "dit_forward: null weight");
     if (!w->n1 || !w->n1b || !w->n2 || !w->n2b || !w->nf) return dgm::fail(g, DGM_ERR_ARG, "dit_forward: null norm");
 
+    const dgm::Lend planes(g, ws + dit_workspace_floats(c), ws_floats - dit_workspace_floats(c));
     int64_t sz[NBUF];
     float* p[NBUF];
     dit_sizes(c, sz);

@@ -1373,12 +1373,12 @@ int dgm_accScale(dgm_gpu* g, float* a, const float* b, int64_t n, float s) {
 
 int64_t dgm_dit_acts_floats(const dgm_dit_cfg* c) {
     if (!c || c->loops < 0 || c->B <= 0 || c->T <= 0) return -1;
-    return acts_floats(c);
+    return acts_floats(c) + dgm::dit_planes_floats(c, false);
 }
 
 int64_t dgm_dit_backward_ws_floats(const dgm_dit_cfg* c) {
     if (!c || c->B <= 0 || c->T <= 0) return -1;
-    return bwd_floats(c);
+    return bwd_floats(c) + dgm::dit_planes_floats(c, true);
 }
 
 int dgm_dit_forward_train(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w, const float* cosv,
@@ -1388,6 +1388,7 @@ int dgm_dit_forward_train(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weight
     DGM_TRY(check_cfg(g, "dit_forward_train", c, w, false));
     if (!x || !acts || !cosv || !sinv) return dgm::fail(g, DGM_ERR_ARG, "dit_forward_train: null buffer");
     if (acts_n < acts_floats(c)) return dgm::fail(g, DGM_ERR_ARG, "dit_forward_train: activation buffer too small");
+    const dgm::Lend planes(g, acts + acts_floats(c), acts_n - acts_floats(c));
     int64_t asz[A_COUNT], fsz[F_COUNT];
     act_sizes(c, asz, fsz);
     const int L = c->loops;
@@ -1487,6 +1488,7 @@ int dgm_dit_backward(dgm_gpu* g, const dgm_dit_cfg* c, const dgm_dit_weights* w,
         if (!p) return dgm::fail(g, DGM_ERR_ARG, "dit_backward: null norm gradient");
     if (acts_n < acts_floats(c)) return dgm::fail(g, DGM_ERR_ARG, "dit_backward: activation buffer too small");
     if (ws_n < bwd_floats(c)) return dgm::fail(g, DGM_ERR_ARG, "dit_backward: workspace too small");
+    const dgm::Lend planes(g, ws + bwd_floats(c), ws_n - bwd_floats(c));
     // The loop shapes' forward keeps k and v of the KV head only, which the
     // one-launch attention backward reads; it needs 16-byte aligned buffers.
     if (dgm::dit_loop_shape_ok(c) && !dgm::dit_attn_bwd_loop_ok(c, acts, ws))

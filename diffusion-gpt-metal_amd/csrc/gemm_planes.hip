@@ -1234,11 +1234,11 @@ size_t layout_bytes(const Product* q, int n, int cus) {
 
 }  // namespace
 
-size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus) {
+size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus, bool forward, bool backward) {
     const dgm_GemmP p{uint32_t(M), uint32_t(N), uint32_t(K), 0u, 1u, 0u, 0u, 0u};
     size_t b = 0;
     Product q[2];
-    if (planes_pay_fwd(M, N, K)) {
+    if (forward && planes_pay_fwd(M, N, K)) {
         q[0] = forward_of(32, nullptr, nullptr, nullptr, nullptr, nullptr, &p, nullptr);   // two planes of any weights
         b = layout_bytes(q, 1, cus);
         for (int64_t stages = K / 32, gps = 1; K % 32 == 0 && gps <= stages; ++gps) {   // one plane, every group
@@ -1249,7 +1249,7 @@ size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus) {
             b = std::max(b, layout_bytes(q, 1, cus));
         }
     }
-    if (planes_pay_bwd(M, N, K)) {
+    if (backward && planes_pay_bwd(M, N, K)) {
         float* const some = reinterpret_cast<float*>(16);   // asked for, never read
         for (int both = 0; both < 3; ++both) {
             const int n = backward_of(q, 32, nullptr, nullptr, nullptr, nullptr, both != 1 ? some : nullptr,

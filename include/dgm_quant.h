@@ -295,7 +295,11 @@ typedef struct dgm_dit_weights {
     const float *n1, *n1b, *n2, *n2b, *nf;
 } dgm_dit_weights;
 
-/* Floats of device workspace dgm_dit_forward needs for cfg (-1 for NULL). */
+/* Floats of device workspace for dgm_dit_forward of cfg (-1 for NULL): what
+ * it needs and, where a linear of the block is a large product, room behind
+ * that for its operand pieces (a workspace without the room is accepted: those
+ * linears then run on the fp32 kernels). dgm_dit_acts_floats and
+ * dgm_dit_backward_ws_floats count the same way. */
 int64_t dgm_dit_workspace_floats(const dgm_dit_cfg* cfg);
 /* The looped block forward (src/DiT.swift:520-550): x holds xs[0] [B*T, C] on
  * entry and xs[loops] on exit. cos_t/sin_t are device copies of
