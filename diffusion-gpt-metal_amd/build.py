@@ -53,9 +53,12 @@ def hipcc() -> str:
 # Sources whose kernels issue loads as inline asm and wait for them by hand
 # (gemm_decode.hip, gemm_stream.hip, and the prefill producers of
 # gemm_bf16.hip): a register spilled while such a load is in flight would be
-# read before the load fills it, so these kernels must not use scratch. The
-# build checks the compiler's resource-usage remarks.
-NO_SCRATCH = {"gemm_decode.hip", "gemm_stream.hip", "gemm_bf16.hip", "gemm_slab.hip"}
+# read before the load fills it, so these kernels must not use scratch. Nor may
+# gemm_planes.hip's, which count their direct-to-LDS loads. The build checks the
+# compiler's resource-usage remarks.
+NO_SCRATCH = {"gemm_decode.hip", "gemm_stream.hip", "gemm_bf16.hip", "gemm_slab.hip", "gemm_planes.hip"}
+# Kernels whose waves per SIMD the host code counts on (file: name, waves).
+WAVES = {"gemm_planes.hip": ("plane_gemm_kernel", 2)}   # kTiles' slots
 REMARK = "-Rpass-analysis=kernel-resource-usage"
 
 
@@ -69,6 +72,20 @@ def _scratch_users(stderr: str) -> list:
         if m and fn and int(m.group(1)) > 0:
             users.append(f"{fn} ({m.group(1)} bytes/lane)")
     return users
+
+
+def _low_occupancy(stderr: str, kernel: str, waves: int) -> list:
+    low, fn, seen = [], None, 0
+    for line in stderr.splitlines():
+        m = re.search(r"remark: Function Name: (\S+)", line)
+        if m:
+            fn = m.group(1)
+        m = re.search(r"Occupancy \[waves/SIMD\]: (\d+)", line)
+        if m and fn and kernel in fn:
+            seen += 1
+            if int(m.group(1)) < waves:
+                low.append(f"{fn} ({m.group(1)})")
+    return low if seen else [f"no {kernel}"]
 
 
 def _compile(src: str) -> str:
@@ -85,6 +102,11 @@ def _compile(src: str) -> str:
         if bad:
             os.remove(obj)
             raise RuntimeError(f"{src}: kernels with hand-waited loads use scratch: {', '.join(bad)}")
+        if os.path.basename(src) in WAVES:
+            low = _low_occupancy(proc.stderr, *WAVES[os.path.basename(src)])
+            if low:
+                os.remove(obj)
+                raise RuntimeError(f"{src}: fewer waves per SIMD than the host code counts on: {', '.join(low)}")
         lines = [l for l in lines if REMARK not in l]
     err = "\n".join(lines)
     if err.strip():

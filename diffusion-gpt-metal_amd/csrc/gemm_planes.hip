@@ -580,8 +580,8 @@ __device__ __forceinline__ void exact_tile(const PlaneArgs& a, int r0, int c0, c
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(64 * T::WAVES) void plane_gemm_kernel(PlaneGroup g) {
+template <typename T>   // two waves to a SIMD: the 8 of a workgroup, or two workgroups of 4
+__global__ __launch_bounds__(64 * T::WAVES, 2) void plane_gemm_kernel(PlaneGroup g) {
     const bool second = int(blockIdx.x) >= g.first;
     const PlaneArgs& a = args_of(second);
     constexpr int MT = T::MT, NT = T::NT, RING = T::RING;
@@ -871,7 +871,7 @@ using CodeTall = Geo<4, 2, 2, 2, true, 3>;
 using CodeSmall = Geo<2, 2, 2, 2, true, 3>;
 
 struct Tile {
-    int tm, tn, slots;   // slots: workgroups a CU holds
+    int tm, tn, slots;   // slots: workgroups a CU holds (build.py checks the registers for it)
 };
 constexpr Tile kTiles[] = {{128, 256, 1}, {256, 128, 1}, {128, 128, 2}};
 
