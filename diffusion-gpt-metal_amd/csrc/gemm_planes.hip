@@ -95,10 +95,10 @@ struct Src {
 struct Operand {
     Src s;
     uint8_t* planes;
-    uint32_t* part;       // largest |element| (its bits) of each row: parts x width; then how many are not zero
+    uint32_t* part;       // largest |element| (its bits) of each row: parts x width
     int parts, width;
-    int* exps;            // row scale 2^e, or kFlag; then (each [32 rb]) the row's elements below
-                          // 2^-31 of its largest but not zero, and how many it may have
+    int* exps;            // row scale 2^e, or kFlag; then (each [32 rb]) how many of the row's elements
+                          // lie below 2^-31 of its largest but are not zero, and how many are zero (of codes, none counts)
     int rb, kb;           // 32-row blocks and 16-c blocks written (padded)
     float* scales;        // codes kept as one plane: their scales 2^e, [group][32 rb]
     int gpad;             // groups written there (padded)
@@ -118,7 +118,7 @@ __device__ __forceinline__ float elem(const Src& s, int r, int c) {
     return code_at(s.p, s.bits, i) * s.scale[si];
 }
 
-// ---- launch 1: largest |element| of each row, and its nonzero ones ----------------
+// ---- launch 1: largest |element| of each row ---------------------------------------
 // One pass over fp32 data (X, dY, W, or the scales that bound the codes'
 // weights). Rows stored contiguously: lpr lanes per row. Rows stored across:
 // a block takes 64 of them and one of `parts` chunks of c.
@@ -126,19 +126,18 @@ struct MaxArg {
     const float* p;
     int64_t ld;
     int R, C, col, lpr, parts, blocks;
-    uint32_t* out;   // [parts][R] largest; then nonzero
-    int* far;        // cleared for the split: `rows` of them
-    int rows;
+    uint32_t* out;
+    int* counts;     // of the split, cleared: n_counts of them
+    int n_counts;
 };
 
 __device__ __forceinline__ void max_part(const MaxArg& a, int block) {
     const int t = threadIdx.x;
-    uint32_t* const nonzero = a.out + int64_t(a.parts) * a.R;
-    for (int i = block * 256 + t; i < a.rows; i += a.blocks * 256) a.far[i] = 0;
+    for (int i = block * 256 + t; i < a.n_counts; i += a.blocks * 256) a.counts[i] = 0;
     if (!a.col) {
         const int per = 256 / a.lpr;
         const int r = block * per + t / a.lpr, l = t % a.lpr;
-        uint32_t m = 0, n = 0;
+        uint32_t m = 0;
         if (r < a.R) {
             const float* row = a.p + int64_t(r) * a.ld;
             const bool vec = (a.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(a.p) & 15) == 0;
@@ -149,47 +148,29 @@ __device__ __forceinline__ void max_part(const MaxArg& a, int block) {
                 for (int i = l; i < n4; i += a.lpr) {
                     const u32x4 v = reinterpret_cast<const u32x4*>(row)[i] & 0x7fffffffu;
                     m = max(max(m, max(v[0], v[1])), max(v[2], v[3]));
-                    n += min(v[0], 1u) + min(v[1], 1u) + min(v[2], 1u) + min(v[3], 1u);
                 }
                 c = n4 << 2;
             }
-            for (int i = c + l; i < a.C; i += a.lpr) {
-                const uint32_t v = __float_as_uint(row[i]) & 0x7fffffffu;
-                m = max(m, v);
-                n += min(v, 1u);
-            }
+            for (int i = c + l; i < a.C; i += a.lpr) m = max(m, __float_as_uint(row[i]) & 0x7fffffffu);
         }
-        for (int off = a.lpr >> 1; off >= 1; off >>= 1) {
-            m = max(m, uint32_t(__shfl_xor(int(m), off)));
-            n += uint32_t(__shfl_xor(int(n), off));
-        }
-        if (r < a.R && l == 0) {
-            a.out[r] = m;
-            nonzero[r] = n;
-        }
+        for (int off = a.lpr >> 1; off >= 1; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off)));
+        if (r < a.R && l == 0) a.out[r] = m;
         return;
     }
-    __shared__ uint32_t sh[2][4][64];
+    __shared__ uint32_t sh[4][64];
     const int nb = (a.R + 63) / 64;
     const int r = (block % nb) * 64 + (t & 63), part = block / nb;
     const int64_t chunk = (int64_t(a.C) + a.parts - 1) / a.parts;
     const int64_t c1 = min(int64_t(a.C), (part + 1) * chunk);
-    uint32_t m = 0, n = 0;
+    uint32_t m = 0;
     if (r < a.R) {
 #pragma unroll 8
-        for (int64_t c = part * chunk + (t >> 6); c < c1; c += 4) {
-            const uint32_t v = __float_as_uint(a.p[c * a.ld + r]) & 0x7fffffffu;
-            m = max(m, v);
-            n += min(v, 1u);
-        }
+        for (int64_t c = part * chunk + (t >> 6); c < c1; c += 4)
+            m = max(m, __float_as_uint(a.p[c * a.ld + r]) & 0x7fffffffu);
     }
-    sh[0][t >> 6][t & 63] = m;
-    sh[1][t >> 6][t & 63] = n;
+    sh[t >> 6][t & 63] = m;
     __syncthreads();
-    if (t < 64 && r < a.R) {
-        a.out[int64_t(part) * a.R + r] = max(max(sh[0][0][t], sh[0][1][t]), max(sh[0][2][t], sh[0][3][t]));
-        nonzero[int64_t(part) * a.R + r] = sh[1][0][t] + sh[1][1][t] + sh[1][2][t] + sh[1][3][t];
-    }
+    if (t < 64 && r < a.R) a.out[int64_t(part) * a.R + r] = max(max(sh[0][t], sh[1][t]), max(sh[2][t], sh[3][t]));
 }
 
 // The operands of up to two products.
@@ -310,10 +291,7 @@ __device__ __forceinline__ void codes_part(const Operand& o, int block) {
     }
     if (chunk != 0) return;
     const int e = row_exp(r < o.s.R ? o.part[r] : 0u, BITS == 8 ? 7 : 3);
-    if (wave == 0 && h == 0) {
-        o.exps[r] = e;
-        o.exps[2 * 32 * o.rb + r] = INT32_MAX;   // codes are exact
-    }
+    if (wave == 0 && h == 0) o.exps[r] = e;   // its counts stay at 0: codes are exact
     const float f = exp_factor(e);
     for (int g = threadIdx.x >> 5; g < o.gpad; g += 8)
         o.scales[int64_t(g) * (o.rb * 32) + r] =
@@ -343,44 +321,39 @@ __device__ __forceinline__ void split_part(const Operand& o, int block) {
         }
     }
     const int e = row_exp(m, BITS == 32 ? 0 : (BITS == 8 ? 7 : 3));
-    if (chunk == 0 && wave == 0 && h == 0) {
-        // How many elements may lie far below the largest (rows past the end:
-        // any). Of codes every one counts as not zero.
-        int limit = INT32_MAX;
-        if (r < o.s.R) {
-            limit = BITS == 32 ? 0 : o.s.C;
-            if constexpr (BITS == 32)
-                for (int i = 0; i < o.parts; ++i) limit += int(o.part[int64_t(o.parts + i) * o.width + r]);
-            limit /= 16;
-        }
-        o.exps[r] = e;
-        o.exps[2 * 32 * o.rb + r] = limit;
-    }
+    if (chunk == 0 && wave == 0 && h == 0) o.exps[r] = e;
     const float f = exp_factor(e);
-    int far = 0;
+    int far = 0, zeros = 0;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int kb = chunk * 16 + u * 4 + wave;
         if (kb >= o.kb) continue;
         f16x8 hi, lo;
-        uint32_t least = ~0u;
+        uint32_t least = ~0u, most = 0;   // of |x| minus one: a zero is the largest
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const float x = v[u][j] * f;
-            least = min(least, (__float_as_uint(x) << 1) - 1);   // a zero gives the largest
+            const uint32_t k = (__float_as_uint(x) << 1) - 1;
+            least = min(least, k);
+            most = max(most, k);
             hi[j] = _Float16(x);
             lo[j] = _Float16((x - float(hi[j])) * (1.0f / kLow));
         }
         uint8_t* out = o.planes + (int64_t(rb) * o.kb + kb) * 2048 + lane * 16;
         *reinterpret_cast<f16x8*>(out) = hi;
         *reinterpret_cast<f16x8*>(out + 1024) = lo;
-        if (least < 2 * 0x37000000u - 1) {   // below 2^-17
+        if (least < 2 * 0x37000000u - 1 || (BITS == 32 && most == ~0u)) {   // below 2^-17, or zero
+            const int n = min(8, o.s.C - kb * 16 - 8 * h);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) far += v[u][j] != 0.0f && fabsf(v[u][j] * f) < 0x1p-17f;
+            for (int j = 0; j < 8; ++j) {
+                zeros += BITS == 32 && j < n && v[u][j] == 0.0f;
+                far += v[u][j] != 0.0f && fabsf(v[u][j] * f) < 0x1p-17f;
+            }
         }
     }
     // From e = 114 on, fp32's own last bit (2^-149) is a multiple of l's (2^-36).
     if (far && e < 114) atomicAdd(o.exps + 32 * o.rb + r, far);
+    if (zeros && r < o.s.R) atomicAdd(o.exps + 64 * o.rb + r, zeros);
 }
 
 __device__ __forceinline__ void split_any(const Operand& o, int block) {
@@ -473,9 +446,9 @@ __device__ __forceinline__ const PlaneArgs& args_of(bool second) {
     return ((const PlaneArgs*)__builtin_amdgcn_kernarg_segment_ptr())[second ? 1 : 0];
 }
 
-// The exponent of row r, or kFlag.
-__device__ __forceinline__ int row_scale(const int* exps, int rows, int r) {
-    return exps[rows + r] > exps[2 * rows + r] ? kFlag : exps[r];
+// The exponent of row r of C elements, or kFlag.
+__device__ __forceinline__ int row_scale(const int* exps, int rows, int r, int C) {
+    return exps[rows + r] > (C - exps[2 * rows + r]) / 16 ? kFlag : exps[r];
 }
 
 // Tile L of the order: groups of GROUP_M tile rows, column after column, so
@@ -614,7 +587,8 @@ __global__ __launch_bounds__(64 * T::WAVES, 2) void plane_gemm_kernel(PlaneGroup
     const int m0 = ti * T::TM, n0 = tj * T::TN;
 
     for (int i = t; i < T::TM + T::TN; i += 64 * T::WAVES)
-        exps[i] = i < T::TM ? row_scale(a.ea, a.rows_a, m0 + i) : row_scale(a.eb, a.rows_b, n0 + i - T::TM);
+        exps[i] = i < T::TM ? row_scale(a.ea, a.rows_a, m0 + i, a.sa.C)
+                                : row_scale(a.eb, a.rows_b, n0 + i - T::TM, a.sa.C);
 
     // This wave's loads of a stage: units wave * UPW ..; first A's (AU to a
     // 32-row block), then B's. A stage further is AU or BU KB further.
@@ -821,8 +795,8 @@ __global__ __launch_bounds__(256, 7) void part_sum_kernel(PlaneGroup g) {
     const int r0 = ti * T::TM + (wave / T::WN * T::MT + sub / T::NT) * 32;
     const int c0 = tj * T::TN + (wave % T::WN * T::NT + sub % T::NT) * 32;
     if (r0 >= a.M || c0 >= a.N) return;
-    const int row_e = row_scale(a.ea, a.rows_a, r0 + (lane & 31));   // used after the sums
-    const int eb = row_scale(a.eb, a.rows_b, c0 + (lane & 31));
+    const int row_e = row_scale(a.ea, a.rows_a, r0 + (lane & 31), a.sa.C);   // used after the sums
+    const int eb = row_scale(a.eb, a.rows_b, c0 + (lane & 31), a.sa.C);
     f32x16 acc;
     for (int p = 0; p < a.splits; ++p) {
         const f32x4* o = reinterpret_cast<const f32x4*>(a.part) +
@@ -1002,8 +976,8 @@ MaxArg max_arg(const Operand& o) {
     m.col = s.col;
     m.parts = o.parts;
     m.out = o.part;
-    m.far = o.exps + 32 * o.rb;
-    m.rows = s.R;
+    m.counts = o.exps + 32 * o.rb;
+    m.n_counts = 64 * o.rb;
     m.R = o.width;
     m.C = codes && !s.col ? s.groups : s.C;
     m.lpr = m.C >= 512 ? 64 : m.C >= 128 ? 16 : 8;
@@ -1080,7 +1054,7 @@ bool layout(const Product* q, int n, int cus, Layout& l) {
                 return false;
             l.at[k][0] = take(int64_t(o.rb) * o.kb * (o.gpad ? 1024 : 2048));
             l.at[k][1] = take(int64_t(o.rb) * 3 * 128);
-            l.at[k][2] = take(int64_t(o.parts) * o.width * 8);
+            l.at[k][2] = take(int64_t(o.parts) * o.width * 4);
             l.at[k][3] = take(int64_t(o.gpad) * o.rb * 128);
         }
         l.parts[i] = take((l.tiles[i] - l.full[i]) * l.splits[i] * tile.tm * tile.tn * 4);

@@ -210,6 +210,28 @@ def test_outlier_channel_against_zeros(gpu, bits, G, ratio):
         assert err <= FAR_ONE, err
 
 
+@pytest.mark.parametrize("nonzero", [2, 15, 17, 200])
+def test_rows_of_mostly_zeros(gpu, nonzero):
+    """Zeros are not counted among the elements that a few small ones may hide in:
+    one huge element and a few others, the huge one against zeros."""
+    import torch
+    M, N, K = 512, 1700, 1003
+    g = torch.Generator(device="cuda").manual_seed(nonzero)
+    x, w = torch.zeros(M, K, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    for i in range(1, nonzero):
+        x[torch.arange(M, device="cuda"), torch.randint(1, K, (M,), generator=g, device="cuda")] = 1.0 + i / 7
+    x[:, 0] = 1e12
+    w[:, 0] = 0
+    y = torch.empty(M, N, device="cuda")
+    torch.cuda.synchronize()
+    gpu.begin()
+    gpu.gemmNT(32, w, None, None, x, None, y, M, N, K, 8)
+    gpu.end()
+    ref = x.double() @ w.double().T
+    err = float((y.double() - ref).norm() / ref.norm())
+    assert err <= FAR_ONE, err
+
+
 @pytest.mark.parametrize("spread", [8, 16, 24, 40, 60])
 def test_tokens_scaled_against_each_other(gpu, spread):
     """Tokens whose X is 2^s as large and whose dY is 2^-s: every product of dW
