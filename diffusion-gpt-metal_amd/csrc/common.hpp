@@ -47,8 +47,8 @@ struct dgm_gpu {
     bool spin_waits = false;
     // Operand planes of the large GEMMs (gemm_planes.hip): apart from `ws`,
     // which captured graphs may read while eager work runs on another stream.
-    // Grow-only like it; used by eager calls only, and a call on another
-    // stream than the last one's waits for that one's work.
+    // Grow-only like it (and at least doubling); used by eager calls only, and a
+    // call on another stream than the last one's waits for that one's work.
     void* planes = nullptr;
     size_t planes_bytes = 0;
     void* planes_retired[kMaxRetired] = {};

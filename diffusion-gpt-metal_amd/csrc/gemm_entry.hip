@@ -3,7 +3,8 @@
 // the call to the router of its direction (gemm_f32.hip): for quantized
 // forwards the few-row and decode-shaped kernels (int8 / f16 / bf16 MFMA over
 // exact activation pieces), the bf16 prefill kernel in the reduced-precision
-// mode, else the fp32 MFMA tiles; dX and dW always on the fp32 tiles.
+// mode, the f16 pieces of large products, else the fp32 MFMA tiles; dX and dW on
+// the pieces or the fp32 tiles.
 #include "common.hpp"
 
 #include <algorithm>

@@ -978,7 +978,8 @@ int launch_fwd_pipe(dgm_gpu* g, const GemmArgs& a) {
 
 // K % 64 == 0 and K <= 1024 (the X block stays in LDS; 512 with fp32
 // weights, which take 16 registers per stage), a group that is a
-// multiple of 16 (one scale per lane per stage), 16-byte aligned rows.
+// multiple of 8 (one scale per lane per stage where it is one of 16, else
+// two), 16-byte aligned rows.
 bool fwd_lds_ok(const GemmArgs& a, int bits, const void* X, const void* W) {
     if (a.K % 64 != 0 || a.K == 0 || a.K > 1024 || a.rows == 0 || a.cols == 0) return false;
     if (!dgm::aligned(X, 16)) return false;

@@ -40,9 +40,11 @@
 //
 // What it gains: v_mfma_f32_16x16x4_f32 peaks at 157 TFLOP/s and its kernels
 // here ran at 50-57; three f16 products per fp32 product at 2.5 PFLOP/s peak at
-// 833, two at 1250. Measured, both sides in turn: 2048 x 14336 x 4096 int4
-// 4816 -> 457 us (527 TFLOP/s), 517 x 4100 x 4128 int8 320 -> 77, dX + dW of 2048 x 4096 x
-// 4096 2416 -> 442, forward + dX + dW of fp32 12288 x 1536 x 384 779 -> 301.
+// 833, two at 1250. Measured, those kernels first: 2048 x 14336 x 4096 int4
+// 4816 and 466 us (517 TFLOP/s), 517 x 4100 x 4128 int8 320 and 80, dX + dW of 2048 x
+// 4096 x 4096 2416 and 418, forward + dX + dW of fp32 12288 x 1536 x 384 779 and 302.
+// (l unscaled, 2^-39 of a row's largest: 451, 76, 417 and 300; the codes' packed
+// multiplies are the difference. The figures beside the rules below are of that form.)
 // What bounds it: the power the matrix unit draws. With zeros for data the
 // GEMM of 4096 x 4096 x 4096 takes 225 us instead of 320 (the clock stays up);
 // interleaving the LDS reads with the MFMAs, raising their priority, one wave

@@ -4,8 +4,9 @@ DiTBlock holds the block's linears quantized once on the device
 (GPU.quantize, src/GPU.swift:220-225), device copies of the RoPE tables
 (ropeTables, src/Macro.swift:509-530, computed on the host as the reference
 does) and the forward's workspace. forward() enqueues the whole loop body
-(dgm_dit_forward) on the context's stream: nothing is allocated and nothing
-waits on the host, so the call can be captured into a HIP graph.
+(dgm_dit_forward) on the context's stream: nothing is allocated (for more than 64
+tokens in the fp32 mode; else run it once first) and nothing waits on the host, so
+the call can be captured into a HIP graph.
 """
 from __future__ import annotations
 

@@ -168,8 +168,8 @@ int dgm_gemmNT(dgm_gpu* g, int64_t bits, const float* w, const void* q,
  * harnesses that forbid hipMalloc). Same arguments, kernels and results
  * (bitwise; where dgm_gemmNT takes the f16 pieces of large products, or cuts
  * a long K at 17 to 64 rows into slices whose sums do not fit the scratch,
- * this entry takes the kernels without that staging, with the same error
- * bound) as dgm_gemmNT, but every staging buffer (the decode kernels'
+ * this entry takes the kernels without that staging, within the same 1e-5)
+ * as dgm_gemmNT, but every staging buffer (the decode kernels'
  * activation pieces, the bf16 copy of X of the reduced-precision prefill
  * path) comes from a static device scratch of DGM_NOALLOC_SCRATCH_BYTES per
  * GPU, held from library load until the process ends; nothing is allocated.
@@ -227,7 +227,9 @@ int dgm_gemmDWAcc(dgm_gpu* g, const float* dy, const float* x, float* dw,
  * GPU.gemmDX with the same dY: the pair the reference's backward issues back
  * to back for every linear (src/GPT.swift:374-376, 384-420). One launch when
  * the shapes allow (the dX and dW tiles run side by side), else the two
- * calls; either way dx and dw are bitwise what the two calls produce. */
+ * calls; either way dx and dw are bitwise what the two calls produce on the
+ * same context at the same time (under capture, or under a reserve that has no
+ * room for operand pieces, those differ from an eager call's). */
 int dgm_gemmBwd(dgm_gpu* g, int64_t bits, const float* w, const void* q, const float* scale,
                 const float* dy, const float* x, float* dx, float* dw, int64_t M, int64_t N,
                 int64_t K, int64_t qGroup, int accumulate);
@@ -314,7 +316,9 @@ int64_t dgm_dit_workspace_floats(const dgm_dit_cfg* cfg);
  * the standalone wrappers compute it. Needs T and D multiples of 16 and
  * C <= 1024 (DGM_ERR_UNSUPPORTED otherwise); x, ws and the tables 16-byte
  * aligned. Enqueued on the context's
- * stream; graph-capturable (no allocation, no host sync). */
+ * stream; graph-capturable (no host sync, and no allocation for more than 64
+ * tokens in all in the fp32 mode; fewer tokens and the reduced-precision mode
+ * stage through the context's workspace, as dgm_gemmNT of these shapes does). */
 int dgm_dit_forward(dgm_gpu* g, const dgm_dit_cfg* cfg, const dgm_dit_weights* w,
                     const float* cos_t, const float* sin_t, float* x, float* ws,
                     int64_t ws_floats);
