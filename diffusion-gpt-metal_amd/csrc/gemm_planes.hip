@@ -1220,6 +1220,7 @@ size_t layout_bytes(const Product* q, int n, int cus) {
 size_t planes_bytes(int64_t M, int64_t N, int64_t K, int cus, bool forward, bool backward) {
     const dgm_GemmP p{uint32_t(M), uint32_t(N), uint32_t(K), 0u, 1u, 0u, 0u, 0u};
     size_t b = 0;
+    forward = forward && K <= (int64_t(1) << 25);   // longer ones layout() refuses
     Product q[2];
     if (forward && planes_pay_fwd(M, N, K)) {
         q[0] = forward_of(32, nullptr, nullptr, nullptr, nullptr, nullptr, &p, nullptr);   // two planes of any weights
